@@ -113,6 +113,13 @@ int tfs_layout_block_colour_bfs(int n, const int *row, const int *col, int block
  * order).  Returns the number of colours. */
 int tfs_layout_brick_colour(int n, const int *row, const int *col, const int *dia, int edge,
                             int cap, int *perm, int *colour, int *block_of);
+/* Blocks of the FP64 sweeps (one workgroup each): order[p] the row at position
+ * p, block_of / step_of the block and step of each row.  Returns the number of
+ * blocks, 0 where the structure has none (the sweeps then go level by level),
+ * -1 on an invalid argument. */
+int tfs_layout_blocks(int n, const int *row, const int *col, const int *dia, int *order,
+                      int *block_of, int *step_of);
+
 /* The layouts the solver builds for a matrix (0-based CRS): s_orig = caller
  * row at each S (reverse Cuthill-McKee) position; level of each caller row in
  * the lower dependency DAG of the caller's numbering (forward sweep) and in

@@ -13,4 +13,9 @@ hipStream_t matrix_stream(const tfs_matrix *A);
 // once, and a cap on one matrix's persistent sweep grid (at least 1).
 int sweep_capacity(const tfs_matrix *A);
 void set_sweep_grid(tfs_matrix *A, int groups);
+// tfs_matrix_create for a matrix whose solves run beside other matrices'
+// (the server): without the block sweeps, so that the sweep grids' shares of
+// one kernel's occupancy hold.
+int matrix_create_shared(int n, long long nnz, const int *row, const int *col, const int *dia,
+                         int base, tfs_matrix **out);
 }  // namespace tfs

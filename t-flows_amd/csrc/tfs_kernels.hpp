@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 
 #include "tfs_device.hpp"
+#include "tfs_layout.hpp"
 
 namespace tfs {
 
@@ -312,35 +313,43 @@ k_gather(int n, const TI *__restrict__ in, const int *__restrict__ idx, TO *__re
 // runs of the row in the L / U layouts (which keep the caller's entry order:
 // the lower run is the entries before the diagonal, the upper run those
 // after it).
-template <typename T>
-__device__ __forceinline__ void values_put(int j, T v, int e0, int dj, int l0, int u0, int k,
-                                           int p, T *s_val, T *s_diag, T *l_val, T *u_val,
+template <typename T, bool S, bool TRI>
+__device__ __forceinline__ void values_put(int j, T v, T *s_at, int s_step, int dj, int l0, int u0,
+                                           int k, int p, T *s_diag, T *l_val, T *u_val,
                                            T *l_diag) {
-  s_val[e0 + j] = v;
-  if (j < dj) {
-    l_val[l0 + j] = v;
-  } else if (j == dj) {
-    s_diag[k] = v;
-    l_diag[p] = v;
-  } else {
-    u_val[u0 + (j - dj - 1)] = v;
+  if (S) s_at[(long long)j * s_step] = v;
+  if (TRI && j < dj) l_val[l0 + j] = v;
+  if (TRI && j > dj) u_val[u0 + (j - dj - 1)] = v;
+  if (j == dj) {
+    if (S) s_diag[k] = v;
+    if (TRI) l_diag[p] = v;
   }
 }
 
-template <typename T>
+// S: the S-order values (with `off`, into the sliced ELL of k_ell64, 64 rows
+// per slice, slot-major -- its stores are then contiguous across the
+// wavefront and no second pass fills the ELL; else into the CSR copy) and the
+// S-order diagonal.  TRI: the level-ordered triangles.
+template <typename T, bool S, bool TRI>
 __global__ void __launch_bounds__(kRedThreads)
 k_values(int n, const double *__restrict__ val, const int *__restrict__ s_row,
          const int *__restrict__ s_src, const int *__restrict__ s_diag_src,
-         const int *__restrict__ s_lpos, const int *__restrict__ s_to_u,
-         const int *__restrict__ l_ptr, const int *__restrict__ u_ptr, T *__restrict__ s_val,
-         T *__restrict__ s_diag, T *__restrict__ l_val, T *__restrict__ u_val,
-         T *__restrict__ l_diag) {
+         const long long *__restrict__ off, const int *__restrict__ s_lpos,
+         const int *__restrict__ s_to_u, const int *__restrict__ l_ptr,
+         const int *__restrict__ u_ptr, T *__restrict__ s_val, T *__restrict__ s_diag,
+         T *__restrict__ l_val, T *__restrict__ u_val, T *__restrict__ l_diag) {
   TFS_GRID_STRIDE(k, n) {
     const int e0 = s_row[k], len = s_row[k + 1] - e0;
     const int c0 = s_src[e0];           // the row's first entry in val[]
     const int dj = s_diag_src[k] - c0;  // the diagonal's place in the row
-    const int p = s_lpos[k], q = s_to_u[k];
-    const int l0 = l_ptr[p], u0 = u_ptr[q];
+    int p = 0, l0 = 0, u0 = 0;
+    if (TRI) {
+      p = s_lpos[k];
+      l0 = l_ptr[p];
+      u0 = u_ptr[s_to_u[k]];
+    }
+    T *const s_at = !S ? nullptr : off ? s_val + off[k / kWave] + k % kWave : s_val + e0;
+    const int s_step = off ? kWave : 1;
     // the first kPrefetch entries: all loads issued before any store
     T v[kPrefetch];
 #pragma unroll
@@ -348,9 +357,12 @@ k_values(int n, const double *__restrict__ val, const int *__restrict__ s_row,
       if (j < len) v[j] = (T)val[c0 + j];
 #pragma unroll
     for (int j = 0; j < kPrefetch; ++j)
-      if (j < len) values_put(j, v[j], e0, dj, l0, u0, k, p, s_val, s_diag, l_val, u_val, l_diag);
+      if (j < len)
+        values_put<T, S, TRI>(j, v[j], s_at, s_step, dj, l0, u0, k, p, s_diag, l_val, u_val,
+                              l_diag);
     for (int j = kPrefetch; j < len; ++j)
-      values_put(j, (T)val[c0 + j], e0, dj, l0, u0, k, p, s_val, s_diag, l_val, u_val, l_diag);
+      values_put<T, S, TRI>(j, (T)val[c0 + j], s_at, s_step, dj, l0, u0, k, p, s_diag, l_val,
+                            u_val, l_diag);
   }
 }
 
@@ -1237,6 +1249,278 @@ k_sweep_syncfree(int n, Tri<T> Tr, T *d, T *b, T *x, T *arm, const KState *st, i
     if (prev == gridDim.x - 1) {  // everyone else has left
       ctr[0] = 0u;
       ctr[1] = 0u;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The sweeps and the factor over the blocks of tfs_layout.hpp: one workgroup
+// of two wavefronts per block of at most kBlockRows rows (8^3 bricks on a
+// lexicographic grid).  The block's entries, factor and right-hand side go to
+// LDS before anything is waited for.  Wavefront 0 then advances the block step
+// by step (a step: rows of one dependency level inside the block, one per
+// lane) on results in LDS, so a level costs an LDS round trip instead of a
+// device-memory one; only the halo -- the rows of earlier blocks this one
+// depends on -- crosses CUs.  Results are stored as they are formed
+// (device-coherent, the value itself the ready flag, as k_sweep_syncfree), so
+// a neighbour starts on a block's first faces while the block still runs.
+// Wavefront 1 polls the halo and puts each value into its LDS slot, which
+// holds the sentinel until then: loads and stores share one in-order counter
+// on this part, so a wavefront that both stores results and waits for loads
+// would wait for its own stores' round trip (about 0.8 us) at every step.
+// Until its first value arrives a block polls only the head of its halo (first
+// needed first): most resident blocks are far behind the front, and their polls
+// would delay the stores everyone waits for.
+//
+// Order and progress: blocks are numbered so that a block depends on earlier
+// ones only; workgroup w takes blocks w, w + G, ... with all G resident, so
+// the lowest unfinished block always runs and every wait ends; the polls are
+// bounded as in k_sweep_syncfree all the same (a halo slot given up is filled
+// with zero, so wavefront 0 always finishes).
+//
+// Every row sum is formed in the caller's entry order; padding entries are
+// 0 * 0 terms, which leave any sum as it is.
+//
+// What bounds it: the dependency chain -- per step an LDS round trip and a
+// row's arithmetic (about 0.12 us), per block on the chain one halo hop (store,
+// poll, LDS: about 1.2 us) -- and above about 5 M rows the traffic.  us per
+// sweep on MI355X, level-ordered sweeps (k_sweep_syncfree / k_levels_small)
+// before, blocks after: 12^3 30 -> 11, 32^3 113 -> 30, 97x75x61 348 -> 82,
+// 128^3 640 -> 138, 200^3 285 after.  Blocks of 8^3 rather than larger ones:
+// 16^3 halves the hops but needs several wavefronts and a barrier per step.
+// Tried and not kept: one wavefront that also polls (its loads wait for its
+// stores: 104 us at 97x75x61, 172 at 128^3), two polling wavefronts (84, 145),
+// polling the whole halo from the start (82, 139), twice the workgroups (82,
+// 141; 264 at 200^3, but two matrices' sweeps must fit side by side).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+struct BlockTri {
+  const Block *__restrict__ blk;
+  const unsigned short *__restrict__ step, *__restrict__ idx;
+  const double *__restrict__ val;
+  const int *__restrict__ halo;
+};
+
+typedef double Vec2d __attribute__((ext_vector_type(2)));
+typedef unsigned Vec4u __attribute__((ext_vector_type(4)));
+constexpr int kBlockThreads = 2 * kWave;
+constexpr int kHaloLane = kBlockHalo / kWave;  // halo entries per lane
+constexpr unsigned kLdsSpinLimit = 1u << 26;
+constexpr int kHaloHead = 8;                   // polled until the first value arrives
+
+// LDS of one block sweep: values (slot-major), right-hand sides, factor,
+// places, step starts, results and halo -- strides fixed, so that a row's data
+// comes through one address.
+inline __host__ __device__ size_t block_lds(int width, int halo) {
+  return (size_t)kBlockRows * (sizeof(double) * (size_t)(width + 2) +
+                               sizeof(short) * (width <= 3 ? 4 : 8)) +
+         sizeof(int) * kWave + sizeof(double) * (size_t)(1 + kBlockRows + halo);
+}
+
+// A halo slot waits while it holds the sentinel; its high word alone tells (a
+// signalling NaN, which no arithmetic produces, whatever the low word).
+__device__ __forceinline__ bool waiting(double v) {
+  return (unsigned)__double2hiint(v) == (unsigned)(Sentinel<double>::bits >> 32);
+}
+
+template <int OP, int W>
+__global__ void __launch_bounds__(kBlockThreads)
+k_block_sweep(int n, int nblk, BlockTri Tr, const int *__restrict__ src,
+              const double *__restrict__ d, double *b, double *out, double *arm, const KState *st,
+              int *err) {
+  constexpr int PL = W <= 3 ? 4 : 8;  // places per row
+  extern __shared__ double lds[];
+  double *const vv = lds;
+  double *const ss = vv + W * kBlockRows, *const dd = ss + kBlockRows;
+  unsigned short *const ii = reinterpret_cast<unsigned short *>(dd + kBlockRows);
+  int *const tt = reinterpret_cast<int *>(ii + PL * kBlockRows);
+  double *const xs = reinterpret_cast<double *>(tt + kWave);
+  const int tid = (int)threadIdx.x, lane = tid % kWave;
+  const int done = st ? st->done : 0;  // looked at once the first loads are under way
+  for (int bk = (int)blockIdx.x; bk < nblk; bk += (int)gridDim.x) {
+    const Block B = Tr.blk[bk];
+    // ---- stage the block.  Indices past an array's end are clamped to its
+    // last element, so that every load is unconditional and all are in flight
+    // together.
+    {
+      constexpr int kR = kBlockRows / kBlockThreads;
+      constexpr int kV = W * kBlockRows / 2 / kBlockThreads;
+      constexpr int kI = PL * kBlockRows / 8 / kBlockThreads;
+      constexpr int kH = kBlockHalo / kBlockThreads;
+      const Vec2d *const vg = reinterpret_cast<const Vec2d *>(Tr.val + B.ent0);
+      const Vec4u *const ig =
+          reinterpret_cast<const Vec4u *>(Tr.idx + (size_t)B.idx0 * PL);
+      const int rp = B.rpad / 2, nv = W * rp, ni = PL * B.rpad / 8;
+      int at[kR];
+      Vec4u ri[kI];
+      Vec2d rv[kV];
+      double rhs[kR], df[kR];
+#pragma unroll
+      for (int c = 0; c < kR; ++c) {
+        const int p = B.row0 + min(c * kBlockThreads + tid, B.rows - 1);
+        at[c] = OP == OP_FWD ? src[p] : OP == OP_BWD ? n - 1 - p : p;
+      }
+#pragma unroll
+      for (int c = 0; c < kI; ++c) ri[c] = ig[min(c * kBlockThreads + tid, ni - 1)];
+#pragma unroll
+      for (int c = 0; c < kV; ++c) rv[c] = vg[min(c * kBlockThreads + tid, nv - 1)];
+      if (OP != OP_FACTOR) {
+#pragma unroll
+        for (int c = 0; c < kR; ++c) {
+          const int p = B.row0 + min(c * kBlockThreads + tid, B.rows - 1);
+          df[c] = d[OP == OP_BWD ? n - 1 - p : p];
+        }
+      }
+      const int t0 = Tr.step[B.step0 + min(tid, B.steps)];
+#pragma unroll
+      for (int c = 0; c < kR; ++c) rhs[c] = b[at[c]];
+      if (__builtin_amdgcn_readfirstlane(done)) return;
+      __syncthreads();  // the previous block is done with LDS
+      if (tid == 0) xs[0] = 0.0;
+      if (tid < kWave) tt[tid] = t0;
+#pragma unroll
+      for (int c = 0; c < kH; ++c)
+        if (c * kBlockThreads + tid < B.halo)
+          xs[1 + B.rows + c * kBlockThreads + tid] = Sentinel<double>::value();
+#pragma unroll
+      for (int c = 0; c < kI; ++c)
+        if (c * kBlockThreads + tid < ni)
+          reinterpret_cast<Vec4u *>(ii)[c * kBlockThreads + tid] = ri[c];
+#pragma unroll
+      for (int c = 0; c < kV; ++c) {
+        const int e = c * kBlockThreads + tid;   // slot k of the rows' pair q
+        if (e < nv) {
+          int k = 0;
+#pragma unroll
+          for (int j = 1; j < W; ++j) k += e >= j * rp;
+          reinterpret_cast<Vec2d *>(vv)[k * (kBlockRows / 2) + e - k * rp] = rv[c];
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < kR; ++c) {
+        const int p = c * kBlockThreads + tid;
+        if (p < B.rows) {
+          if (OP == OP_BWD) {
+            rhs[c] = rhs[c] / (df[c] + kTiny);
+            b[at[c]] = Sentinel<double>::value();  // re-armed: this block is its only reader
+          }
+          if (OP == OP_FWD) arm[B.row0 + p] = Sentinel<double>::value();
+          ss[p] = rhs[c];
+          if (OP != OP_FACTOR) dd[p] = df[c];
+        }
+      }
+    }
+    __syncthreads();
+    if (tid >= kWave) {
+      // ---- wavefront 1: the halo
+      int hq[kHaloLane];
+      unsigned lack = 0;
+#pragma unroll
+      for (int c = 0; c < kHaloLane; ++c)
+        if (c * kWave < B.halo) {
+          hq[c] = Tr.halo[B.halo0 + min(c * kWave + lane, B.halo - 1)];
+          if (c * kWave + lane < B.halo) lack |= 1u << c;
+        }
+      double *const slot = xs + 1 + B.rows + lane;
+      bool started = B.halo <= kHaloHead;
+      for (unsigned spins = 1; __any(lack != 0); ++spins) {
+        if (spins > kSpinLimit || ((spins & 255u) == 0 && coherent_load(err) != 0)) {
+          // out of patience, or another block gave up
+          coherent_store(err, 1);
+#pragma unroll
+          for (int c = 0; c < kHaloLane; ++c)
+            if (lack >> c & 1u)
+              __hip_atomic_store(slot + c * kWave, 0.0, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_WORKGROUP);
+          break;
+        }
+        if (!started) {
+          double v = Sentinel<double>::value();
+          if (lane < kHaloHead) v = coherent_load(&out[hq[0]]);
+          if (!__any(!waiting(v))) continue;
+          started = true;
+          if (!waiting(v)) {
+            __hip_atomic_store(slot, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            lack &= ~1u;
+          }
+        }
+        double v[kHaloLane];
+#pragma unroll
+        for (int c = 0; c < kHaloLane; ++c)
+          if (c * kWave < B.halo) {
+            v[c] = Sentinel<double>::value();
+            if (lack >> c & 1u) v[c] = coherent_load(&out[hq[c]]);
+          }
+#pragma unroll
+        for (int c = 0; c < kHaloLane; ++c)
+          if (c * kWave < B.halo && !waiting(v[c])) {
+            __hip_atomic_store(slot + c * kWave, v[c], __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+            lack &= ~(1u << c);
+          }
+      }
+    } else {
+      // ---- wavefront 0: the steps.  Row data of the next step is read from
+      // LDS while this one computes (two register sets in turn).
+      const char *const xb = reinterpret_cast<const char *>(xs);
+      const int starts = tt[lane];
+      unsigned waits = 0;
+      struct Row {
+        unsigned short id[PL];
+        double a[W], s, dp;
+        int p, p1;
+      } r0, r1;
+      auto read_row = [&](Row &r, int t) {  // step t's rows: one per lane
+        const int first = __builtin_amdgcn_readlane(starts, t);
+        r.p1 = __builtin_amdgcn_readlane(starts, t + 1);
+        r.p = first + lane;
+        const int q = min(r.p, r.p1 - 1);
+        __builtin_memcpy(r.id, ii + q * PL, sizeof(r.id));
+#pragma unroll
+        for (int k = 0; k < W; ++k) r.a[k] = vv[k * kBlockRows + q];
+        r.s = ss[q];
+        if (OP != OP_FACTOR) r.dp = dd[q];
+      };
+      auto advance = [&](const Row &r, Row &next, int t) {
+        double x[W];
+#pragma unroll
+        for (int k = 0; k < W; ++k)
+          x[k] = __hip_atomic_load(reinterpret_cast<const double *>(xb + r.id[k]),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        read_row(next, min(t + 1, B.steps - 1));
+        for (;;) {
+          bool miss = false;
+#pragma unroll
+          for (int k = 0; k < W; ++k) miss = miss || waiting(x[k]);
+          if (!__any(miss)) break;
+          if (++waits > kLdsSpinLimit) {  // wavefront 1 fills every slot long before this
+            coherent_store(err, 1);
+            break;
+          }
+#pragma unroll
+          for (int k = 0; k < W; ++k)
+            x[k] = __hip_atomic_load(reinterpret_cast<const double *>(xb + r.id[k]),
+                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        double v = r.s;
+#pragma unroll
+        for (int k = 0; k < W; ++k) v = sweep_term<OP>(v, r.a[k], x[k]);
+        v = OP == OP_FACTOR ? 1.0 / v : v * r.dp;
+        if (r.p < r.p1) {
+          __hip_atomic_store(&xs[1 + r.p], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          coherent_store(&out[B.row0 + r.p], v);
+        }
+        wave_sync();
+      };
+      read_row(r0, 0);
+      for (int t = 0; t < B.steps; t += 2) {
+        advance(r0, r1, t);
+        if (t + 1 < B.steps) advance(r1, r0, t + 1);
+      }
     }
   }
 }

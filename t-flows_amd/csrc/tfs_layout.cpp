@@ -183,6 +183,82 @@ void build_sweep(int n, const int *row, const int *col, const int *dia, bool low
   }
 }
 
+// The brick blocks of rows [r0, r1), which no entry couples to other rows:
+// blk[i] for each of them (numbered from 0 in order of the groups' first rows);
+// returns their number.  See brick_colour_order.  With `split`, index steps of
+// at most three binary orders are a class each, whatever their counts (a box
+// whose shorter sides come first merges two of them otherwise).
+int brick_blocks(int r0, int r1, const int *row, const int *col, const int *dia, int edge, int cap,
+                 bool split, int *blk) {
+  const int n = r1 - r0;
+  // classes of the dependencies j -> i by the binary order of i - j
+  constexpr int kClasses = 3;
+  std::vector<long long> hist(32, 0);
+  auto order_of = [](unsigned d) { return 31 - __builtin_clz(d); };
+  long long ntri = 0;
+  for (int i = r0; i < r1; ++i)
+    for (int e = row[i]; e < dia[i]; ++e) {
+      hist[order_of((unsigned)(i - col[e]))]++;
+      ++ntri;
+    }
+  std::vector<int> cls(32, 0);
+  {
+    int c = 0;
+    long long acc = 0;
+    bool any = false;
+    int orders = 0;
+    for (int o = 0; o < 32; ++o) orders += hist[o] > 0;
+    const bool own = split && orders <= kClasses;
+    for (int o = 0; o < 32; ++o) {
+      if (!hist[o]) continue;
+      if (any && c < kClasses - 1 && (own || acc * kClasses >= (long long)(c + 1) * ntri)) ++c;
+      cls[o] = c;
+      acc += hist[o];
+      any = true;
+    }
+  }
+  // potentials, row by row in caller order (dependencies come first)
+  std::vector<int> phi((size_t)n * kClasses, 0);
+  for (int i = r0; i < r1; ++i) {
+    int *f = &phi[(size_t)(i - r0) * kClasses];
+    for (int e = row[i]; e < dia[i]; ++e) {
+      const int j = col[e], c = cls[order_of((unsigned)(i - j))];
+      const int *g = &phi[(size_t)(j - r0) * kClasses];
+      for (int k = 0; k < kClasses; ++k) f[k] = std::max(f[k], g[k] + (k == c ? 1 : 0));
+    }
+  }
+  // groups: one id per distinct brick key, in order of their first row; a
+  // group's rows in caller order, split into blocks of at most cap rows
+  long long span = 1;
+  for (size_t i = 0; i < phi.size(); ++i) span = std::max<long long>(span, phi[i] / edge + 1);
+  std::unordered_map<long long, int> gid;
+  gid.reserve((size_t)n / (size_t)std::max(1, edge * edge * edge) + 16);
+  std::vector<int> grp(n);
+  std::vector<int> gcount;
+  for (int i = 0; i < n; ++i) {
+    const int *f = &phi[(size_t)i * kClasses];
+    const long long key = (f[0] / edge) + span * ((f[1] / edge) + span * (long long)(f[2] / edge));
+    auto it = gid.find(key);
+    if (it == gid.end()) {
+      it = gid.emplace(key, (int)gcount.size()).first;
+      gcount.push_back(0);
+    }
+    grp[i] = it->second;
+    gcount[(size_t)it->second]++;
+  }
+  std::vector<int>().swap(phi);
+  const int ng = (int)gcount.size();
+  std::vector<int> gfirst((size_t)ng + 1, 0);  // blocks of each group
+  for (int g = 0; g < ng; ++g) gfirst[(size_t)g + 1] = gfirst[(size_t)g] + (gcount[(size_t)g] + cap - 1) / cap;
+  const int nb = gfirst[(size_t)ng];
+  std::vector<int> seen_in_group((size_t)ng, 0);
+  for (int i = 0; i < n; ++i) {
+    const int g = grp[i];
+    blk[r0 + i] = gfirst[(size_t)g] + seen_in_group[(size_t)g]++ / cap;
+  }
+  return nb;
+}
+
 }  // namespace
 
 int colour_order(int n, const int *row, const int *col, std::vector<int> &perm,
@@ -322,68 +398,8 @@ int brick_colour_order(int n, const int *row, const int *col, const int *dia, in
   if (n <= 0) return 0;
   edge = std::max(1, edge);
   cap = std::max(1, cap);
-  // classes of the dependencies j -> i by the binary order of i - j
-  constexpr int kClasses = 3;
-  std::vector<long long> hist(32, 0);
-  auto order_of = [](unsigned d) { return 31 - __builtin_clz(d); };
-  long long ntri = 0;
-  for (int i = 0; i < n; ++i)
-    for (int e = row[i]; e < dia[i]; ++e) {
-      hist[order_of((unsigned)(i - col[e]))]++;
-      ++ntri;
-    }
-  std::vector<int> cls(32, 0);
-  {
-    int c = 0;
-    long long acc = 0;
-    bool any = false;
-    for (int o = 0; o < 32; ++o) {
-      if (!hist[o]) continue;
-      if (any && c < kClasses - 1 && acc * kClasses >= (long long)(c + 1) * ntri) ++c;
-      cls[o] = c;
-      acc += hist[o];
-      any = true;
-    }
-  }
-  // potentials, row by row in caller order (dependencies come first)
-  std::vector<int> phi((size_t)n * kClasses, 0);
-  for (int i = 0; i < n; ++i) {
-    int *f = &phi[(size_t)i * kClasses];
-    for (int e = row[i]; e < dia[i]; ++e) {
-      const int j = col[e], c = cls[order_of((unsigned)(i - j))];
-      const int *g = &phi[(size_t)j * kClasses];
-      for (int k = 0; k < kClasses; ++k) f[k] = std::max(f[k], g[k] + (k == c ? 1 : 0));
-    }
-  }
-  // groups: one id per distinct brick key, in order of their first row; a
-  // group's rows in caller order, split into blocks of at most cap rows
-  long long span = 1;
-  for (size_t i = 0; i < phi.size(); ++i) span = std::max<long long>(span, phi[i] / edge + 1);
-  std::unordered_map<long long, int> gid;
-  gid.reserve((size_t)n / (size_t)std::max(1, edge * edge * edge) + 16);
-  std::vector<int> grp(n);
-  std::vector<int> gcount;
-  for (int i = 0; i < n; ++i) {
-    const int *f = &phi[(size_t)i * kClasses];
-    const long long key = (f[0] / edge) + span * ((f[1] / edge) + span * (long long)(f[2] / edge));
-    auto it = gid.find(key);
-    if (it == gid.end()) {
-      it = gid.emplace(key, (int)gcount.size()).first;
-      gcount.push_back(0);
-    }
-    grp[i] = it->second;
-    gcount[(size_t)it->second]++;
-  }
-  std::vector<int>().swap(phi);
-  const int ng = (int)gcount.size();
-  std::vector<int> gfirst((size_t)ng + 1, 0);  // blocks of each group
-  for (int g = 0; g < ng; ++g) gfirst[(size_t)g + 1] = gfirst[(size_t)g] + (gcount[(size_t)g] + cap - 1) / cap;
-  const int nb = gfirst[(size_t)ng];
-  std::vector<int> blk(n), seen_in_group((size_t)ng, 0);
-  for (int i = 0; i < n; ++i) {
-    const int g = grp[i];
-    blk[i] = gfirst[(size_t)g] + seen_in_group[(size_t)g]++ / cap;
-  }
+  std::vector<int> blk(n);
+  const int nb = brick_blocks(0, n, row, col, dia, edge, cap, false, blk.data());
   // greedy colouring of the block graph (symmetrised pattern), blocks in id order
   std::vector<int> bstart_c((size_t)nb + 1, 0);
   for (int i = 0; i < n; ++i) bstart_c[(size_t)blk[i] + 1]++;
@@ -446,6 +462,186 @@ int brick_colour_order(int n, const int *row, const int *col, const int *dia, in
     bcolour.push_back(bcol[(size_t)b]);
   }
   return ncol;
+}
+
+namespace {
+
+// One triangle of the blocks in block order: `orig` the caller row of each
+// position, blocks [bstart[b], bstart[b + 1]), and per position its step.
+// False if a limit is exceeded.
+bool build_block_triangle(const int *row, const int *col, const int *dia, bool lower,
+                          const std::vector<int> &orig, const std::vector<int> &of_orig,
+                          const std::vector<int> &bstart, const std::vector<int> &lstep,
+                          int width, int places, BlockTriangle &T) {
+  const int nb = (int)bstart.size() - 1;
+  std::vector<int> slot_of(orig.size(), -1), in_halo;  // halo number of a position, this block
+  T.blk.resize((size_t)nb);
+  for (int b = 0; b < nb; ++b) {
+    Block &B = T.blk[(size_t)b];
+    B.row0 = bstart[(size_t)b];
+    B.rows = bstart[(size_t)b + 1] - B.row0;
+    B.rpad = (B.rows + 7) & ~7;
+    B.ent0 = (int)T.src.size();
+    B.idx0 = (int)(T.idx.size() / (size_t)places);
+    B.halo0 = (int)T.halo.size();
+    B.step0 = (int)T.step.size();
+    if (T.src.size() + (size_t)width * B.rpad > 0x7fffffffu) return false;
+    T.src.resize(T.src.size() + (size_t)width * B.rpad, -1);
+    T.idx.resize(T.idx.size() + (size_t)places * B.rpad, 0);
+    in_halo.clear();
+    for (int p = 0; p < B.rows; ++p) {
+      const int i = orig[(size_t)(B.row0 + p)];
+      const int j0 = lower ? row[i] : dia[i] + 1, j1 = lower ? dia[i] : row[i + 1];
+      for (int j = j0; j < j1; ++j) {
+        const int q = of_orig[(size_t)col[j]];
+        int slot;
+        if (q >= B.row0 && q < B.row0 + B.rows) {
+          if (lstep[(size_t)q] >= lstep[(size_t)(B.row0 + p)]) return false;
+          slot = 1 + q - B.row0;
+        } else {
+          if (q > B.row0) return false;  // only earlier blocks
+          if (slot_of[(size_t)q] < 0) {
+            slot_of[(size_t)q] = (int)in_halo.size();
+            in_halo.push_back(q);
+          }
+          slot = 1 + B.rows + slot_of[(size_t)q];
+        }
+        T.idx[((size_t)B.idx0 + p) * places + (j - j0)] = (unsigned short)(slot * sizeof(double));
+        T.src[(size_t)B.ent0 + (size_t)(j - j0) * B.rpad + p] = j;
+      }
+      // a step: one lane per row, so at most a wavefront of one level's rows
+      if (p == 0 || lstep[(size_t)(B.row0 + p)] != lstep[(size_t)(B.row0 + p - 1)] ||
+          p - T.step.back() == kBlockLanes)
+        T.step.push_back((unsigned short)p);
+    }
+    B.steps = (int)T.step.size() - B.step0;
+    T.step.push_back((unsigned short)B.rows);
+    B.halo = (int)in_halo.size();
+    for (int q : in_halo) slot_of[(size_t)q] = -1;
+    if (B.steps > kBlockSteps || B.halo > kBlockHalo) return false;
+    T.halo.insert(T.halo.end(), in_halo.begin(), in_halo.end());
+    T.halo_max = std::max(T.halo_max, B.halo);
+  }
+  return true;
+}
+
+}  // namespace
+
+void build_blocks(int n, const int *row, const int *col, const int *dia,
+                  const std::vector<int> &s_of_orig, int nlev, BlockLayout &out) {
+  out = BlockLayout();
+  if (n <= 0 || nlev < kBlockLevels) return;
+  // the triangles: at most kBlockWide entries a row, and structurally
+  // symmetric (the upper sweep runs the lower order backwards, which needs
+  // every upper entry to mirror a lower one)
+  int width = 0;
+  {
+    std::vector<int> next(row, row + n);  // per row, the first lower entry not yet mirrored
+    for (int i = 0; i < n; ++i) {
+      width = std::max({width, dia[i] - row[i], row[i + 1] - dia[i] - 1});
+      for (int j = dia[i] + 1; j < row[i + 1]; ++j) {
+        const int k = col[j];  // row k's lower columns ascend, so its mirrors come in order
+        if (next[(size_t)k] >= dia[k] || col[next[(size_t)k]] != i) return;
+        ++next[(size_t)k];
+      }
+    }
+    for (int i = 0; i < n; ++i)
+      if (next[(size_t)i] != dia[i]) return;
+  }
+  if (width > kBlockWide) return;
+  out.width = width <= 3 ? 3 : kBlockWide;
+  // blocks per range of rows that no entry leaves (the systems of a batch)
+  std::vector<int> blk((size_t)n);
+  int nb = 0;
+  for (int r0 = 0, reach = 0, i = 0; i < n; ++i) {
+    reach = std::max(reach, col[row[i + 1] - 1]);
+    if (reach > i) continue;
+    const int m = brick_blocks(r0, i + 1, row, col, dia, kBlockEdge, kBlockRows, true, blk.data());
+    for (int k = r0; k <= i; ++k) blk[(size_t)k] += nb;
+    nb += m;
+    r0 = i + 1;
+  }
+  // depth of each block in the block graph (its edges, sorted and distinct)
+  std::vector<long long> edges;
+  for (int i = 0; i < n; ++i)
+    for (int j = row[i]; j < dia[i]; ++j) {
+      const int from = blk[(size_t)col[j]], to = blk[(size_t)i];
+      if (from == to) continue;
+      const long long e = (long long)from * nb + to;
+      if (edges.empty() || edges.back() != e) edges.push_back(e);
+    }
+  std::sort(edges.begin(), edges.end());
+  edges.erase(std::unique(edges.begin(), edges.end()), edges.end());
+  std::vector<int> indeg((size_t)nb, 0), lev((size_t)nb, 0), order;
+  std::vector<size_t> first((size_t)nb + 1, 0);
+  for (long long e : edges) {
+    indeg[(size_t)(e % nb)]++;
+    first[(size_t)(e / nb) + 1]++;
+  }
+  for (int b = 0; b < nb; ++b) first[(size_t)b + 1] += first[(size_t)b];
+  order.reserve((size_t)nb);
+  for (int b = 0; b < nb; ++b)
+    if (!indeg[(size_t)b]) order.push_back(b);
+  int depth = 0;
+  for (size_t k = 0; k < order.size(); ++k) {
+    const int b = order[k];
+    depth = std::max(depth, lev[(size_t)b] + 1);
+    for (size_t e = first[(size_t)b]; e < first[(size_t)b + 1]; ++e) {
+      const int to = (int)(edges[e] % nb);
+      lev[(size_t)to] = std::max(lev[(size_t)to], lev[(size_t)b] + 1);
+      if (--indeg[(size_t)to] == 0) order.push_back(to);
+    }
+  }
+  if ((int)order.size() != nb || (long long)depth * kBlockGain > nlev) return;
+  // blocks by depth (then number), rows of a block by their level inside it,
+  // ties in S order (whose right-hand side they gather)
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+    return lev[(size_t)a] != lev[(size_t)b] ? lev[(size_t)a] < lev[(size_t)b] : a < b;
+  });
+  std::vector<int> place((size_t)nb);
+  for (int k = 0; k < nb; ++k) place[(size_t)order[(size_t)k]] = k;
+  std::vector<int> rlev((size_t)n, 0), bstart((size_t)nb + 1, 0);
+  for (int i = 0; i < n; ++i) {
+    for (int j = row[i]; j < dia[i]; ++j)
+      if (blk[(size_t)col[j]] == blk[(size_t)i])
+        rlev[(size_t)i] = std::max(rlev[(size_t)i], rlev[(size_t)col[j]] + 1);
+    bstart[(size_t)place[(size_t)blk[(size_t)i]] + 1]++;
+  }
+  for (int k = 0; k < nb; ++k) bstart[(size_t)k + 1] += bstart[(size_t)k];
+  out.orig.resize((size_t)n);
+  {
+    std::vector<int> fill(bstart.begin(), bstart.end() - 1);
+    for (int i = 0; i < n; ++i)
+      out.orig[(size_t)fill[(size_t)place[(size_t)blk[(size_t)i]]]++] = i;
+  }
+  for (int k = 0; k < nb; ++k)
+    std::sort(out.orig.begin() + bstart[(size_t)k], out.orig.begin() + bstart[(size_t)k + 1],
+              [&](int a, int b) {
+                return rlev[(size_t)a] != rlev[(size_t)b]
+                           ? rlev[(size_t)a] < rlev[(size_t)b]
+                           : s_of_orig[(size_t)a] < s_of_orig[(size_t)b];
+              });
+  out.of_orig.resize((size_t)n);
+  for (int p = 0; p < n; ++p) out.of_orig[(size_t)out.orig[(size_t)p]] = p;
+  std::vector<int> lstep((size_t)n);
+  for (int p = 0; p < n; ++p) lstep[(size_t)p] = rlev[(size_t)out.orig[(size_t)p]];
+  if (!build_block_triangle(row, col, dia, true, out.orig, out.of_orig, bstart, lstep, out.width,
+                            out.places(), out.L))
+    return;
+  // the upper triangle: everything backwards
+  std::vector<int> orig_u(out.orig.rbegin(), out.orig.rend()), of_u((size_t)n),
+      step_u((size_t)n), bstart_u((size_t)nb + 1);
+  for (int q = 0; q < n; ++q) {
+    of_u[(size_t)orig_u[(size_t)q]] = q;
+    step_u[(size_t)q] = -lstep[(size_t)(n - 1 - q)];
+  }
+  for (int k = 0; k <= nb; ++k) bstart_u[(size_t)k] = n - bstart[(size_t)(nb - k)];
+  if (!build_block_triangle(row, col, dia, false, orig_u, of_u, bstart_u, step_u, out.width,
+                            out.places(), out.U))
+    return;
+  out.nblk = nb;
+  out.depth = depth;
+  out.ok = true;
 }
 
 void build_layout(int n, const int *row, const int *col, const int *dia, int spmv_rows,

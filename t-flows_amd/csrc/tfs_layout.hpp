@@ -99,6 +99,56 @@ int brick_colour_order(int n, const int *row, const int *col, const int *dia, in
                        std::vector<int> &perm, std::vector<int> &bstart,
                        std::vector<int> &bcolour);
 
+// Blocks of the two triangular sweeps in the caller's own order (the factor
+// the drop-in must apply), one workgroup per block (k_block_sweep): rows
+// grouped by their monotone potentials as brick_colour_order groups them
+// (kBlockEdge^3 bricks on a lexicographic grid), every block's rows sorted by
+// their dependency level inside the block.  A row then depends on earlier
+// steps of its own block and on rows of earlier blocks (its halo).
+constexpr int kBlockEdge = 8;
+constexpr int kBlockRows = 512;      // rows of one block
+constexpr int kBlockSteps = 63;      // steps of one block (their starts fit one wavefront)
+constexpr int kBlockHalo = 384;      // halo entries of one block (six per lane)
+constexpr int kBlockLanes = 64;      // rows of one step
+constexpr int kBlockWide = 6;        // entries of a row in one triangle
+
+struct Block {     // one block of one triangle, as the kernel reads it
+  int row0, rows;  // its rows in block order (upper triangle: the order backwards)
+  int rpad;        // rows rounded up to eight: the stride between entry slots
+  int ent0;        // first entry slot: slot k of row p is ent0 + k rpad + p
+  int idx0;        // its rows' places begin at idx0 times the places per row
+  int halo0, halo; // its halo entries
+  int step0, steps;
+};
+
+struct BlockTriangle {
+  std::vector<Block> blk;
+  // per row, 4 (8 for wide rows) places of its entries' values in the block's
+  // LDS array, as byte offsets: slot 0 holds zero (the padding), 1 + p a row
+  // of the block, 1 + rows + h a halo entry
+  std::vector<unsigned short> idx;
+  std::vector<int> src;               // entry of the caller's val[], -1 padding
+  std::vector<int> halo;              // block-order position of each halo entry
+  std::vector<unsigned short> step;   // steps + 1 row starts per block
+  int halo_max = 0;
+};
+
+struct BlockLayout {
+  bool ok = false;                    // the structure suits block sweeps
+  int nblk = 0, depth = 0, width = 0; // blocks, depth of their graph, entry slots per row
+  int places() const { return width <= 3 ? 4 : 8; }
+  std::vector<int> orig, of_orig;     // block-order position <-> caller row
+  BlockTriangle L, U;
+};
+
+// Builds the blocks if the structure suits them (`out.ok`): structurally
+// symmetric, within the limits above, at least kBlockLevels levels deep (a
+// random numbering of a hex mesh has 13 to 20, in no blocks worth having) and
+// the block graph at least kBlockGain times shallower than the nlev levels.
+constexpr int kBlockGain = 4, kBlockLevels = 24;
+void build_blocks(int n, const int *row, const int *col, const int *dia,
+                  const std::vector<int> &s_of_orig, int nlev, BlockLayout &out);
+
 void build_layout(int n, const int *row, const int *col, const int *dia, int spmv_rows,
                   int spmv_cap, int small_level, Layout &out, bool identity_s = false);
 

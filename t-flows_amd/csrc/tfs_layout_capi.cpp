@@ -77,3 +77,25 @@ extern "C" int tfs_layout_brick_colour(int n, const int *row, const int *col, co
     }
   return ncol;
 }
+
+extern "C" int tfs_layout_blocks(int n, const int *row, const int *col, const int *dia, int *order,
+                                 int *block_of, int *step_of) {
+  if (n < 1 || !row || !col || !dia || !order || !block_of || !step_of) return -1;
+  tfs::Layout L;
+  tfs::build_layout(n, row, col, dia, 64, 512, 2048, L);
+  tfs::BlockLayout B;
+  tfs::build_blocks(n, row, col, dia, L.s_of_orig, L.L.nlev, B);
+  if (!B.ok) return 0;
+  for (int b = 0; b < B.nblk; ++b) {
+    const tfs::Block &K = B.L.blk[(std::size_t)b];
+    for (int t = 0; t < K.steps; ++t)
+      for (int p = B.L.step[(std::size_t)(K.step0 + t)];
+           p < B.L.step[(std::size_t)(K.step0 + t + 1)]; ++p) {
+        const int i = B.orig[(std::size_t)(K.row0 + p)];
+        order[K.row0 + p] = i;
+        block_of[i] = b;
+        step_of[i] = t;
+      }
+  }
+  return B.nblk;
+}

@@ -63,14 +63,14 @@ struct Request {
 
 // Device bytes of a resident case before its first solve (then replaced by
 // the exact figure), an upper bound: per entry, col + source index in the S
-// layout, the caller-order and S-order FP64 values, the FP64 sliced ELL (col,
-// source index, value; up to 1.25 nnz slots with padding), and col + value in
-// the L or U triangle (off-diagonal entries); per row, row pointers, maps,
+// layout, the caller-order FP64 values, the S-order ones (CSR, or the sliced
+// ELL's column and value in up to 1.25 nnz slots), and col + value in the L or
+// U triangle (off-diagonal entries); per row, row pointers, maps,
 // diagonal copies, the factor in two orders, two staging vectors and up to 12
 // work vectors (Cgs); plus the fixed per-matrix buffers (state, the partial
 // sums of the reductions, flags).
 long long estimate_bytes(int n, long long nnz) {
-  return 24 * nnz + 20 * nnz + 12 * (nnz - n) + 200 * (long long)n + (320 << 10);
+  return 16 * nnz + 15 * nnz + 12 * (nnz - n) + 200 * (long long)n + (320 << 10);
 }
 
 }  // namespace
@@ -162,8 +162,8 @@ struct tfs_server {
       for (tfs_matrix *e : evict) tfs_matrix_destroy(e);
       int rc = 0;
       if (create) {
-        rc = tfs_matrix_create(c->n, c->nnz, c->row.data(), c->col.data(), c->dia.data(), c->base,
-                               &c->A);
+        rc = tfs::matrix_create_shared(c->n, c->nnz, c->row.data(), c->col.data(),
+                                       c->dia.data(), c->base, &c->A);
         if (rc == 0) rc = tfs_matrix_set_sweep_schedule(c->A, TFS_SWEEP_STATIC);
         if (rc == 0)
           tfs::set_sweep_grid(c->A, tfs::sweep_capacity(c->A) / nworkers);

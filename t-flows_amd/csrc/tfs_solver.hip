@@ -123,14 +123,26 @@ struct DevSweep {
   long long ntri = 0;
 };
 
+// One triangle of the block sweeps (tfs_layout.hpp), FP64.
+struct DevBlocks {
+  Block *blk = nullptr;
+  unsigned short *step = nullptr, *idx = nullptr;
+  int *src = nullptr, *halo = nullptr;
+  double *val = nullptr;
+  long long slots = 0;
+  int halo_max = 0;
+};
+
 // Values and factor in one precision, in the S, L and U layouts.
 template <typename T>
 struct Values {
   T *s_val = nullptr, *s_diag = nullptr, *l_val = nullptr, *u_val = nullptr, *l_diag = nullptr;
   T *dL = nullptr, *dU = nullptr;
-  bool allocated = false;
-  bool ready = false;     // copies match the caller's values
-  int factor_prec = -1;   // prec the factor was built for, -1 = stale
+  bool allocated = false;      // the S part
+  bool tri_allocated = false;  // the L / U part (level order; made when first swept)
+  bool ready = false;          // the S copies match the caller's values
+  bool tri_ready = false;      // the triangles (level or block order) do
+  int factor_prec = -1;        // prec the factor was built for, -1 = stale
 };
 
 // Krylov work vectors of one precision (S order unless noted).
@@ -159,6 +171,18 @@ struct tfs_matrix {
   // level-sorted copy the L order is the S order)
   bool l_ident = false, u_rev = false, s_to_u_rev = false;
   int *s_lpos = nullptr;  // L position of the row at S position k
+  // block sweeps (FP64): built where the structure suits them
+  bool blk_ok = false;
+  int blk_n = 0, blk_width = 0;
+  DevBlocks bL, bU;
+  int *b_to_s = nullptr;      // S position of the row at block position p
+  int *b_of_orig = nullptr;   // block position of each caller row
+  int *s_to_bz = nullptr;     // position of S row k in the backward block sweep's output
+  int *b_diag_src = nullptr;  // the diagonals in block order: entry of val, value
+  double *b_diag = nullptr, *b_d = nullptr;  // and the factor
+  bool blk_allocated = false;
+  int blk_grid = 0;
+  bool blk_off = false;       // another sweep schedule set by the caller or the environment
   double *val = nullptr;       // caller-order FP64 values
   Values<double> v64;
   Values<float> v32;
@@ -210,7 +234,7 @@ struct tfs_matrix {
   int e64_nslice = 0;
   long long e64_len = 0;
   long long *e64_off = nullptr;
-  int *e64_col = nullptr, *e64_src = nullptr;
+  int *e64_col = nullptr;
   double *e64_val = nullptr;
   // Point-coloured incomplete-Cholesky sweeps of the inner copy: per colour,
   // sliced ELL of the strictly-lower (L) and strictly-upper (U) entries.
@@ -227,7 +251,7 @@ struct tfs_matrix {
 namespace {
 
 int matrix_create(int n, long long nnz, const int *row, const int *col, const int *dia, int base,
-                  tfs_matrix **out, Layout *keep, bool identity_s = false);
+                  tfs_matrix **out, Layout *keep, bool identity_s = false, bool blocks = true);
 
 int dev_alloc(tfs_matrix *A, void **p, size_t bytes) {
   if (bytes == 0) bytes = 8;
@@ -391,44 +415,92 @@ void launch_sweep(tfs_matrix *A, const DevSweep &S, const Tri<T> &Tr, T *d, cons
   tm_end(kc);
 }
 
+// Whether the FP64 sweeps run over blocks (k_block_sweep): where the structure
+// has them (build_blocks), under the static schedule (the default); a server's
+// matrices have none (matrix_create_shared).  No timing decides: wherever the block graph is kBlockGain times
+// shallower than the rows' levels the blocks measured 2 to 4 times faster
+// (figures at k_block_sweep).
+inline bool use_blocks(const tfs_matrix *A) {
+  return A->blk_ok && !A->blk_off;
+}
+
 template <typename T>
 int alloc_values(tfs_matrix *A) {
   Values<T> &V = vals<T>(A);
   if (V.allocated) return 0;
-  const size_t n = (size_t)std::max(A->n, 1);
-  TFS_TRY(dev_alloc(A, (void **)&V.s_val, sizeof(T) * (size_t)std::max(A->nnz, 1LL)));
-  TFS_TRY(dev_alloc(A, (void **)&V.l_val, sizeof(T) * (size_t)std::max(A->L.ntri, 1LL)));
-  TFS_TRY(dev_alloc(A, (void **)&V.u_val, sizeof(T) * (size_t)std::max(A->U.ntri, 1LL)));
-  TFS_TRY(dev_alloc(A, (void **)&V.s_diag, sizeof(T) * n));
-  TFS_TRY(dev_alloc(A, (void **)&V.l_diag, sizeof(T) * n));
-  TFS_TRY(dev_alloc(A, (void **)&V.dL, sizeof(T) * n));
-  TFS_TRY(dev_alloc(A, (void **)&V.dU, sizeof(T) * n));
+  // FP64 values go straight into the sliced ELL where there is one
+  if (sizeof(T) == 4 || A->e64_len == 0)
+    TFS_TRY(dev_alloc(A, (void **)&V.s_val, sizeof(T) * (size_t)std::max(A->nnz, 1LL)));
+  TFS_TRY(dev_alloc(A, (void **)&V.s_diag, sizeof(T) * (size_t)std::max(A->n, 1)));
   V.allocated = true;
   return 0;
 }
 
-// Copies of the caller's values into the S, L and U layouts in precision T
-// (part of the work the reference does each call: the matrix changed).
 template <typename T>
-int prepare_values(tfs_matrix *A) {
+int alloc_triangles(tfs_matrix *A) {
+  Values<T> &V = vals<T>(A);
+  const size_t n = (size_t)std::max(A->n, 1);
+  if (sizeof(T) == 8 && use_blocks(A)) {
+    if (A->blk_allocated) return 0;
+    for (DevBlocks *D : {&A->bL, &A->bU})
+      TFS_TRY(dev_alloc(A, (void **)&D->val, sizeof(double) * (size_t)D->slots));
+    TFS_TRY(dev_alloc(A, (void **)&A->b_diag, sizeof(double) * n));
+    TFS_TRY(dev_alloc(A, (void **)&A->b_d, sizeof(double) * n));
+    A->blk_allocated = true;
+    return 0;
+  }
+  if (V.tri_allocated) return 0;
+  TFS_TRY(dev_alloc(A, (void **)&V.l_val, sizeof(T) * (size_t)std::max(A->L.ntri, 1LL)));
+  TFS_TRY(dev_alloc(A, (void **)&V.u_val, sizeof(T) * (size_t)std::max(A->U.ntri, 1LL)));
+  TFS_TRY(dev_alloc(A, (void **)&V.l_diag, sizeof(T) * n));
+  TFS_TRY(dev_alloc(A, (void **)&V.dL, sizeof(T) * n));
+  TFS_TRY(dev_alloc(A, (void **)&V.dU, sizeof(T) * n));
+  V.tri_allocated = true;
+  return 0;
+}
+
+template <typename T, bool S, bool TRI>
+void launch_values(tfs_matrix *A) {
+  Values<T> &V = vals<T>(A);
+  const bool ell = sizeof(T) == 8 && A->e64_len > 0;
+  T *s_val = ell ? reinterpret_cast<T *>(A->e64_val) : V.s_val;
+  hipLaunchKernelGGL((k_values<T, S, TRI>), dim3(vgrid(A->n)), dim3(kRedThreads), 0, cur_stream(),
+                     A->n, A->val, A->s_row, A->s_src, A->s_diag_src, ell ? A->e64_off : nullptr,
+                     A->s_lpos, A->s_to_u, A->L.ptr, A->U.ptr, s_val, V.s_diag, V.l_val, V.u_val,
+                     V.l_diag);
+}
+
+// Copies of the caller's values in precision T into the S layout and, with
+// `tri`, into the triangles of the sweeps (part of the work the reference does
+// each call: the matrix changed).  What is up to date stays; both level-order
+// parts together take one pass over the caller's values.
+template <typename T>
+int prepare_values(tfs_matrix *A, bool tri = false) {
   TFS_TRY(alloc_values<T>(A));
   Values<T> &V = vals<T>(A);
-  if (V.ready) return 0;
-  const int n = A->n;
-  if (n > 0)
-    hipLaunchKernelGGL(k_values<T>, dim3(vgrid(n)), dim3(kRedThreads), 0, cur_stream(), n,
-                       A->val, A->s_row, A->s_src, A->s_diag_src, A->s_lpos, A->s_to_u,
-                       A->L.ptr, A->U.ptr, V.s_val, V.s_diag, V.l_val, V.u_val, V.l_diag);
-  if (sizeof(T) == 8 && A->e64_len > 0)
-    hipLaunchKernelGGL(k_ell_values<double>, dim3(grid_for(A->e64_len, kRedThreads, 8192)),
-                       dim3(kRedThreads), 0, cur_stream(), A->e64_len, A->e64_src, A->val,
-                       A->e64_val);
+  const bool blocks = sizeof(T) == 8 && use_blocks(A);
+  tri = tri && !V.tri_ready;
+  if (tri) TFS_TRY(alloc_triangles<T>(A));
+  if (A->n > 0) {
+    const bool levels = tri && !blocks;
+    if (!V.ready && levels) launch_values<T, true, true>(A);
+    else if (!V.ready) launch_values<T, true, false>(A);
+    else if (levels) launch_values<T, false, true>(A);
+    if (tri && blocks) {
+      for (DevBlocks *D : {&A->bL, &A->bU})
+        hipLaunchKernelGGL(k_ell_values<double>, dim3(grid_for(D->slots, kRedThreads, 8192)),
+                           dim3(kRedThreads), 0, cur_stream(), D->slots, D->src, A->val, D->val);
+      gather(A->n, A->val, A->b_diag_src, A->b_diag);
+    }
+  }
   V.ready = true;
+  if (tri) V.tri_ready = true;
   return 0;
 }
 
 void values_changed(tfs_matrix *A) {
   A->v64.ready = A->v32.ready = false;
+  A->v64.tri_ready = A->v32.tri_ready = false;
   A->v64.factor_prec = A->v32.factor_prec = -1;
   A->inner_ready = false;
   A->ell_ready = false;
@@ -439,12 +511,36 @@ template <typename T>
 int tune_sweeps(tfs_matrix *A);
 int check_sweep(tfs_matrix *A);
 
+// One sweep (or the factor) over the blocks.  d: the factor in block order;
+// b: right-hand side (S order), diagonals or forward result (block order);
+// out: block order (the backward sweep's runs it backwards).
+template <int OP>
+void launch_blocks(tfs_matrix *A, const DevBlocks &D, const double *d, const double *b,
+                   double *out, double *armv, const KState *st) {
+  const int kc = OP == OP_FACTOR ? TFS_KC_FACTOR : TFS_KC_SWEEP;
+  const BlockTri Tr{D.blk, D.step, D.idx, D.val, D.halo};
+  const size_t lds = block_lds(A->blk_width, D.halo_max);
+  tm_begin(kc);
+  auto kern = A->blk_width == 3 ? k_block_sweep<OP, 3> : k_block_sweep<OP, kBlockWide>;
+  hipLaunchKernelGGL(kern, dim3(A->blk_grid), dim3(kBlockThreads), lds, cur_stream(), A->n, A->blk_n,
+                     Tr, A->b_to_s, d, const_cast<double *>(b), out, armv,
+                     st, A->sweep_err);
+  tm_end(kc);
+}
+
 template <typename T>
 int prec_form(tfs_matrix *A, int prec) {
   if (prec < 0 || prec > 2) prec = 0;  // the reference treats any other value as none
-  TFS_TRY(prepare_values<T>(A));
+  TFS_TRY(prepare_values<T>(A, prec == 2));
   Values<T> &V = vals<T>(A);
   if (V.factor_prec == prec) return 0;
+  if (sizeof(T) == 8 && A->n > 0 && prec == 2 && use_blocks(A)) {
+    arm(A->n, A->b_d);
+    launch_blocks<OP_FACTOR>(A, A->bL, nullptr, A->b_diag, A->b_d, nullptr, nullptr);
+    TFS_HIP(hipGetLastError());
+    V.factor_prec = prec;
+    return 0;
+  }
   if (A->n > 0 && prec == 2) {
     const Tri<T> Tr{A->L.ptr, A->L.col, V.l_val, V.l_diag, nullptr};
     if (A->persistent) arm(A->n, V.dL);
@@ -458,10 +554,28 @@ int prec_form(tfs_matrix *A, int prec) {
   return 0;
 }
 
-// zU := M^-1 b for prec 2, b in S order, result in U order (yL scratch).
+// Where the backward sweep of precision T leaves the row at S position k.
+template <typename T>
+inline const int *z_of_s(const tfs_matrix *A) {
+  return sizeof(T) == 8 && use_blocks(A) ? A->s_to_bz : A->s_to_u;
+}
+template <typename T>
+inline bool z_reversed(const tfs_matrix *A) {
+  return A->s_to_u_rev && !(sizeof(T) == 8 && use_blocks(A));
+}
+
+// zU := M^-1 b for prec 2, b in S order, result in U order (z_of_s; yL
+// scratch).
 template <typename T>
 void dic_apply(tfs_matrix *A, const T *bS, T *yL, T *zU, const KState *st) {
   Values<T> &V = vals<T>(A);
+  if constexpr (sizeof(T) == 8) {
+    if (use_blocks(A)) {
+      launch_blocks<OP_FWD>(A, A->bL, A->b_d, bS, yL, zU, st);
+      launch_blocks<OP_BWD>(A, A->bU, A->b_d, yL, zU, nullptr, st);
+      return;
+    }
+  }
   // The FP32 sweeps form an identity or reversed right-hand-side index
   // instead of loading it; the FP64 ones (latency-bound) measured faster
   // loading it (256^3: 1430.5 against 1438.3 us per sweep; 128^3: 633.9
@@ -480,7 +594,7 @@ template <typename T>
 void prec_apply_S(tfs_matrix *A, int prec, const T *bS, T *xS, T *yL, T *zU, const KState *st) {
   if (prec == 2) {
     dic_apply<T>(A, bS, yL, zU, st);
-    gather(A->n, zU, A->s_to_u, xS, st);
+    gather(A->n, zU, z_of_s<T>(A), xS, st);
   } else {
     hipLaunchKernelGGL(k_diag_apply<T>, dim3(vgrid(A->n)), dim3(kRedThreads), 0, cur_stream(),
                        A->n, bS, vals<T>(A).s_diag, xS, prec, st);
@@ -610,10 +724,10 @@ template <typename T>
 void cg_iteration(tfs_matrix *A, int prec, const Vecs<T> &V, KState *st) {
   const int n = A->n, g = vgrid(n);
   if (prec == 2) dic_apply<T>(A, V.r, V.yL, V.zU, st);
-  const int mode = prec == 2 ? (A->s_to_u_rev ? 4 : 2) : prec == 1 ? 1 : 0;
+  const int mode = prec == 2 ? (z_reversed<T>(A) ? 4 : 2) : prec == 1 ? 1 : 0;
   T *z = prec == 0 ? V.r : V.z;  // prec 0: z is a copy of r (Prec_Solve.f90:72-75)
   hipLaunchKernelGGL(k_rho<T>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, V.r, V.z,
-                     vals<T>(A).s_diag, V.zU, A->s_to_u, mode, st, A->partials);
+                     vals<T>(A).s_diag, V.zU, z_of_s<T>(A), mode, st, A->partials);
   finish(g, A->partials, EPI_RHO, st);
   hipLaunchKernelGGL(k_pupdate<T>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, z, V.p, st);
   launch_spmv<T, SPMV_DOT>(A, V.p, V.q, V.p, nullptr, nullptr, st);
@@ -1061,7 +1175,7 @@ int build_inner(tfs_matrix *A) {
   }
   Layout Ly;
   tfs_matrix *C = nullptr;
-  TFS_TRY(matrix_create(n, nnz, prow.data(), pcol.data(), pdia.data(), 0, &C, &Ly, true));
+  TFS_TRY(matrix_create(n, nnz, prow.data(), pcol.data(), pdia.data(), 0, &C, &Ly, true, false));
   std::vector<int> from_s(n);
   for (int i = 0; i < n; ++i) from_s[i] = perm[Ly.s_orig[i]];
   int rc = upload(A, &A->inner_emap, emap);
@@ -1605,22 +1719,73 @@ int build_ell64(tfs_matrix *A, const Layout &Ly) {
   }
   const long long len = off[(size_t)ns];
   if (n == 0 || (double)len > 1.25 * (double)A->nnz) return 0;
-  std::vector<int> ecol((size_t)len, -1), esrc((size_t)len, -1);
+  std::vector<int> ecol((size_t)len, -1);
   for (int i = 0; i < n; ++i) {
     const int sl = i / kWave, lane = i % kWave;
     int j = 0;
-    for (int e = Ly.s_row[i]; e < Ly.s_row[i + 1]; ++e, ++j) {
-      const size_t q = (size_t)(off[(size_t)sl] + (long long)j * kWave + lane);
-      ecol[q] = Ly.s_col[e];
-      esrc[q] = Ly.s_src[e];
-    }
+    for (int e = Ly.s_row[i]; e < Ly.s_row[i + 1]; ++e, ++j)
+      ecol[(size_t)(off[(size_t)sl] + (long long)j * kWave + lane)] = Ly.s_col[e];
   }
   TFS_TRY(upload(A, &A->e64_off, off));
   TFS_TRY(upload(A, &A->e64_col, ecol));
-  TFS_TRY(upload(A, &A->e64_src, esrc));
   TFS_TRY(dev_alloc(A, (void **)&A->e64_val, sizeof(double) * (size_t)len));
   A->e64_nslice = ns;
   A->e64_len = len;
+  return 0;
+}
+
+// The block sweeps' structure, if it suits them, and their grid: at most half
+// the workgroups that fit at once, so that two matrices' block sweeps fit
+// beside each other (the static schedule needs all of them resident).
+int build_block_sweeps(tfs_matrix *A, const Layout &Ly, const int *row, const int *col,
+                       const int *dia) {
+  const int n = A->n;
+  BlockLayout BL;
+  build_blocks(n, row, col, dia, Ly.s_of_orig, Ly.L.nlev, BL);
+  if (!BL.ok) return 0;
+  const BlockTriangle *T[2] = {&BL.L, &BL.U};
+  DevBlocks *D[2] = {&A->bL, &A->bU};
+  for (int k = 0; k < 2; ++k) {
+    TFS_TRY(upload(A, &D[k]->blk, T[k]->blk));
+    TFS_TRY(upload(A, &D[k]->step, T[k]->step));
+    TFS_TRY(upload(A, &D[k]->idx, T[k]->idx));
+    TFS_TRY(upload(A, &D[k]->src, T[k]->src));
+    TFS_TRY(upload(A, &D[k]->halo, T[k]->halo));
+    D[k]->slots = (long long)T[k]->src.size();
+    D[k]->halo_max = T[k]->halo_max;
+  }
+  std::vector<int> to_s((size_t)n), bz((size_t)n), dsrc((size_t)n);
+  for (int p = 0; p < n; ++p) {
+    const int i = BL.orig[(size_t)p];
+    to_s[(size_t)p] = Ly.s_of_orig[(size_t)i];
+    dsrc[(size_t)p] = dia[i];
+    bz[(size_t)to_s[(size_t)p]] = n - 1 - p;
+  }
+  TFS_TRY(upload(A, &A->b_to_s, to_s));
+  TFS_TRY(upload(A, &A->s_to_bz, bz));
+  TFS_TRY(upload(A, &A->b_diag_src, dsrc));
+  TFS_TRY(upload(A, &A->b_of_orig, BL.of_orig));
+  A->blk_n = BL.nblk;
+  A->blk_width = BL.width;
+  const size_t lds = block_lds(BL.width, std::max(BL.L.halo_max, BL.U.halo_max));
+  int dev = 0, n_cu = 0, per_cu = 0;
+  TFS_HIP(hipGetDevice(&dev));
+  TFS_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
+  const bool narrow = BL.width == 3;
+  for (const void *kern :
+       {narrow ? reinterpret_cast<const void *>(k_block_sweep<OP_FACTOR, 3>)
+               : reinterpret_cast<const void *>(k_block_sweep<OP_FACTOR, kBlockWide>),
+        narrow ? reinterpret_cast<const void *>(k_block_sweep<OP_FWD, 3>)
+               : reinterpret_cast<const void *>(k_block_sweep<OP_FWD, kBlockWide>),
+        narrow ? reinterpret_cast<const void *>(k_block_sweep<OP_BWD, 3>)
+               : reinterpret_cast<const void *>(k_block_sweep<OP_BWD, kBlockWide>)}) {
+    int b = 0;
+    TFS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, kern, kBlockThreads, lds));
+    per_cu = per_cu == 0 ? b : std::min(per_cu, b);
+  }
+  if (per_cu < 1) return 0;
+  A->blk_grid = std::max(1, std::min(BL.nblk, n_cu * per_cu / 2));
+  A->blk_ok = true;
   return 0;
 }
 
@@ -1633,7 +1798,8 @@ int occupancy(int *per_cu) {
   return 0;
 }
 
-int create_device(tfs_matrix *A, const Layout &Ly) {
+int create_device(tfs_matrix *A, const Layout &Ly, const int *row, const int *col,
+                  const int *dia, bool blocks) {
   const int n = A->n;
   TFS_HIP(hipStreamCreateWithFlags(&A->stream, hipStreamNonBlocking));
   TFS_HIP(hipEventCreate(&A->ev0));
@@ -1664,6 +1830,7 @@ int create_device(tfs_matrix *A, const Layout &Ly) {
     for (int k = 0; k < n; ++k) lpos[(size_t)k] = Ly.L.of_orig[(size_t)Ly.s_orig[(size_t)k]];
     TFS_TRY(upload(A, &A->s_lpos, lpos));
   }
+  if (blocks) TFS_TRY(build_block_sweeps(A, Ly, row, col, dia));
   const size_t nb = sizeof(double) * (size_t)std::max(n, 1);
   TFS_TRY(dev_alloc(A, (void **)&A->val, sizeof(double) * (size_t)std::max(A->nnz, 1LL)));
   TFS_TRY(dev_alloc(A, (void **)&A->stage_x, nb));
@@ -1704,6 +1871,7 @@ int create_device(tfs_matrix *A, const Layout &Ly) {
     if (std::strcmp(e, "levels") == 0) A->persistent = false;
     if (std::strcmp(e, "dynamic") == 0) A->dynamic = true;
     if (std::strcmp(e, "cooperative") == 0) A->coop = true;
+    A->blk_off = !A->persistent || A->dynamic || A->coop;
     A->sweep_fixed = true;  // "static" (or anything else): the persistent static schedule
   }
   if (const char *e = std::getenv("TFS_SWEEP_GROUPS")) {  // the cap, up to the occupancy
@@ -1711,6 +1879,7 @@ int create_device(tfs_matrix *A, const Layout &Ly) {
     if (g > 0) {
       A->grid_persistent = std::max(1, std::min({chunks, n_cu * std::max(1, per_cu), g}));
       A->grid_fixed = true;
+      if (A->blk_ok) A->blk_grid = std::min(A->blk_grid, g);
     }
   }
   A->bandwidth = Ly.bandwidth;
@@ -1755,7 +1924,7 @@ namespace {
 // touching the device, so a bad structure is rejected without a GPU; then
 // builds the layouts and uploads them.  `keep` receives the host layout.
 int matrix_create(int n, long long nnz, const int *row, const int *col, const int *dia, int base,
-                  tfs_matrix **out, Layout *keep, bool identity_s) {
+                  tfs_matrix **out, Layout *keep, bool identity_s, bool blocks) {
   if (!out) return TFS_ERR_INVALID;
   *out = nullptr;
   if (n < 0 || nnz < n || nnz > 0x7ffffffeLL || (base != 0 && base != 1)) return TFS_ERR_INVALID;
@@ -1784,7 +1953,7 @@ int matrix_create(int n, long long nnz, const int *row, const int *col, const in
   tfs_matrix *A = new tfs_matrix;
   A->n = n;
   A->nnz = nnz;
-  const int rc = create_device(A, Ly);
+  const int rc = create_device(A, Ly, hr.data(), hc.data(), hd.data(), blocks);
   if (rc < 0) {
     tfs_matrix_destroy(A);
     return rc;
@@ -1798,6 +1967,11 @@ int matrix_create(int n, long long nnz, const int *row, const int *col, const in
 extern "C" int tfs_matrix_create(int n, long long nnz, const int *row, const int *col,
                                  const int *dia, int base, tfs_matrix **out) {
   return matrix_create(n, nnz, row, col, dia, base, out, nullptr);
+}
+
+int tfs::matrix_create_shared(int n, long long nnz, const int *row, const int *col, const int *dia,
+                              int base, tfs_matrix **out) {
+  return matrix_create(n, nnz, row, col, dia, base, out, nullptr, false, false);
 }
 
 extern "C" int tfs_matrix_destroy(tfs_matrix *A) {
@@ -1878,7 +2052,7 @@ extern "C" int tfs_matrix_get_info(const tfs_matrix *A, tfs_matrix_info *info) {
   info->ell64_slices = A->e64_len > 0 ? A->e64_nslice : 0;
   info->inner_order = A->inner ? A->inner_built : -1;
   info->inner_brick_edge = A->inner && A->inner_built == TFS_INNER_BRICKS ? A->inner_brick : 0;
-  info->sweep_groups = A->persistent ? A->grid_persistent : 0;
+  info->sweep_groups = use_blocks(A) ? A->blk_grid : A->persistent ? A->grid_persistent : 0;
   info->inner_sweep_groups =
       A->inner ? (A->inner->persistent ? A->inner->grid_persistent : 0) : -1;
   return TFS_OK;
@@ -2079,7 +2253,8 @@ extern "C" int tfs_prec_diag_device(tfs_matrix *A, double *d_out) {
   if (fp < 0) return TFS_ERR_INVALID;
   if (A->n == 0) return TFS_OK;
   if (fp == 2) {
-    gather(A->n, A->v64.dL, A->L.of_orig, d_out);
+    if (use_blocks(A)) gather(A->n, A->b_d, A->b_of_orig, d_out);
+    else gather(A->n, A->v64.dL, A->L.of_orig, d_out);
   } else if (fp == 1) {
     gather(A->n, A->v64.s_diag, A->s_of_orig, d_out);
   } else {
@@ -2305,7 +2480,7 @@ void batch_cg_iteration(tfs_batch *B, int prec, const Vecs<T> &V, KState *st, KS
   const int mode = prec == 2 ? 2 : prec == 1 ? 1 : 0;
   T *z = prec == 0 ? V.r : V.z;
   hipLaunchKernelGGL(k_rho_seg<T>, dim3(nt), dim3(kRedThreads), 0, cur_stream(), tl, V.r, V.z,
-                     vals<T>(A).s_diag, V.zU, A->s_to_u, mode, st, all, B->partials);
+                     vals<T>(A).s_diag, V.zU, z_of_s<T>(A), mode, st, all, B->partials);
   finish_seg(B, EPI_RHO, st, all);
   hipLaunchKernelGGL(k_pupdate_seg<T>, dim3(nt), dim3(kRedThreads), 0, cur_stream(), tl, z, V.p,
                      st, all);
@@ -2353,6 +2528,7 @@ int batch_graph_fn(tfs_batch *B, int slot, int prec, F &&one, hipGraphExec_t *ex
       (void)hipGraphExecDestroy(B->graph[slot]);
       B->graph[slot] = nullptr;
     }
+    if (use_blocks(B->A)) break;  // ordinary launches: the sweeps are not what failed
     B->A->persistent = false;  // retry with per-level sweeps
   }
   std::fprintf(stderr, "tfs: batch iteration not capturable; launching kernels directly\n");
@@ -2476,8 +2652,8 @@ namespace {
 // states, SpMV shape.  `Ly` receives the host layout.  On failure the
 // caller destroys B.
 int batch_build(tfs_batch *B, long long N, long long NNZ, const int *cr, const int *cc,
-                const int *cd, Layout &Ly) {
-  int rc = matrix_create((int)N, NNZ, cr, cc, cd, 0, &B->A, &Ly);
+                const int *cd, Layout &Ly, bool blocks) {
+  int rc = matrix_create((int)N, NNZ, cr, cc, cd, 0, &B->A, &Ly, false, blocks);
   if (rc < 0) return rc;
   B->A->sweep_fixed = true;  // the batch picks its sweeps when it captures its graph
   const int nsys = B->nsys;
@@ -2614,7 +2790,7 @@ int build_batch_inner(tfs_batch *B) {
     eo += B->nnz_of[s];
   }
   Layout Ly;
-  int rc = batch_build(C, n, nnz, prow.data(), pcol.data(), pdia.data(), Ly);
+  int rc = batch_build(C, n, nnz, prow.data(), pcol.data(), pdia.data(), Ly, false);
   if (rc == 0) rc = build_ell(C->A, Ly);  // the reliable-update loop's FP32 operator
   if (rc < 0) {
     tfs_batch_destroy(C);
@@ -2680,7 +2856,7 @@ extern "C" int tfs_batch_create(int nsys, const int *n, const long long *nnz,
   }
   cr[N] = (int)NNZ;
   Layout Ly;
-  const int rc = batch_build(B, N, NNZ, cr.data(), cc.data(), cd.data(), Ly);
+  const int rc = batch_build(B, N, NNZ, cr.data(), cc.data(), cd.data(), Ly, true);
   if (rc < 0) {
     tfs_batch_destroy(B);
     return rc;
@@ -3239,16 +3415,28 @@ extern "C" int tfs_matrix_set_sweep_schedule(tfs_matrix *A, int schedule) {
     return TFS_ERR_INVALID;
   StreamScope scope(A->stream);
   TFS_HIP(hipStreamSynchronize(A->stream));
-  const bool was_levels = !A->persistent;
+  const bool was_levels = !A->persistent, was_blocks = use_blocks(A);
   A->persistent = schedule != TFS_SWEEP_LEVELS;
   A->dynamic = schedule == TFS_SWEEP_DYNAMIC;
   A->coop = schedule == TFS_SWEEP_COOPERATIVE;
+  A->blk_off = schedule != TFS_SWEEP_STATIC;
   A->sweep_fixed = true;
   if (was_levels && A->persistent) {
     // the persistent sweeps need their outputs armed
     if (A->vec64) arm(A->n, A->vec64 + 2 * (size_t)A->n);
     if (A->vec32) arm(A->n, A->vec32 + 2 * (size_t)A->n);
     TFS_HIP(hipStreamSynchronize(A->stream));
+  }
+  if (use_blocks(A) != was_blocks && A->v64.tri_ready) {
+    // the triangles and the factor move to the other layout
+    const int formed = A->v64.factor_prec;
+    A->v64.tri_ready = false;
+    if (formed == 2) {
+      A->v64.factor_prec = -1;
+      TFS_TRY(prec_form<double>(A, 2));
+      TFS_HIP(hipStreamSynchronize(A->stream));
+      TFS_TRY(check_sweep(A));
+    }
   }
   if (A->inner) return tfs_matrix_set_sweep_schedule(A->inner, schedule);
   return TFS_OK;

@@ -86,6 +86,8 @@ def _lib():
         lib.tfs_layout_block_colour_bfs.restype = ctypes.c_int
         lib.tfs_layout_block_colour_bfs.argtypes = [ctypes.c_int, _I32P, _I32P, ctypes.c_int,
                                                     _I32P, _I32P, _I32P]
+        lib.tfs_layout_blocks.restype = ctypes.c_int
+        lib.tfs_layout_blocks.argtypes = [ctypes.c_int, _I32P, _I32P, _I32P, _I32P, _I32P, _I32P]
         lib.tfs_mesh_read_cns.restype = ctypes.c_int
         lib.tfs_mesh_read_cns.argtypes = [ctypes.c_char_p] + [ctypes.POINTER(ctypes.c_int)] * 3 + \
             [ctypes.c_void_p, ctypes.c_void_p]
@@ -242,6 +244,20 @@ def layout_brick_colour(row, col, dia, edge=4, cap=64):
     if k < 0:
         raise ValueError("tfs_layout_brick_colour failed")
     return k, perm, colour, block_of
+
+
+def layout_blocks(row, col, dia):
+    """Blocks of the FP64 sweeps (one workgroup each) of a 0-based CRS matrix:
+    (nblocks, order, block_of, step_of) per caller row, or None where the
+    structure has none and the sweeps go level by level."""
+    row = np.ascontiguousarray(row, np.int32)
+    n = len(row) - 1
+    order, block_of, step_of = (np.empty(n, np.int32) for _ in range(3))
+    k = _lib().tfs_layout_blocks(n, row, np.ascontiguousarray(col, np.int32),
+                                 np.ascontiguousarray(dia, np.int32), order, block_of, step_of)
+    if k < 0:
+        raise ValueError("tfs_layout_blocks failed")
+    return (k, order, block_of, step_of) if k else None
 
 
 def layout_summary(row, col, dia):
