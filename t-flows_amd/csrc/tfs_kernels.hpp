@@ -1525,6 +1525,173 @@ k_block_sweep(int n, int nblk, BlockTri Tr, const int *__restrict__ src,
   }
 }
 
+// ---------------------------------------------------------------------------
+// The FP32 incomplete-Cholesky sweeps of a brick-ordered copy, one wavefront
+// per unit of bricks of one colour (tfs_layout.hpp).  Bricks of one colour do
+// not couple, so a launch per colour needs no polling and no sentinels: the
+// halo is complete and goes to LDS at once.  A unit's rows then advance level by
+// level, one row per lane, step after step, on values in LDS.  A row's entries
+// and factor come coalesced as one 16-byte record of values and one 8-byte one
+// of 16-bit LDS offsets, its S position with them and its right-hand side after
+// it, all several steps ahead; rows with more than three entries (at the faces
+// towards other colours) have a second pair.  Every load and store of a step is
+// unconditional -- lanes beyond its rows and steps beyond the last repeat a row
+// -- since with conditional ones the compiler must assume they were not issued
+// and waits for the next steps' loads too.
+// Bound by memory: 36 to 60 bytes per row, 55-60 us per launch at 256^3 (two
+// colours of 16^3 bricks, 8.4 M rows a launch) at a large copy's rate.  There it
+// takes 86 us forward and 76 us backward, 325 us per application; the
+// synchronisation-free sweeps, whose rows wait for values from device memory,
+// took 232 + 225 us.  One wavefront per unit, not more: its steps then need no
+// workgroup barrier, and LDS holds only live values (7 KB for a 16^3 brick), so
+// the registers and not LDS decide how many units run at once.
+// Forward: y from r; backward: z from y; all in S order.  Arithmetic as
+// sweep_row: FP64 on FP32 storage, terms in the copy's entry order (padding:
+// 0 * 0), results rounded once per row.  The product of two FP32 values is exact
+// in FP64, so s - a x is one fused multiply-add with the same result as a
+// product and a difference.
+constexpr int kBrickAhead = 6;   // steps whose records are under way
+constexpr int kBrickRhs = 3;     // steps whose right-hand sides are
+typedef float Vec4f __attribute__((ext_vector_type(4)));
+typedef float Vec3f __attribute__((ext_vector_type(3)));
+typedef unsigned Vec2u __attribute__((ext_vector_type(2)));
+struct BrickTri {
+  const BrickStep *__restrict__ step;
+  const Vec2u *__restrict__ idx;
+  const Vec4f *__restrict__ val;
+  const int *__restrict__ halo;
+};
+
+// base[i] through a 32-bit byte offset (one scalar base, no 64-bit vector adds)
+template <typename T>
+__device__ __forceinline__ T at32(const T *base, unsigned i) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) +
+                                      (size_t)(i * (unsigned)sizeof(T)));
+}
+
+// The records' values: entry places and, in a first record, the row whose
+// factor (in L order, through its L position) is the fourth value.
+__global__ void __launch_bounds__(kRedThreads)
+k_brick_values(int m, const BrickSource *__restrict__ src, const double *__restrict__ val,
+               const int *__restrict__ lpos, const float *__restrict__ dL,
+               Vec4f *__restrict__ out) {
+  TFS_GRID_STRIDE(i, m) {
+    const BrickSource s = src[i];
+    Vec4f v;
+    v.x = s.e[0] >= 0 ? (float)val[s.e[0]] : 0.0f;
+    v.y = s.e[1] >= 0 ? (float)val[s.e[1]] : 0.0f;
+    v.z = s.e[2] >= 0 ? (float)val[s.e[2]] : 0.0f;
+    v.w = s.e[3] >= 0 ? dL[lpos[s.e[3]]] : 0.0f;
+    out[i] = v;
+  }
+}
+
+// LDS of a unit: step table, values.
+inline size_t brick_lds_bytes(int slots, int steps) {
+  return sizeof(BrickStep) * (size_t)steps + sizeof(float) * (size_t)slots;
+}
+
+struct BrickRow {   // one lane's row of a step
+  bool more;
+  int pos;
+  float rhs;
+  Vec4f a;
+  Vec3f a2;  // three values: a fourth register, unused, would be reused at once
+  Vec2u at, at2;  // and its load waited for
+};
+
+template <bool BWD>
+__global__ void __launch_bounds__(kWave)
+k_brick_sweep(int u0, int nu, int steps_max, const BrickUnit *__restrict__ unit, BrickTri Tr,
+              const int *__restrict__ pos, const float *__restrict__ in, float *out,
+              const KState *st) {
+  if (st && solve_done(st)) return;
+  extern __shared__ Vec2u brick_lds[];
+  Vec2u *const table = brick_lds;
+  float *const xs = reinterpret_cast<float *>(table + steps_max);
+  // contiguous units per XCD (workgroups go round the eight): neighbouring
+  // bricks share the lines at their borders in S order
+  const int per = (nu + 7) / 8, b = (int)blockIdx.x % 8 * per + (int)blockIdx.x / 8;
+  if ((int)blockIdx.x / 8 >= per || b >= nu) return;
+  const BrickUnit B = unit[u0 + b];
+  const int lane = (int)threadIdx.x, T = B.steps;
+  // the step table in LDS: from memory each step would wait for it before it
+  // could ask for its records
+  static_assert(sizeof(BrickStep) == sizeof(Vec2u), "step table rows");
+  const Vec2u *const steps = reinterpret_cast<const Vec2u *>(Tr.step + B.step0);
+  for (int k = lane; k < T; k += kWave) table[BWD ? T - 1 - k : k] = steps[k];
+  const int *const list = Tr.halo + (BWD ? B.uh0 : B.lh0);
+  const int nh = BWD ? B.uh : B.lh;
+  constexpr int kGroup = 8;
+  for (int h = lane; h < nh; h += kGroup * kWave) {
+    int at[kGroup];
+    float v[kGroup];
+#pragma unroll
+    for (int c = 0; c < kGroup; ++c) at[c] = list[min(h + c * kWave, nh - 1)];
+#pragma unroll
+    for (int c = 0; c < kGroup; ++c) v[c] = out[at[c]];
+#pragma unroll
+    for (int c = 0; c < kGroup; ++c) xs[1 + min(h + c * kWave, nh - 1)] = v[c];
+  }
+  if (lane == 0) xs[0] = 0.0f;
+  wave_sync();
+  // The table row of the step after the one being asked for is read ahead.
+  Vec2u next = table[0];
+  auto load = [&](BrickRow &R, int k) {
+    const int x0 = (int)next.x, p0 = (int)(next.y & 0xfffu), rows = (int)(next.y >> 12 & 0x7fu);
+    const int more = (int)(next.y >> 20), i = min(lane, rows - 1);
+    next = table[min(k + 1, T - 1)];
+    R.more = i < more;
+    const unsigned g = (unsigned)(B.row0 + p0 + i);
+    const unsigned x = (unsigned)(x0 + min(i, max(more - 1, 0)));
+    R.pos = at32(pos, g);
+    R.a = at32(Tr.val, g);
+    R.at = at32(Tr.idx, g);
+    R.a2 = at32(reinterpret_cast<const Vec3f *>(Tr.val), x);
+    R.at2 = at32(Tr.idx, x);
+    __builtin_amdgcn_sched_barrier(0);  // in this order, or a wait takes later loads along
+  };
+  auto load_rhs = [&](BrickRow &R) {
+    R.rhs = at32(in, (unsigned)R.pos);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  char *const xb = reinterpret_cast<char *>(xs);
+  auto at = [&](unsigned off) { return (double)*reinterpret_cast<const float *>(xb + off); };
+  auto advance = [&](const BrickRow &R) {
+    const double dp = (double)R.a.w;
+    const double x0 = at(R.at.x & 0xffffu), x1 = at(R.at.x >> 16), x2 = at(R.at.y & 0xffffu);
+    const double x3 = at(R.at2.x & 0xffffu), x4 = at(R.at2.x >> 16), x5 = at(R.at2.y & 0xffffu);
+    double s = (double)R.rhs;
+    if (BWD) s = s / (dp + kTiny);
+    s = __builtin_fma(-(double)R.a.x, x0, s);
+    s = __builtin_fma(-(double)R.a.y, x1, s);
+    s = __builtin_fma(-(double)R.a.z, x2, s);
+    double w = __builtin_fma(-(double)R.a2.x, x3, s);
+    w = __builtin_fma(-(double)R.a2.y, x4, w);
+    w = __builtin_fma(-(double)R.a2.z, x5, w);
+    s = R.more ? w : s;
+    const float v = (float)(s * dp);
+    *reinterpret_cast<float *>(xb + (R.at.y >> 16)) = v;
+    out[R.pos] = v;
+    wave_sync();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr int kRing = kBrickAhead + 1;
+  BrickRow R[kRing];
+#pragma unroll
+  for (int j = 0; j < kBrickAhead; ++j) load(R[j], j);
+#pragma unroll
+  for (int j = 0; j < kBrickRhs; ++j) load_rhs(R[j]);
+  for (int k = 0; k < T; k += kRing) {
+#pragma unroll
+    for (int j = 0; j < kRing; ++j) {
+      load(R[(j + kBrickAhead) % kRing], k + j + kBrickAhead);
+      load_rhs(R[(j + kBrickRhs) % kRing]);
+      advance(R[j]);
+    }
+  }
+}
+
 template <typename T>
 __global__ void __launch_bounds__(kRedThreads)
 k_arm(int n, T *__restrict__ x) {

@@ -79,6 +79,60 @@ int colour_order(int n, const int *row, const int *col, std::vector<int> &perm,
 int block_colour_order(int n, const int *row, const int *col, int block, std::vector<int> &perm,
                        std::vector<int> *colour = nullptr, std::vector<int> *block_of = nullptr);
 
+// The FP32 sweeps of a brick-ordered copy, one wavefront per unit of bricks of
+// one colour (k_brick_sweep): bricks of one colour do not couple, so a unit of
+// several has no more levels than one and fuller ones.  A unit's rows are sorted
+// by their level inside their brick and cut into steps of at most a
+// wavefront's rows of one level, one row per lane; both triangles use the same order.  A
+// row's first three entries of a triangle and its factor are one record; the
+// rows of a step with more come first and have a second record.
+constexpr int kBrickLanes = 64;      // rows of one step
+constexpr int kBrickWide = 6;        // entries of a row in one triangle
+constexpr int kUnitRows = 4096;      // rows of a unit (one 16^3 brick)
+constexpr int kUnitFull = 1024;      // bricks are merged up to this many rows
+struct BrickUnit {
+  int row0, rows, step0, steps;      // first row, rows, first step, steps
+  int lh0, lh, uh0, uh;              // halo entries of the lower / upper triangle
+};
+struct BrickStep {                   // one step of one triangle
+  int x0;                            // its first second record
+  unsigned what;                     // first row in the unit, rows, rows with a second record
+  int p0() const { return (int)(what & 0xfffu); }
+  int rows() const { return (int)(what >> 12 & 0x7fu); }
+  int more() const { return (int)(what >> 20); }
+};
+struct BrickSource { int e[4]; };    // where a record's values come from
+struct BrickPlaces { unsigned short at[4]; };
+struct BrickTriangle {
+  std::vector<BrickStep> step;
+  // Per row, then per second record (after all rows' first ones): the byte
+  // offsets in the unit's LDS array of floats of its entries' values -- slot 0
+  // holds zero (padding), 1 + h halo entry h at the start -- and, fourth in a
+  // first record, of its own result.  A slot is used again once the last step
+  // that reads its value is over, so the array holds what is live, not the unit.
+  std::vector<BrickPlaces> idx;
+  // the entries' places in val[] (-1 padding); fourth in a first record the
+  // row's place in the copy, for its factor
+  std::vector<BrickSource> src;
+  std::vector<int> halo;             // S position of each halo entry
+};
+struct BrickLayout {
+  bool ok = false;
+  int slots[2] = {0, 0};             // LDS floats of the largest unit, per triangle
+  int steps = 0;                     // steps of the largest unit
+  std::vector<BrickUnit> unit;       // colour after colour
+  std::vector<int> colour0;          // first unit of each colour (ncolours + 1)
+  std::vector<int> row, pos;         // copy row and its S position, unit order
+  BrickTriangle L, U;
+};
+// row/col/dia: the copy's CRS (0-based, its own order); blk and colour: the
+// block of each row and the colour of each block; s_of: S position of each row.
+// Not ok where a coupling does not stay in its block or go between colours in
+// the copy's order, or a limit is exceeded.
+void build_bricks(int n, const int *row, const int *col, const int *dia,
+                  const std::vector<int> &blk, const std::vector<int> &colour,
+                  const std::vector<int> &s_of, BrickLayout &out);
+
 // row/col/dia are 0-based, validated (diagonal present, columns ascending).
 // identity_s keeps the caller's order as the S order (for a matrix whose rows
 // are already in the order its kernels want, e.g. a block multi-colour copy).

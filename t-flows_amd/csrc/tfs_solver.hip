@@ -246,6 +246,19 @@ struct tfs_matrix {
   int *csw_col[2] = {nullptr, nullptr}, *csw_src[2] = {nullptr, nullptr};
   float *csw_val[2] = {nullptr, nullptr};
   bool csw_ready = false;
+  // Brick sweeps of the inner copy (k_brick_sweep): [0] lower, [1] upper triangle
+  bool brk_ok = false;
+  int brk_slots[2] = {0, 0}, brk_steps = 0;
+  std::vector<int> brk_colour0;           // host: first unit of each colour
+  BrickUnit *brk = nullptr;
+  int *brk_pos = nullptr;                 // S position of each row, unit order
+  BrickStep *brk_step[2] = {nullptr, nullptr};
+  BrickPlaces *brk_idx[2] = {nullptr, nullptr};
+  BrickSource *brk_src[2] = {nullptr, nullptr};
+  int *brk_halo[2] = {nullptr, nullptr};
+  int brk_len[2] = {0, 0};                // records
+  Vec4f *brk_val[2] = {nullptr, nullptr};
+  bool brk_ready = false;                 // values and factor match
 };
 
 namespace {
@@ -505,11 +518,16 @@ void values_changed(tfs_matrix *A) {
   A->inner_ready = false;
   A->ell_ready = false;
   A->csw_ready = false;
+  A->brk_ready = false;
 }
+
+// Whether this (inner) copy's FP32 sweeps run brick by brick (k_brick_sweep).
+inline bool use_bricks(const tfs_matrix *A) { return A->brk_ok && !A->blk_off; }
 
 template <typename T>
 int tune_sweeps(tfs_matrix *A);
 int check_sweep(tfs_matrix *A);
+int prepare_bricks(tfs_matrix *A);
 
 // One sweep (or the factor) over the blocks.  d: the factor in block order;
 // b: right-hand side (S order), diagonals or forward result (block order);
@@ -533,7 +551,8 @@ int prec_form(tfs_matrix *A, int prec) {
   if (prec < 0 || prec > 2) prec = 0;  // the reference treats any other value as none
   TFS_TRY(prepare_values<T>(A, prec == 2));
   Values<T> &V = vals<T>(A);
-  if (V.factor_prec == prec) return 0;
+  const bool bricks = sizeof(T) == 4 && prec == 2 && use_bricks(A);
+  if (V.factor_prec == prec) return bricks ? prepare_bricks(A) : 0;
   if (sizeof(T) == 8 && A->n > 0 && prec == 2 && use_blocks(A)) {
     arm(A->n, A->b_d);
     launch_blocks<OP_FACTOR>(A, A->bL, nullptr, A->b_diag, A->b_d, nullptr, nullptr);
@@ -549,6 +568,7 @@ int prec_form(tfs_matrix *A, int prec) {
     TFS_HIP(hipGetLastError());
   }
   V.factor_prec = prec;
+  if (bricks) return prepare_bricks(A);
   if (A->n > 0 && prec == 2 && !A->sweep_tuned && !A->sweep_fixed && A->persistent)
     TFS_TRY(tune_sweeps<T>(A));
   return 0;
@@ -718,13 +738,30 @@ int tune_sweeps(tfs_matrix *A) {
   return check_sweep(A);
 }
 
+void brick_sweeps(tfs_matrix *A, const float *r, float *y, float *z, const KState *st);
+
+// z := M^-1 r of a CG iteration for prec 2: over the bricks (z in S order,
+// returns true; the zU slot holds the forward result), or left in zU.
+template <typename T>
+bool cg_precondition(tfs_matrix *A, const T *r, T *yL, T *zU, T *z, const KState *st) {
+  if constexpr (sizeof(T) == 4) {
+    if (use_bricks(A)) {
+      brick_sweeps(A, r, zU, z, st);
+      return true;
+    }
+  }
+  dic_apply<T>(A, r, yL, zU, st);
+  return false;
+}
+
 // One CG iteration (Cg.f90:97-178) in precision T; Bicg takes the same path
 // (its shadow sequence equals the primary one bit for bit, Bicg.f90:91-175).
 template <typename T>
 void cg_iteration(tfs_matrix *A, int prec, const Vecs<T> &V, KState *st) {
   const int n = A->n, g = vgrid(n);
-  if (prec == 2) dic_apply<T>(A, V.r, V.yL, V.zU, st);
-  const int mode = prec == 2 ? (z_reversed<T>(A) ? 4 : 2) : prec == 1 ? 1 : 0;
+  const bool have_z = prec == 2 && cg_precondition<T>(A, V.r, V.yL, V.zU, V.z, st);
+  const int mode =
+      have_z ? 3 : prec == 2 ? (z_reversed<T>(A) ? 4 : 2) : prec == 1 ? 1 : 0;
   T *z = prec == 0 ? V.r : V.z;  // prec 0: z is a copy of r (Prec_Solve.f90:72-75)
   hipLaunchKernelGGL(k_rho<T>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, V.r, V.z,
                      vals<T>(A).s_diag, V.zU, z_of_s<T>(A), mode, st, A->partials);
@@ -1035,6 +1072,68 @@ int colour_sweeps(tfs_matrix *A, const float *r, float *y, float *z, const KStat
   return parts;
 }
 
+// The brick sweeps of a brick-ordered copy from its host layout; blk and
+// colour as build_bricks takes them.
+int build_brick_sweeps(tfs_matrix *A, const Layout &Ly, const int *row, const int *col,
+                       const int *dia, const std::vector<int> &blk,
+                       const std::vector<int> &colour) {
+  const int n = A->n;
+  BrickLayout BL;
+  build_bricks(n, row, col, dia, blk, colour, Ly.s_of_orig, BL);
+  if (!BL.ok || brick_lds_bytes(std::max(BL.slots[0], BL.slots[1]), BL.steps) > 65536) return 0;
+  TFS_TRY(upload(A, &A->brk, BL.unit));
+  TFS_TRY(upload(A, &A->brk_pos, BL.pos));
+  const BrickTriangle *T[2] = {&BL.L, &BL.U};
+  for (int t = 0; t < 2; ++t) {
+    TFS_TRY(upload(A, &A->brk_step[t], T[t]->step));
+    TFS_TRY(upload(A, &A->brk_idx[t], T[t]->idx));
+    TFS_TRY(upload(A, &A->brk_src[t], T[t]->src));
+    TFS_TRY(upload(A, &A->brk_halo[t], T[t]->halo));
+    A->brk_len[t] = (int)T[t]->idx.size();
+    TFS_TRY(dev_alloc(A, (void **)&A->brk_val[t], sizeof(Vec4f) * (size_t)A->brk_len[t]));
+  }
+  std::copy(BL.slots, BL.slots + 2, A->brk_slots);
+  A->brk_steps = BL.steps;
+  A->brk_colour0 = BL.colour0;
+  A->brk_ok = true;
+  return 0;
+}
+
+// The brick streams' values and factor (after prec_form<float>).
+int prepare_bricks(tfs_matrix *A) {
+  if (!use_bricks(A) || A->brk_ready) return 0;
+  // (the copy's own row order is its caller order: its L positions by row)
+  for (int t = 0; t < 2; ++t)
+    hipLaunchKernelGGL(k_brick_values, dim3(vgrid(A->brk_len[t])), dim3(kRedThreads), 0,
+                       cur_stream(), A->brk_len[t], A->brk_src[t], A->val, A->L.of_orig,
+                       A->v32.dL, A->brk_val[t]);
+  TFS_HIP(hipGetLastError());
+  A->brk_ready = true;
+  return 0;
+}
+
+// z := M^-1 r brick by brick, all in S order (y: the forward result), one
+// launch per colour and direction; the timing takes each direction as one sweep.
+void brick_sweeps(tfs_matrix *A, const float *r, float *y, float *z, const KState *st) {
+  const int K = (int)A->brk_colour0.size() - 1;
+  auto launch = [&](int c, int t) {
+    const int u0 = A->brk_colour0[(size_t)c], nu = A->brk_colour0[(size_t)c + 1] - u0;
+    if (nu < 1) return;
+    const BrickTri Tr{A->brk_step[t], reinterpret_cast<const Vec2u *>(A->brk_idx[t]),
+                      A->brk_val[t], A->brk_halo[t]};
+    auto kern = t == 0 ? k_brick_sweep<false> : k_brick_sweep<true>;
+    hipLaunchKernelGGL(kern, dim3((nu + 7) / 8 * 8), dim3(kWave),
+                       brick_lds_bytes(A->brk_slots[t], A->brk_steps), cur_stream(), u0, nu,
+                       A->brk_steps, A->brk, Tr, A->brk_pos, t == 0 ? r : y, t == 0 ? y : z, st);
+  };
+  tm_begin(TFS_KC_SWEEP);
+  for (int c = 0; c < K; ++c) launch(c, 0);
+  tm_end(TFS_KC_SWEEP);
+  tm_begin(TFS_KC_SWEEP);
+  for (int c = K - 1; c >= 0; --c) launch(c, 1);
+  tm_end(TFS_KC_SWEEP);
+}
+
 // The ELL values and row sums from the caller-order FP64 values.
 int prepare_ell(tfs_matrix *A) {
   if (A->ell_ready) return 0;
@@ -1083,7 +1182,7 @@ int build_inner(tfs_matrix *A) {
   TFS_HIP(hipMemcpyAsync(src.data(), A->s_src, sizeof(int) * nnz, hipMemcpyDeviceToHost,
                          cur_stream()));
   TFS_HIP(hipStreamSynchronize(cur_stream()));
-  std::vector<int> perm, bstart, bcolour;
+  std::vector<int> perm, bstart, bcolour, brick_of;  // brick_of: per S row
   int ncol = 0;
   bool bricks = false;
   if (A->inner_order == TFS_INNER_REFERENCE) {
@@ -1114,6 +1213,9 @@ int build_inner(tfs_matrix *A) {
                               bstart, bcolour);
     perm.resize(n);
     for (int i = 0; i < n; ++i) perm[i] = s_of[pc[i]];
+    brick_of.resize(n);
+    for (size_t b = 0; b + 1 < bstart.size(); ++b)
+      for (int k = bstart[b]; k < bstart[b + 1]; ++k) brick_of[perm[k]] = (int)b;
     bricks = true;
     if (A->inner_order == TFS_INNER_AUTO && ncol != 2) {  // irregular blocks: points
       bricks = false;
@@ -1181,9 +1283,16 @@ int build_inner(tfs_matrix *A) {
   int rc = upload(A, &A->inner_emap, emap);
   if (rc == 0) rc = upload(A, &A->inner_from_s, from_s);
   if (rc == 0) rc = build_ell(C, Ly);
-  // the point-coloured copy sweeps with k_colour_sweep; the brick-ordered one
-  // with the synchronisation-free sweeps (its DAG is a few levels deep: 4E - 2
-  // for E^3 bricks in two colours, 14 / 30 / 62 for E = 4 / 8 / 16)
+  // the point-coloured copy sweeps with k_colour_sweep, the one of bricks in two
+  // colours with k_brick_sweep (the synchronisation-free sweeps form its factor).
+  // With more colours a launch has few bricks and each costs a level count:
+  // 64 systems of 24..40 cells a side (7 colours, 2.2 M rows) took 14 launches of
+  // 34 us against two sweeps of 155 us, so those keep the latter.
+  if (rc == 0 && bricks && ncol == 2) {
+    std::vector<int> blk(n);
+    for (int i = 0; i < n; ++i) blk[i] = brick_of[perm[i]];
+    rc = build_brick_sweeps(C, Ly, prow.data(), pcol.data(), pdia.data(), blk, bcolour);
+  }
   if (rc == 0 && !bricks && A->inner_order != TFS_INNER_REFERENCE && A->inner_block == 1)
     rc = build_colour_sweeps(C, Ly);
   if (rc < 0) {
@@ -1193,6 +1302,7 @@ int build_inner(tfs_matrix *A) {
   C->persistent = A->persistent;
   C->dynamic = A->dynamic;
   C->coop = A->coop;
+  C->blk_off = A->blk_off;
   if (A->grid_fixed) {  // a caller's limit holds for the copy too
     C->grid_persistent = std::min(C->grid_persistent, A->grid_persistent);
     C->grid_fixed = true;
@@ -1234,10 +1344,11 @@ void reliable_iteration(tfs_matrix *I, int prec, const Vecs<float> &F, double *c
   }
   // z stays in the backward sweep's (reversed) order when that is the S
   // order backwards: k_rho and the p update read it from there
-  const bool zrev = prec == 2 && !csw && I->s_to_u_rev;
+  const bool zrev = prec == 2 && !csw && !use_bricks(I) && I->s_to_u_rev;
   if (!csw) {
-    if (prec == 2) dic_apply<float>(I, F.r, F.yL, F.zU, st);
-    const int mode = prec == 2 ? (zrev ? 5 : 2) : prec == 1 ? 1 : 0;
+    const bool have_z =
+        prec == 2 && cg_precondition<float>(I, F.r, F.yL, F.zU, F.z, st);
+    const int mode = have_z ? 3 : prec == 2 ? (zrev ? 5 : 2) : prec == 1 ? 1 : 0;
     hipLaunchKernelGGL(k_rho<float>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, F.r, F.z,
                        vals<float>(I).s_diag, F.zU, I->s_to_u, mode, st, I->partials);
     finish(g, I->partials, EPI_RHO, st);
