@@ -28,7 +28,7 @@ HIP_FLAGS = [
 ]
 HIP_SOURCES = ["tfs_solver.hip", "tfs_layout.cpp", "tfs_server.cpp", "tfs_assembly.hip",
                "tfs_topology.hip", "tfs_gradient.hip"]
-HIP_DEPS = ["tfs_device.hpp", "tfs_kernels.hpp", "tfs_layout.hpp"]
+HIP_DEPS = ["tfs_device.hpp", "tfs_kernels.hpp", "tfs_layout.hpp", "tfs_faces.hpp"]
 
 
 def _run(cmd, cwd=None):

@@ -897,4 +897,95 @@ void build_layout(int n, const int *row, const int *col, const int *dia, int spm
   for (int k = 0; k < n; ++k) out.s_to_u[k] = out.U.of_orig[out.s_orig[k]];
 }
 
+namespace {
+
+// 128-byte lines of a cell field and of a face field that the slices of an
+// order touch, summed over up to 256 slices spread over the mesh.
+long long lines_touched(int n, const int *faces, int base, const std::vector<int> &ptr,
+                        const std::vector<unsigned> &inc, const std::vector<int> *orig,
+                        const std::vector<int> *of) {
+  const int nslice = (n + 63) / 64, step = std::max(1, nslice / 256);
+  long long lines = 0;
+  std::vector<long long> seen;
+  for (int s = 0; s < nslice; s += step) {
+    seen.clear();
+    for (int k = 64 * s; k < std::min(n, 64 * s + 64); ++k) {
+      const int c = orig ? (*orig)[(size_t)k] : k;
+      seen.push_back(k / 16);
+      for (int e = ptr[(size_t)c]; e < ptr[(size_t)c + 1]; ++e) {
+        const long long f = inc[(size_t)e] >> 1;
+        const int o = faces[2 * f + ((inc[(size_t)e] & 1) ? 0 : 1)] - base;
+        seen.push_back(-1 - f / 16);
+        if (o >= 0) seen.push_back((of ? (*of)[(size_t)o] : o) / 16);
+      }
+    }
+    std::sort(seen.begin(), seen.end());
+    lines += std::unique(seen.begin(), seen.end()) - seen.begin();
+  }
+  return lines;
+}
+
+}  // namespace
+
+void build_face_lists(int n, long long nf, const int *faces, int base, FaceLists &out) {
+  out = FaceLists();
+  out.n = n;
+  // per cell, its faces in ascending order (a counting sort over the faces)
+  std::vector<int> ptr((size_t)n + 1, 0);
+  for (long long s = 0; s < nf; ++s) {
+    ptr[(size_t)(faces[2 * s] - base) + 1]++;
+    if (faces[2 * s + 1] >= base) ptr[(size_t)(faces[2 * s + 1] - base) + 1]++;
+  }
+  for (int c = 0; c < n; ++c) ptr[(size_t)c + 1] += ptr[(size_t)c];
+  std::vector<unsigned> inc((size_t)ptr[(size_t)n]);
+  {
+    std::vector<int> fill(ptr.begin(), ptr.end() - 1);
+    for (long long s = 0; s < nf; ++s) {
+      inc[(size_t)fill[(size_t)(faces[2 * s] - base)]++] = (unsigned)(2 * s);
+      if (faces[2 * s + 1] >= base)
+        inc[(size_t)fill[(size_t)(faces[2 * s + 1] - base)]++] = (unsigned)(2 * s + 1);
+    }
+  }
+  // the order of first naming (cells of no face last)
+  std::vector<int> orig, of((size_t)n, -1);
+  orig.reserve((size_t)n);
+  auto name = [&](int c) {
+    if (c < 0 || of[(size_t)c] >= 0) return;
+    of[(size_t)c] = (int)orig.size();
+    orig.push_back(c);
+  };
+  for (long long s = 0; s < nf; ++s) {
+    name(faces[2 * s] - base);
+    name(faces[2 * s + 1] - base);
+  }
+  for (int c = 0; c < n; ++c) name(c);
+  if (lines_touched(n, faces, base, ptr, inc, nullptr, nullptr) >
+      2 * lines_touched(n, faces, base, ptr, inc, &orig, &of)) {
+    out.reordered = true;
+    out.orig = std::move(orig);
+    out.of = std::move(of);
+  }
+  const int nslice = (n + 63) / 64;
+  out.off.assign((size_t)nslice + 1, 0);
+  bool tails = false;
+  auto cell = [&](int k) { return out.reordered ? out.orig[(size_t)k] : k; };
+  auto width = [&](int c) { return ptr[(size_t)c + 1] - ptr[(size_t)c]; };
+  for (int s = 0; s < nslice; ++s) {
+    int w = 0;
+    for (int k = 64 * s; k < std::min(n, 64 * s + 64); ++k) w = std::max(w, width(cell(k)));
+    tails = tails || w > kFaceSlots;
+    out.off[(size_t)s + 1] = out.off[(size_t)s] + 64LL * std::min(w, kFaceSlots);
+  }
+  out.inc.assign((size_t)out.off[(size_t)nslice], kNoFace);
+  if (tails) out.tptr.assign((size_t)n + 1, 0);
+  for (int k = 0; k < n; ++k) {
+    const int c = cell(k), w = width(c);
+    for (int j = 0; j < std::min(w, kFaceSlots); ++j)
+      out.inc[(size_t)(out.off[(size_t)(k / 64)] + 64LL * j + k % 64)] =
+          inc[(size_t)(ptr[(size_t)c] + j)];
+    for (int j = kFaceSlots; j < w; ++j) out.tail.push_back(inc[(size_t)(ptr[(size_t)c] + j)]);
+    if (tails) out.tptr[(size_t)k + 1] = (int)out.tail.size();
+  }
+}
+
 }  // namespace tfs

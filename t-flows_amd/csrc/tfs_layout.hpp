@@ -17,6 +17,7 @@
 //      first; the backward sweep reads the forward sweep's output in runs.
 #pragma once
 
+#include <cstddef>
 #include <vector>
 
 namespace tfs {
@@ -205,5 +206,32 @@ void build_blocks(int n, const int *row, const int *col, const int *dia,
 
 void build_layout(int n, const int *row, const int *col, const int *dia, int spmv_rows,
                   int spmv_cap, int small_level, Layout &out, bool identity_s = false);
+
+// The faces of every cell for the kernels that give a cell one lane: 64 cells a
+// slice, slot-major, so that a wavefront's list entries are one contiguous run.
+// An entry is 2 s + side (side 0: the cell is the face's first one), a cell's
+// entries ascend by face -- the order of the reference's face loops -- and
+// entries past kFaceSlots stand in a per-cell tail.
+// The cells' order is the caller's or, where that scatters, the order in which
+// the face list first names them: face lists follow the mesh's geometry even
+// where cells are numbered at random, and face arrays are then read in order
+// too.  Reordering pays with a pass in and out, so it has to halve the 128-byte
+// lines of a cell field and a face field that a slice touches (on a 96^3 box 42 in
+// lexicographic order, 707 in a random one, 42 in its first-named order).
+constexpr int kFaceSlots = 32;
+constexpr unsigned kNoFace = 0xffffffffu;
+struct FaceLists {
+  int n = 0;
+  bool reordered = false;
+  std::vector<int> orig, of;         // position <-> caller's cell, if reordered
+  std::vector<long long> off;        // entries before each slice, and in all
+  std::vector<unsigned> inc;         // slot j of lane l of slice s: off[s] + 64 j + l
+  std::vector<int> tptr;             // n + 1, empty if no cell has a tail
+  std::vector<unsigned> tail;
+  int at(int c) const { return reordered ? of[(std::size_t)c] : c; }
+};
+// faces: pairs (c1, c2) in 1..n (base 1) or 0..n-1 (base 0), c1 an interior cell,
+// c2 below that range for a boundary face; at most 2^31 entries in all.
+void build_face_lists(int n, long long nf, const int *faces, int base, FaceLists &out);
 
 }  // namespace tfs

@@ -99,3 +99,26 @@ extern "C" int tfs_layout_blocks(int n, const int *row, const int *col, const in
   }
   return B.nblk;
 }
+
+extern "C" int tfs_layout_faces(int n, long long nf, const int *faces, int base, int *order,
+                                int *first, unsigned *entry) {
+  if (n < 1 || nf < 0 || (nf > 0 && !faces) || !order || !first || !entry) return -1;
+  tfs::FaceLists F;
+  tfs::build_face_lists(n, nf, faces, base, F);
+  int at = 0;
+  for (int c = 0; c < n; ++c) {
+    const int k = F.at(c), s = k / 64;
+    const int wd = (int)((F.off[(std::size_t)s + 1] - F.off[(std::size_t)s]) / 64);
+    order[k] = c;
+    first[c] = at;
+    for (int j = 0; j < wd; ++j) {
+      const unsigned e = F.inc[(std::size_t)(F.off[(std::size_t)s] + 64LL * j + k % 64)];
+      if (e != tfs::kNoFace) entry[at++] = e;
+    }
+    if (!F.tptr.empty())
+      for (int t = F.tptr[(std::size_t)k]; t < F.tptr[(std::size_t)k + 1]; ++t)
+        entry[at++] = F.tail[(std::size_t)t];
+  }
+  first[n] = at;
+  return F.reordered ? 1 : 0;
+}

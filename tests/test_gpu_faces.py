@@ -1,0 +1,129 @@
+"""The device face loops (gradients, Correct_Velocity, both pressure face loops,
+assembly) bitwise against the oracle on meshes whose cells the face lists take
+in another order than the caller's, on cells of more faces than a slice has
+slots for, and at the edges of a slice."""
+import numpy as np
+import pytest
+
+from tflows_amd import mesh
+
+pytestmark = pytest.mark.gpu
+
+
+def box(nx, ny, nz, permute):
+    c = mesh.make_case(nx=nx, ny=ny, nz=nz, permute=permute, with_faces=True)
+    return c.n, c.faces
+
+
+def star(spokes):
+    """A cell of many faces, first or second in them, and a boundary face of every cell."""
+    n = spokes + 70
+    f = [(3, 4 + k) if k % 2 else (4 + k, 3) for k in range(1, spokes)]
+    f += [(k, -k) for k in range(1, n + 1)]
+    return n, np.array(f, np.int32).reshape(-1)
+
+
+MESHES = {
+    "one": lambda: box(1, 1, 1, False),
+    "slice": lambda: box(4, 4, 4, False),
+    "slice+1": lambda: box(13, 5, 1, True),
+    "ordered": lambda: box(37, 11, 29, False),
+    "reordered": lambda: box(31, 30, 17, True),
+    "slots": lambda: star(32),
+    "tails": lambda: star(150),
+}
+
+
+@pytest.fixture(scope="module")
+def S():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.fail("no GPU visible")
+    from tflows_amd import solvers
+    return solvers
+
+
+def dev(a):
+    import torch
+    return torch.from_numpy(np.array(np.ravel(a), np.float64)).cuda()
+
+
+def empty(n):
+    return dev(np.full(n, np.nan))
+
+
+@pytest.mark.parametrize("name", MESHES)
+@pytest.mark.parametrize("kinds", [(0,), (0, 1, 2), (0, 1, 2, 3)])
+def test_gradients_and_velocity(S, oracle, name, kinds):
+    n, faces = MESHES[name]()
+    nf, nb = faces.size // 2, int(max(0, -faces[1::2].min()))
+    print(f"face loops {name} n={n} nf={nf} kinds={kinds}", flush=True)
+    u = np.random.default_rng(len(kinds))
+    d, xc = u.standard_normal((3, nf)), u.standard_normal((3, n + nb))
+    bc = np.array(kinds, np.uint8)[u.integers(0, len(kinds), max(nb, 1))][:nb]
+    phi = u.uniform(-1, 1, n + nb)
+    G = S.Gradient(n, nb, faces, d, xc, bc)
+    g = oracle.gradient_matrix(n, faces, d)
+    assert np.array_equal(G.matrix(), g)
+    p = [empty(n) for _ in range(3)]
+    x = dev(phi)
+    G.grad_phi(x, *p)
+    for a, b in zip(p, oracle.graphi(n, faces, d, g, phi, bc)):
+        assert np.array_equal(a.cpu().numpy(), b)
+    G.grad_p(x, *p)
+    for a, b in zip([x] + p, oracle.gradp(n, faces, d, g, xc, phi, bc)):
+        assert np.array_equal(a.cpu().numpy(), b)
+
+    vol, sav, scoef = u.uniform(0.5, 1.5, n), u.uniform(0.5, 1.5, n), u.uniform(0.5, 1.5, nf)
+    grad = [u.uniform(-1, 1, n) for _ in range(3)]
+    vel = [u.uniform(-1, 1, n + nb) for _ in range(3)]
+    pp, coef, flux = u.uniform(-1, 1, n + nb), u.uniform(-1, 0, nf), u.uniform(-1, 1, nf)
+    den = np.full(n, 1.25)
+    # coef is that of interior faces; a boundary face's is not read
+    want = oracle.correct_velocity(n, faces, vol, sav, *grad, *vel, pp, coef, scoef, d, 0.01, 1e-3,
+                                   flux, den, bc)
+    got = dict(u=dev(vel[0]), v=dev(vel[1]), w=dev(vel[2]), flux=dev(flux), b=empty(n))
+    em, cm, pm = G.correct_velocity(dev(vol), dev(sav), *map(dev, grad), got["u"], got["v"],
+                                    got["w"], dev(pp), dev(coef), dev(den), dev(scoef), 0.01,
+                                    1e-3, got["flux"], got["b"])
+    for k, t in got.items():
+        assert np.array_equal(t.cpu().numpy(), want[k]), k
+    assert (em, cm, pm) == (want["errmax"], want["cfl"], want["pe"])
+
+
+@pytest.mark.parametrize("name", MESHES)
+def test_pressure_and_assembly(S, oracle, name):
+    import torch
+    n, faces = MESHES[name]()
+    nf, nb = faces.size // 2, int(max(0, -faces[1::2].min()))
+    print(f"pressure and assembly {name} n={n} nf={nf}", flush=True)
+    u = np.random.default_rng(5)
+    d = u.standard_normal((3, nf))
+    sv = d * u.uniform(0.5, 1.5, nf) + 0.1 * u.uniform(-1, 1, (3, nf))
+    bc = np.array((0, 1, 2, 4, 5, 6), np.uint8)[u.integers(0, 6, nb)]
+    f, vol, sav = u.uniform(0.3, 0.7, nf), u.uniform(0.5, 1.5, n), u.uniform(0.5, 1.5, n)
+    vel = [u.uniform(-1, 1, n + nb) for _ in range(3)]
+    grad = [u.uniform(-1, 1, n) for _ in range(3)]
+    p, den = u.uniform(-1, 1, n + nb), u.uniform(0.9, 1.1, n + nb)
+    row, col, dia, pos = mesh.topology(n, faces, base=1, with_pos=True)
+    A = S.Matrix(row - 1, col - 1, dia - 1)
+    asm = S.Assembly(A, faces, pos, dia, base=1)
+    G = S.Gradient(n, nb, faces, d, bc=bc)
+    flux, a12, b = empty(nf), empty(nf), empty(n)
+    args = [dev(a) for a in (f, sv, vol, sav, *vel, *grad, p, den)]
+    G.pressure_fractional(*args, flux, a12, b)
+    w = oracle.pressure_fractional(n, faces, f, sv, vol, sav, *vel, *grad, p, den)
+    for t, a in zip((flux, a12, b), w):
+        assert np.array_equal(t.cpu().numpy(), a)
+    asm.assemble(a12)
+    assert np.array_equal(A.get_values(), oracle.assemble(n, faces, pos, dia, len(col), w[1]))
+
+    flux, a12, b = empty(nf), empty(nf), empty(n)
+    on = torch.full((nf,), 7, dtype=torch.uint8, device="cuda")
+    G.pressure_simple(*args, flux, a12, on, b)
+    w = oracle.pressure_simple(n, faces, f, sv, d, vol, sav, *vel, p, *grad, den, bc, pos, dia,
+                               len(col))
+    for t, k in ((flux, "flux"), (a12, "a12"), (on, "bnd_on"), (b, "b")):
+        assert np.array_equal(t.cpu().numpy(), w[k]), k
+    asm.assemble(a12, bnd_on=on)
+    assert np.array_equal(A.get_values(), w["val"])
