@@ -577,13 +577,15 @@ k_ell_values(long long len, const int *__restrict__ src, const double *__restric
 // products left to right, as k_spmv and the reference do (Cg.f90:128-134,
 // Residual.f90:22-27) -- bitwise the same results -- but with every col/val
 // load of a wave one contiguous 256-byte run and no row pointers or LDS
-// staging.  Modes as k_spmv; the dot products are summed per workgroup.
+// staging.  Modes as k_spmv; the dot products are summed per workgroup.  `perm`
+// (plain and residual; may be null) is the caller's row of each row: y is then
+// the caller's array, without a pass into S order and one back.
 template <int MODE>
 __global__ void __launch_bounds__(kEllWaves * kWave)
 k_ell64(int n, int nslice, const long long *__restrict__ off, const int *__restrict__ col,
         const double *__restrict__ val, const double *__restrict__ x, double *__restrict__ y,
         const double *__restrict__ w, double *__restrict__ xs, double *__restrict__ rs,
-        const KState *st, double *partials, int xcd) {
+        const KState *st, double *partials, int xcd, const int *__restrict__ perm) {
   if (st && solve_done(st)) return;
   const int lane = threadIdx.x % kWave;
   const double alpha = MODE == SPMV_CGS_TAIL ? st->alpha : 0.0;
@@ -595,7 +597,8 @@ k_ell64(int n, int nslice, const long long *__restrict__ off, const int *__restr
     const int wd = (int)((off[su + 1] - e0) / kWave);
     const int i = su * kWave + lane;
     const bool live = i < n;
-    double acc = MODE == SPMV_RESID && live ? y[i] : 0.0;
+    const int at = (MODE == SPMV_PLAIN || MODE == SPMV_RESID) && perm && live ? perm[i] : i;
+    double acc = MODE == SPMV_RESID && live ? y[at] : 0.0;
     const long long base = e0 + lane;
     for (int j0 = 0; j0 < wd; j0 += kEllBatch) {
       int c[kEllBatch];
@@ -617,7 +620,7 @@ k_ell64(int n, int nslice, const long long *__restrict__ off, const int *__restr
         }
     }
     if (live) {
-      y[i] = acc;
+      y[at] = acc;
       if (MODE == SPMV_DOT) red += w[i] * acc;
       if (MODE == SPMV_CGS_TAIL) {
         xs[i] = xs[i] + alpha * x[i];

@@ -846,6 +846,20 @@ void build_bricks(int n, const int *row, const int *col, const int *dia,
   out.ok = true;
 }
 
+double gather_lines(int n, const int *row, const int *col) {
+  const int ngroup = (n + 63) / 64, step = std::max(1, ngroup / 256);
+  long long lines = 0;
+  int taken = 0;
+  std::vector<int> seen;
+  for (int g = 0; g < ngroup; g += step, ++taken) {
+    seen.clear();
+    for (int e = row[64 * g]; e < row[std::min(n, 64 * g + 64)]; ++e) seen.push_back(col[e] / 16);
+    std::sort(seen.begin(), seen.end());
+    lines += std::unique(seen.begin(), seen.end()) - seen.begin();
+  }
+  return taken ? (double)lines / taken : 0.0;
+}
+
 void build_layout(int n, const int *row, const int *col, const int *dia, int spmv_rows,
                   int spmv_cap, int small_level, Layout &out, bool identity_s) {
   out.n = n;

@@ -204,6 +204,10 @@ constexpr int kBlockGain = 4, kBlockLevels = 24;
 void build_blocks(int n, const int *row, const int *col, const int *dia,
                   const std::vector<int> &s_of_orig, int nlev, BlockLayout &out);
 
+// Average number of 128-byte lines of x that 64 consecutive rows gather from, over
+// up to 256 such groups spread over the matrix.
+double gather_lines(int n, const int *row, const int *col);
+
 void build_layout(int n, const int *row, const int *col, const int *dia, int spmv_rows,
                   int spmv_cap, int small_level, Layout &out, bool identity_s = false);
 
