@@ -388,20 +388,17 @@ k_pf_cells(int n, long long na, const int *__restrict__ of, const double *__rest
            const double *__restrict__ den, double *__restrict__ rec) {
   for (long long c = blockIdx.x * (long long)kThreads + threadIdx.x; c < na;
        c += (long long)gridDim.x * kThreads) {
-    double *r = rec + R * (of && c < n ? (long long)of[c] : c);
+    double r[R] = {u[c], v[c], w[c], 0.0, p[c], den[c]};
     if (c < n) {
       r[0] = u[c] + px[c] * vol[c] / sav[c];
       r[1] = v[c] + py[c] * vol[c] / sav[c];
       r[2] = w[c] + pz[c] * vol[c] / sav[c];
       r[3] = sav[c];
-    } else {
-      r[0] = u[c];
-      r[1] = v[c];
-      r[2] = w[c];
-      r[3] = 0.0;
     }
-    r[4] = p[c];
-    r[5] = den[c];
+    double2 *const to =
+        reinterpret_cast<double2 *>(rec + R * (of && c < n ? (long long)of[c] : c));
+#pragma unroll
+    for (int j = 0; j < R / 2; ++j) to[j] = make_double2(r[2 * j], r[2 * j + 1]);
   }
 }
 
