@@ -59,7 +59,10 @@ enum Epi {
 // (Cg.f90:148-153, Cgs.f90:157-162); cgs tail: q2 = A p1, xs += alpha p1,
 // rs -= alpha q2 and partial ||rs||^2 (Cgs.f90:182-221, row-local once alpha
 // is known).
-enum SpmvMode { SPMV_PLAIN = 0, SPMV_RESID, SPMV_DOT, SPMV_CGS_TAIL };
+// pdot (k_ell64): the dot mode with p = z + beta p (Cg.f90:114-123) formed where it
+// is gathered -- x is z, w the old p and xs the new one, another array -- which
+// saves a pass and a launch for a second gather.
+enum SpmvMode { SPMV_PLAIN = 0, SPMV_RESID, SPMV_DOT, SPMV_CGS_TAIL, SPMV_PDOT };
 
 // Reductions that run whatever the solve's state (the rest return at once
 // once the solve is done).
@@ -124,11 +127,54 @@ __device__ inline void epilogue(int epi, double tot, KState *st) {
   }
 }
 
+template <typename T>
+__device__ __forceinline__ T coherent_load(const T *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void coherent_store(T *p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 template <int NT>
 __device__ __forceinline__ void store_partial(double v, double *partials) {
   __shared__ double lds[NT / kWave];
   const double s = block_sum<NT>(v, lds);
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
+}
+
+// store_partial, and with `fin` k_finish with it: the workgroup that stores last
+// sums the partials in k_finish's order and applies the state transition, which
+// saves a launch.  A partial is stored past the caches and has arrived before its
+// workgroup counts itself, so no cache is written back; the last one reads them
+// past the caches.  The workgroups meet at one counter, which costs more than the
+// launch where there are many (kFuseGrid).  NT is k_finish's workgroup, so the
+// sum is the same bit for bit.
+template <int NT>
+__device__ __forceinline__ void finish_partial(double v, double *partials, int epi, KState *fin) {
+  if (!fin) {
+    store_partial<NT>(v, partials);
+    return;
+  }
+  static_assert(NT == kRedThreads, "sums in k_finish's order");
+  __shared__ double lds[NT / kWave];
+  __shared__ int last;
+  const double s = block_sum<NT>(v, lds);
+  if (threadIdx.x == 0) {
+    coherent_store(&partials[blockIdx.x], s);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = __hip_atomic_fetch_add(&fin->ctr[1], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+           gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  double t = 0.0;
+  for (int k = threadIdx.x; k < (int)gridDim.x; k += NT) t += coherent_load(&partials[k]);
+  t = block_sum<NT>(t, lds);
+  if (threadIdx.x == 0) {
+    fin->ctr[1] = 0u;
+    epilogue(epi, t, fin);
+  }
 }
 
 // Sums the partials of the previous kernel in index order and applies the
@@ -151,14 +197,14 @@ k_finish(int nparts, const double *__restrict__ partials, int epi, KState *st) {
 
 template <typename T>
 __global__ void __launch_bounds__(kRedThreads)
-k_sumsq(int n, const T *__restrict__ v, int epi, const KState *st, double *partials) {
+k_sumsq(int n, const T *__restrict__ v, int epi, const KState *st, double *partials, KState *fin) {
   if (!epi_always(epi) && solve_done(st)) return;
   double s = 0.0;
   TFS_GRID_STRIDE(i, n) {
     const double a = v[i];
     s += a * a;
   }
-  store_partial<kRedThreads>(s, partials);
+  finish_partial<kRedThreads>(s, partials, epi, fin);
 }
 
 // Plain dot product with per-workgroup partials (outer loop of the
@@ -198,7 +244,7 @@ template <typename T>
 __global__ void __launch_bounds__(kRedThreads)
 k_rho(int n, const T *__restrict__ r, T *__restrict__ z, const T *__restrict__ d,
       const T *__restrict__ zU, const int *__restrict__ s_to_u, int mode, const KState *st,
-      double *partials) {
+      double *partials, KState *fin) {
   if (solve_done(st)) return;
   double s = 0.0;
   TFS_GRID_STRIDE(i, n) {
@@ -222,7 +268,7 @@ k_rho(int n, const T *__restrict__ r, T *__restrict__ z, const T *__restrict__ d
     }
     s += (double)ri * (double)zi;
   }
-  store_partial<kRedThreads>(s, partials);
+  finish_partial<kRedThreads>(s, partials, EPI_RHO, fin);
 }
 
 // p = z (first iteration) or p = z + beta p  (Cg.f90:114-123)
@@ -253,7 +299,7 @@ k_pupdate_rev(int n, const T *__restrict__ zU, T *__restrict__ p, const KState *
 template <typename T>
 __global__ void __launch_bounds__(kRedThreads)
 k_axpy_norm(int n, T *__restrict__ x, T *__restrict__ r, const T *__restrict__ p,
-            const T *__restrict__ q, const KState *st, double *partials) {
+            const T *__restrict__ q, const KState *st, double *partials, KState *fin) {
   if (solve_done(st)) return;
   const T alpha = (T)st->alpha;
   double s = 0.0;
@@ -263,7 +309,7 @@ k_axpy_norm(int n, T *__restrict__ x, T *__restrict__ r, const T *__restrict__ p
     r[i] = ri;
     s += (double)ri * (double)ri;
   }
-  store_partial<kRedThreads>(s, partials);
+  finish_partial<kRedThreads>(s, partials, EPI_NORM, fin);
 }
 
 // CGS: u1 = r1 + beta q1; u2 = u1 + beta (q1 + beta u2)  (Cgs.f90:115-126)
@@ -585,10 +631,16 @@ __global__ void __launch_bounds__(kEllWaves * kWave)
 k_ell64(int n, int nslice, const long long *__restrict__ off, const int *__restrict__ col,
         const double *__restrict__ val, const double *__restrict__ x, double *__restrict__ y,
         const double *__restrict__ w, double *__restrict__ xs, double *__restrict__ rs,
-        const KState *st, double *partials, int xcd, const int *__restrict__ perm) {
+        const KState *st, double *partials, int xcd, const int *__restrict__ perm, KState *fin) {
   if (st && solve_done(st)) return;
   const int lane = threadIdx.x % kWave;
   const double alpha = MODE == SPMV_CGS_TAIL ? st->alpha : 0.0;
+  const bool first = MODE == SPMV_PDOT && st->iter == 0;
+  const double beta = MODE == SPMV_PDOT ? st->beta : 0.0;
+  auto at_x = [&](int c) {
+    if (MODE != SPMV_PDOT || first) return x[c];
+    return x[c] + beta * w[c];
+  };
   double red = 0.0;
   const SliceWalk sw(nslice, xcd != 0);
   for (int s = sw.first; s < sw.end; s += sw.step) {
@@ -611,7 +663,7 @@ k_ell64(int n, int nslice, const long long *__restrict__ off, const int *__restr
         }
 #pragma unroll
       for (int k = 0; k < kEllBatch; ++k)
-        if (j0 + k < wd) xv[k] = c[k] >= 0 ? x[c[k]] : 0.0;
+        if (j0 + k < wd) xv[k] = c[k] >= 0 ? at_x(c[k]) : 0.0;
 #pragma unroll
       for (int k = 0; k < kEllBatch; ++k)
         if (j0 + k < wd && c[k] >= 0) {
@@ -622,6 +674,11 @@ k_ell64(int n, int nslice, const long long *__restrict__ off, const int *__restr
     if (live) {
       y[at] = acc;
       if (MODE == SPMV_DOT) red += w[i] * acc;
+      if (MODE == SPMV_PDOT) {
+        const double p = at_x(i);
+        xs[i] = p;
+        red += p * acc;
+      }
       if (MODE == SPMV_CGS_TAIL) {
         xs[i] = xs[i] + alpha * x[i];
         const double ri = rs[i] - alpha * acc;
@@ -630,8 +687,9 @@ k_ell64(int n, int nslice, const long long *__restrict__ off, const int *__restr
       }
     }
   }
-  if (MODE == SPMV_DOT || MODE == SPMV_CGS_TAIL)
-    store_partial<kEllWaves * kWave>(red, partials);
+  if (MODE == SPMV_DOT || MODE == SPMV_CGS_TAIL || MODE == SPMV_PDOT)
+    finish_partial<kEllWaves * kWave>(red, partials, MODE == SPMV_CGS_TAIL ? EPI_NORM : EPI_ALPHA,
+                                      fin);
 }
 
 // Row sums of the operator, summed in FP64 over the caller's entries of each
@@ -1056,15 +1114,6 @@ template <> struct Sentinel<float> {
   __device__ static float value() { return __int_as_float((int)bits); }
   __device__ static bool is(float v) { return (unsigned int)__float_as_int(v) == bits; }
 };
-
-template <typename T>
-__device__ __forceinline__ T coherent_load(const T *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ void coherent_store(T *p, T v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // One row of a sweep, as a thread holds it.
 template <typename T>

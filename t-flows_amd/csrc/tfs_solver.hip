@@ -358,9 +358,18 @@ template <typename T>
 void arm(int n, T *x) {
   hipLaunchKernelGGL(k_arm<T>, dim3(vgrid(n)), dim3(kRedThreads), 0, cur_stream(), n, x);
 }
+// The sums of a kernel of at most this many workgroups end in the kernel itself
+// (finish_partial); k_finish sums those of larger ones.  Cg of 12^3 cells: 2376 us
+// with k_finish and k_pupdate, 2198 us without; 32^3 the same either way; with both
+// limits at 443 k rows 97x75x61 took 96.8 ms against 93.8.
+constexpr int kFuseGrid = 128;
+inline KState *fused(int grid, KState *st) { return grid <= kFuseGrid ? st : nullptr; }
 void finish(int nparts, const double *partials, int epi, KState *st) {
   hipLaunchKernelGGL(k_finish, dim3(1), dim3(kRedThreads), 0, cur_stream(), nparts, partials, epi,
                      st);
+}
+void finish_rest(int nparts, const double *partials, int epi, KState *st) {
+  if (!fused(nparts, st)) finish(nparts, partials, epi, st);
 }
 template <typename T>
 Values<T> &vals(tfs_matrix *A);
@@ -629,13 +638,13 @@ void prec_apply_S(tfs_matrix *A, int prec, const T *bS, T *xS, T *yL, T *zU, con
 
 template <typename T, int MODE>
 void launch_spmv(tfs_matrix *A, const T *x, T *y, const T *w, T *xs, T *rs, const KState *st,
-                 const int *perm = nullptr) {
+                 const int *perm = nullptr, KState *fin = nullptr) {
   tm_begin(TFS_KC_SPMV);
   if constexpr (sizeof(T) == 8) {
     if (A->e64_len > 0) {
       hipLaunchKernelGGL(k_ell64<MODE>, dim3(ell64_grid(A)), dim3(kEllWaves * kWave), 0,
                          cur_stream(), A->n, A->e64_nslice, A->e64_off, A->e64_col, A->e64_val,
-                         x, y, w, xs, rs, st, A->partials, kEll64Xcd, perm);
+                         x, y, w, xs, rs, st, A->partials, kEll64Xcd, perm, fin);
       tm_end(TFS_KC_SPMV);
       return;
     }
@@ -763,30 +772,58 @@ bool cg_precondition(tfs_matrix *A, const T *r, T *yL, T *zU, T *z, const KState
 
 // One CG iteration (Cg.f90:97-178) in precision T; Bicg takes the same path
 // (its shadow sequence equals the primary one bit for bit, Bicg.f90:91-175).
+// p = z + beta p, q = A p and (p, q).  Up to kGatherP rows p is formed in the
+// product (a second gather from the caches costs less than a launch); V.p and
+// V.r2 then change places.  Above, in a pass of its own (figures at kFuseGrid).
+constexpr int kGatherP = 1 << 16;
 template <typename T>
-void cg_iteration(tfs_matrix *A, int prec, const Vecs<T> &V, KState *st) {
+inline bool gathers_p(const tfs_matrix *A) {
+  return sizeof(T) == 8 && A->e64_len > 0 && A->n <= kGatherP;
+}
+
+template <typename T>
+void cg_product(tfs_matrix *A, const T *z, Vecs<T> &V, KState *st) {
+  const int parts = spmv_parts<T>(A);
+  KState *fin = sizeof(T) == 8 && A->e64_len > 0 ? fused(parts, st) : nullptr;
+  if constexpr (sizeof(T) == 8) {
+    if (gathers_p<T>(A)) {
+      launch_spmv<T, SPMV_PDOT>(A, z, V.q, V.p, V.r2, nullptr, st, nullptr, fin);
+      std::swap(V.p, V.r2);
+      if (!fin) finish(parts, A->partials, EPI_ALPHA, st);
+      return;
+    }
+  }
+  hipLaunchKernelGGL(k_pupdate<T>, dim3(vgrid(A->n)), dim3(kRedThreads), 0, cur_stream(), A->n, z,
+                     V.p, st);
+  launch_spmv<T, SPMV_DOT>(A, V.p, V.q, V.p, nullptr, nullptr, st, nullptr, fin);
+  if (!fin) finish(parts, A->partials, EPI_ALPHA, st);
+}
+
+// One CG iteration (Cg.f90:97-178) in precision T; Bicg takes the same path
+// (its shadow sequence equals the primary one bit for bit, Bicg.f90:91-175).
+template <typename T>
+void cg_iteration(tfs_matrix *A, int prec, Vecs<T> &V, KState *st) {
   const int n = A->n, g = vgrid(n);
   const bool have_z = prec == 2 && cg_precondition<T>(A, V.r, V.yL, V.zU, V.z, st);
   const int mode =
       have_z ? 3 : prec == 2 ? (z_reversed<T>(A) ? 4 : 2) : prec == 1 ? 1 : 0;
   T *z = prec == 0 ? V.r : V.z;  // prec 0: z is a copy of r (Prec_Solve.f90:72-75)
   hipLaunchKernelGGL(k_rho<T>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, V.r, V.z,
-                     vals<T>(A).s_diag, V.zU, z_of_s<T>(A), mode, st, A->partials);
-  finish(g, A->partials, EPI_RHO, st);
-  hipLaunchKernelGGL(k_pupdate<T>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, z, V.p, st);
-  launch_spmv<T, SPMV_DOT>(A, V.p, V.q, V.p, nullptr, nullptr, st);
-  finish(spmv_parts<T>(A), A->partials, EPI_ALPHA, st);
+                     vals<T>(A).s_diag, V.zU, z_of_s<T>(A), mode, st, A->partials, fused(g, st));
+  finish_rest(g, A->partials, EPI_RHO, st);
+  cg_product<T>(A, z, V, st);
   hipLaunchKernelGGL(k_axpy_norm<T>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, V.x, V.r,
-                     V.p, V.q, st, A->partials);
-  finish(g, A->partials, EPI_NORM, st);
+                     V.p, V.q, st, A->partials, fused(g, st));
+  finish_rest(g, A->partials, EPI_NORM, st);
 }
 
 // One CGS iteration (Cgs.f90:104-226), FP64.
 void cgs_iteration(tfs_matrix *A, int prec, const Vecs<double> &V, KState *st) {
-  const int n = A->n, g = vgrid(n);
+  const int n = A->n, g = vgrid(n), parts = spmv_parts<double>(A);
+  KState *fin = A->e64_len > 0 ? fused(parts, st) : nullptr;
   hipLaunchKernelGGL(k_rho<double>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, V.r, V.r2,
-                     nullptr, nullptr, nullptr, 3, st, A->partials);  // rho = (r1, r2)
-  finish(g, A->partials, EPI_RHO, st);
+                     nullptr, nullptr, nullptr, 3, st, A->partials, fused(g, st));  // rho = (r1, r2)
+  finish_rest(g, A->partials, EPI_RHO, st);
   hipLaunchKernelGGL(k_cgs_u, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, V.r, V.q1, V.u1,
                      V.u2, st);
   double *pp2 = V.u2;  // prec 0: p2 is a copy of u2
@@ -794,8 +831,9 @@ void cgs_iteration(tfs_matrix *A, int prec, const Vecs<double> &V, KState *st) {
     prec_apply_S<double>(A, prec, V.u2, V.p2, V.yL, V.zU, st);
     pp2 = V.p2;
   }
-  launch_spmv<double, SPMV_DOT>(A, pp2, V.v2, V.r2, nullptr, nullptr, st);  // v2 = A p2, (r2,v2)
-  finish(spmv_parts<double>(A), A->partials, EPI_ALPHA, st);
+  // v2 = A p2, (r2, v2)
+  launch_spmv<double, SPMV_DOT>(A, pp2, V.v2, V.r2, nullptr, nullptr, st, nullptr, fin);
+  if (!fin) finish(parts, A->partials, EPI_ALPHA, st);
   hipLaunchKernelGGL(k_cgs_q, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, V.u1, V.v2, V.q1,
                      V.w, st);
   double *pp1 = V.w;
@@ -804,8 +842,8 @@ void cgs_iteration(tfs_matrix *A, int prec, const Vecs<double> &V, KState *st) {
     pp1 = V.p1;
   }
   // q2 = A p1 into the v2 slot (v2 is dead once q1 and w are formed)
-  launch_spmv<double, SPMV_CGS_TAIL>(A, pp1, V.v2, nullptr, V.x, V.r, st);
-  finish(spmv_parts<double>(A), A->partials, EPI_NORM, st);
+  launch_spmv<double, SPMV_CGS_TAIL>(A, pp1, V.v2, nullptr, V.x, V.r, st, nullptr, fin);
+  if (!fin) finish(parts, A->partials, EPI_NORM, st);
 }
 
 // A persistent sweep that gave up waiting leaves a flag: report it (the
@@ -894,9 +932,9 @@ int solve_device(tfs_matrix *A, int method, int prec, double *x, double *r1, int
     return TFS_OK;
   }
   if (!x || !r1) return TFS_ERR_INVALID;
-  TFS_TRY(ensure_vec64(A, method == TFS_CGS ? 12 : 7));
+  TFS_TRY(ensure_vec64(A, method == TFS_CGS ? 12 : gathers_p<double>(A) ? 8 : 7));
   TFS_TRY(prec_form<double>(A, prec));  // Cg.f90:42 (kept while the values are unchanged)
-  const Vecs<double> V = vecs_of(A->vec64, n);
+  Vecs<double> V = vecs_of(A->vec64, n);
   KState *st = A->d_st;
   TFS_TRY(init_state(A, 0, tol, cap, *ini_res));
   const int g = vgrid(n);
@@ -905,13 +943,13 @@ int solve_device(tfs_matrix *A, int method, int prec, double *x, double *r1, int
   gather(n, r1, A->s_orig, V.r);
   // ||b|| and its early exit; r = b - A x; ||r|| and its early exit
   hipLaunchKernelGGL(k_sumsq<double>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, V.r,
-                     (int)EPI_BNRM, st, A->partials);
-  finish(g, A->partials, EPI_BNRM, st);
+                     (int)EPI_BNRM, st, A->partials, fused(g, st));
+  finish_rest(g, A->partials, EPI_BNRM, st);
   launch_spmv<double, SPMV_RESID>(A, V.x, V.r, nullptr, nullptr, nullptr, st);
   if (method == TFS_CGS) gather(n, V.r, (const int *)nullptr, V.r2, st);  // r2 = r1 (Cgs.f90:75-77)
   hipLaunchKernelGGL(k_sumsq<double>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, V.r,
-                     (int)EPI_INIRES, st, A->partials);
-  finish(g, A->partials, EPI_INIRES, st);
+                     (int)EPI_INIRES, st, A->partials, fused(g, st));
+  finish_rest(g, A->partials, EPI_INIRES, st);
   TFS_HIP(hipGetLastError());
   TFS_TRY(read_state(A));
   if (method == TFS_CGS)
@@ -1357,7 +1395,7 @@ void reliable_iteration(tfs_matrix *I, int prec, const Vecs<float> &F, double *c
         prec == 2 && cg_precondition<float>(I, F.r, F.yL, F.zU, F.z, st);
     const int mode = have_z ? 3 : prec == 2 ? (zrev ? 5 : 2) : prec == 1 ? 1 : 0;
     hipLaunchKernelGGL(k_rho<float>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, F.r, F.z,
-                       vals<float>(I).s_diag, F.zU, I->s_to_u, mode, st, I->partials);
+                       vals<float>(I).s_diag, F.zU, I->s_to_u, mode, st, I->partials, nullptr);
     finish(g, I->partials, EPI_RHO, st);
   }
   if (zrev)
@@ -1434,7 +1472,7 @@ int solve_reliable_device(tfs_matrix *A, int prec, double *x, double *r1, int *n
     gather(n, bS, (const int *)nullptr, D.r);
     launch_spmv<double, SPMV_RESID>(A, D.x, D.r, nullptr, nullptr, nullptr, nullptr);
     hipLaunchKernelGGL(k_sumsq<double>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, D.r,
-                       (int)EPI_BNRM, A->d_st + 1, A->partials);
+                       (int)EPI_BNRM, A->d_st + 1, A->partials, nullptr);
     finish(g, A->partials, EPI_BNRM, A->d_st + 1);
     TFS_HIP(hipGetLastError());
     return read_state(A, 1);
@@ -1584,7 +1622,7 @@ int solve_mixed_device(tfs_matrix *A, int prec, double *x, double *r1, int *nite
   // sweep slots (yL, zU) are not touched: they stay armed for FP64 solves.
   const Vecs<double> D = vecs_of(A->vec64, n);
   double *bS = D.r2;
-  const Vecs<float> F = vecs_of(I->vec32, n);    // inner solve: x = correction
+  Vecs<float> F = vecs_of(I->vec32, n);    // inner solve: x = correction
   KState *so = A->d_st + 1, *si = I->d_st;
   KState *ho = A->h_st + 1;
   const int g = vgrid(n);
@@ -1597,7 +1635,7 @@ int solve_mixed_device(tfs_matrix *A, int prec, double *x, double *r1, int *nite
   };
   auto sumsq = [&](const double *u, int epi) {
     hipLaunchKernelGGL(k_sumsq<double>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, u, epi,
-                       so, A->partials);
+                       so, A->partials, nullptr);
     finish(g, A->partials, epi, so);
   };
   // true residual r = b - A x and its norm (FP64) into bnrm2; with
@@ -1606,7 +1644,7 @@ int solve_mixed_device(tfs_matrix *A, int prec, double *x, double *r1, int *nite
     TFS_TRY(init_state(A, 1, tol, cap, 0.0));
     if (update_norms) {
       hipLaunchKernelGGL(k_sumsq<float>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, F.x,
-                         (int)EPI_NAUX4, so, A->partials);
+                         (int)EPI_NAUX4, so, A->partials, nullptr);
       finish(g, A->partials, EPI_NAUX4, so);
       sumsq(D.x, EPI_NAUX5);
     }
@@ -1636,7 +1674,7 @@ int solve_mixed_device(tfs_matrix *A, int prec, double *x, double *r1, int *nite
     hipLaunchKernelGGL(k_fill<float>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, F.x, 0.0f);
     TFS_TRY(init_state(I, 0, inner_tol, 100000, 0.0));
     hipLaunchKernelGGL(k_sumsq<float>, dim3(g), dim3(kRedThreads), 0, cur_stream(), n, F.r,
-                       (int)EPI_INIRES, si, I->partials);
+                       (int)EPI_INIRES, si, I->partials, nullptr);
     finish(g, I->partials, EPI_INIRES, si);
     TFS_HIP(hipGetLastError());
     TFS_TRY(read_state(I));
