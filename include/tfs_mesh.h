@@ -120,6 +120,11 @@ int tfs_layout_brick_colour(int n, const int *row, const int *col, const int *di
 int tfs_layout_blocks(int n, const int *row, const int *col, const int *dia, int *order,
                       int *block_of, int *step_of);
 
+/* The columns of a sliced ELL (slot-major, 64 rows a slice, off[s] slots before
+ * slice s) through their 16-bit codes and back into out.  Returns 1, 0 where a
+ * slice needs more windows than a code names, -1 on an invalid argument. */
+int tfs_layout_short_columns(int nslice, const long long *off, const int *col, int *out);
+
 /* The cells' face lists of the device face loops (pairs c1, c2 numbered from
  * base, c2 below base a boundary face): order[k] = cell at position k, and per
  * cell first[c] .. first[c + 1] its entries 2 face + side in the order they are

@@ -487,9 +487,20 @@ struct SliceWalk {
 };
 constexpr int kEllBatch = 8;  // entries per lane loaded before their gathers
 
-template <bool DOT>
+// The columns, either as they are or as 16-bit codes (tfs_layout.hpp), whose
+// windows' first rows lie in the lanes of a register.  The codes take 12 bytes a
+// row instead of 24 of the 60 that a hex mesh's row moves.  On MI355X 256^3 in
+// 16^3 bricks 219 -> 178 us, a batch of 7.8 M rows 98 -> 84 us.
+struct EllColumns {
+  const int *__restrict__ col;                            // or null:
+  const int *__restrict__ window;
+  const long long *__restrict__ off;
+  const unsigned *__restrict__ code;
+};
+
+template <bool DOT, bool SHORT>
 __global__ void __launch_bounds__(kEllWaves * kWave)
-k_ell_diff(int n, int nslice, const long long *__restrict__ off, const int *__restrict__ col,
+k_ell_diff(int n, int nslice, const long long *__restrict__ off, EllColumns C,
            const float *__restrict__ val, const float *__restrict__ rsum,
            const float *__restrict__ x, float *__restrict__ y, const KState *st,
            double *partials, int xcd) {
@@ -501,6 +512,8 @@ k_ell_diff(int n, int nslice, const long long *__restrict__ off, const int *__re
     const int su = __builtin_amdgcn_readfirstlane(s);
     const long long e0 = off[su];
     const int w = (int)((off[su + 1] - e0) / kWave);
+    const long long q0 = SHORT ? C.off[su] + lane : 0;
+    const int window = SHORT ? C.window[su * kWindows + lane % kWindows] : 0;
     const int i = su * kWave + lane;
     const bool live = i < n;
     const double xi = live ? (double)x[i] : 0.0;
@@ -509,12 +522,28 @@ k_ell_diff(int n, int nslice, const long long *__restrict__ off, const int *__re
     for (int j0 = 0; j0 < w; j0 += kEllBatch) {
       int c[kEllBatch];
       float a[kEllBatch], xv[kEllBatch];
+      if (SHORT) {
+        unsigned code[kEllBatch / 2];
 #pragma unroll
-      for (int k = 0; k < kEllBatch; ++k)
-        if (j0 + k < w) {
-          c[k] = col[base + (long long)(j0 + k) * kWave];
-          a[k] = val[base + (long long)(j0 + k) * kWave];
-        }
+        for (int k = 0; k < kEllBatch; k += 2)
+          if (j0 + k < w) code[k / 2] = C.code[q0 + (long long)((j0 + k) / 2) * kWave];
+#pragma unroll
+        for (int k = 0; k < kEllBatch; ++k)
+          if (j0 + k < w) a[k] = val[base + (long long)(j0 + k) * kWave];
+#pragma unroll
+        for (int k = 0; k < kEllBatch; ++k)
+          if (j0 + k < w) {
+            const unsigned h = k % 2 ? code[k / 2] >> 16 : code[k / 2] & 0xffffu;
+            c[k] = __shfl(window, (int)(h >> 12)) + (int)(h & 0xfffu);
+          }
+      } else {
+#pragma unroll
+        for (int k = 0; k < kEllBatch; ++k)
+          if (j0 + k < w) {
+            c[k] = C.col[base + (long long)(j0 + k) * kWave];
+            a[k] = val[base + (long long)(j0 + k) * kWave];
+          }
+      }
 #pragma unroll
       for (int k = 0; k < kEllBatch; ++k)
         if (j0 + k < w) xv[k] = x[c[k]];

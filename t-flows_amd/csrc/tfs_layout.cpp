@@ -846,6 +846,40 @@ void build_bricks(int n, const int *row, const int *col, const int *dia,
   out.ok = true;
 }
 
+void short_columns(const std::vector<long long> &off, const std::vector<int> &col,
+                   ShortColumns &out) {
+  out = ShortColumns();
+  const size_t ns = off.size() - 1;
+  out.window.assign(ns * kWindows, 0);
+  out.off.assign(ns + 1, 0);
+  for (size_t s = 0; s < ns; ++s) {
+    const long long w = (off[s + 1] - off[s]) / 64;
+    out.off[s + 1] = out.off[s] + 64 * ((w + 1) / 2);
+  }
+  out.code.assign((size_t)out.off[ns], 0);
+  std::vector<int> seen;
+  for (size_t s = 0; s < ns; ++s) {
+    // each window starts at the smallest column that none before it holds
+    seen.assign(col.begin() + (long)off[s], col.begin() + (long)off[s + 1]);
+    std::sort(seen.begin(), seen.end());
+    int *const first = &out.window[s * kWindows];
+    int nw = 0;
+    for (const int c : seen)
+      if (nw == 0 || c - first[nw - 1] >= kWindow) {
+        if (nw == kWindows) return;
+        first[nw++] = c;
+      }
+    for (long long i = off[s]; i < off[s + 1]; ++i) {
+      const int c = col[(size_t)i];
+      const int k = (int)(std::upper_bound(first, first + nw, c) - first) - 1;
+      const long long slot = (i - off[s]) / 64, lane = (i - off[s]) % 64;
+      out.code[(size_t)(out.off[s] + 64 * (slot / 2) + lane)] |=
+          ((unsigned)k << 12 | (unsigned)(c - first[k])) << (slot % 2 ? 16 : 0);
+    }
+  }
+  out.ok = true;
+}
+
 double gather_lines(int n, const int *row, const int *col) {
   const int ngroup = (n + 63) / 64, step = std::max(1, ngroup / 256);
   long long lines = 0;

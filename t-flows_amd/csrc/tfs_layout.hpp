@@ -204,6 +204,21 @@ constexpr int kBlockGain = 4, kBlockLevels = 24;
 void build_blocks(int n, const int *row, const int *col, const int *dia,
                   const std::vector<int> &s_of_orig, int nlev, BlockLayout &out);
 
+// Columns of a sliced ELL (64 rows a slice, slot-major) in 16 bits: a slice's
+// columns fall in at most kWindows windows of kWindow rows each, a code is 4 bits
+// of window and 12 of place in it, two consecutive slots in one word (the first
+// in the low half).  Not ok where some slice needs more windows.
+constexpr int kWindows = 16, kWindow = 4096;
+struct ShortColumns {
+  bool ok = false;
+  std::vector<int> window;           // kWindows first rows per slice
+  std::vector<long long> off;        // words before each slice, and in all
+  std::vector<unsigned> code;        // slots 2 q, 2 q + 1 of lane l: off[s] + 64 q + l
+};
+// off: slots before each slice and in all; col: their columns, none negative.
+void short_columns(const std::vector<long long> &off, const std::vector<int> &col,
+                   ShortColumns &out);
+
 // Average number of 128-byte lines of x that 64 consecutive rows gather from, over
 // up to 256 such groups spread over the matrix.
 double gather_lines(int n, const int *row, const int *col);

@@ -122,3 +122,20 @@ extern "C" int tfs_layout_faces(int n, long long nf, const int *faces, int base,
   first[n] = at;
   return F.reordered ? 1 : 0;
 }
+
+extern "C" int tfs_layout_short_columns(int nslice, const long long *off, const int *col,
+                                        int *out) {
+  if (nslice < 0 || !off || (off[nslice] > 0 && (!col || !out))) return -1;
+  tfs::ShortColumns S;
+  tfs::short_columns(std::vector<long long>(off, off + nslice + 1),
+                     std::vector<int>(col, col + off[nslice]), S);
+  if (!S.ok) return 0;
+  for (int s = 0; s < nslice; ++s)
+    for (long long i = off[s]; i < off[s + 1]; ++i) {
+      const long long slot = (i - off[s]) / 64, lane = (i - off[s]) % 64;
+      const unsigned h = S.code[(std::size_t)(S.off[(std::size_t)s] + 64 * (slot / 2) + lane)] >>
+                             (slot % 2 ? 16 : 0) & 0xffffu;
+      out[i] = S.window[(std::size_t)s * tfs::kWindows + (h >> 12)] + (int)(h & 0xfffu);
+    }
+  return 1;
+}

@@ -226,7 +226,10 @@ struct tfs_matrix {
   int ell_nslice = 0;
   long long ell_len = 0;
   long long *ell_off = nullptr;
-  int *ell_col = nullptr, *ell_src = nullptr;
+  int *ell_col = nullptr, *ell_src = nullptr;  // ell_col null: codes
+  int *ell_window = nullptr;
+  long long *ell_coff = nullptr;
+  unsigned *ell_code = nullptr;
   float *ell_val = nullptr, *ell_rsum = nullptr;
   bool ell_ready = false;
   // FP64 SpMV over a sliced ELL of all entries in S order (k_ell64); absent
@@ -1002,7 +1005,15 @@ int build_ell(tfs_matrix *A, const Layout &Ly) {
   A->ell_nslice = ns;
   A->ell_len = len;
   TFS_TRY(upload(A, &A->ell_off, off));
-  TFS_TRY(upload(A, &A->ell_col, ecol));
+  ShortColumns sc;
+  short_columns(off, ecol, sc);
+  if (sc.ok) {
+    TFS_TRY(upload(A, &A->ell_window, sc.window));
+    TFS_TRY(upload(A, &A->ell_coff, sc.off));
+    TFS_TRY(upload(A, &A->ell_code, sc.code));
+  } else {
+    TFS_TRY(upload(A, &A->ell_col, ecol));
+  }
   TFS_TRY(upload(A, &A->ell_src, esrc));
   TFS_TRY(dev_alloc(A, (void **)&A->ell_val, sizeof(float) * (size_t)std::max(len, 1LL)));
   TFS_TRY(dev_alloc(A, (void **)&A->ell_rsum, sizeof(float) * (size_t)std::max(n, 1)));
@@ -1200,9 +1211,11 @@ inline int ell_grid(const tfs_matrix *A) { return grid_for(A->ell_nslice, kEllWa
 template <bool DOT>
 void launch_ell(tfs_matrix *A, const float *x, float *y, const KState *st) {
   tm_begin(TFS_KC_SPMV32);
-  hipLaunchKernelGGL(k_ell_diff<DOT>, dim3(ell_grid(A)), dim3(kEllWaves * kWave), 0, cur_stream(),
-                     A->n, A->ell_nslice, A->ell_off, A->ell_col, A->ell_val, A->ell_rsum, x, y,
-                     st, A->partials, kEllDiffXcd);
+  const EllColumns C{A->ell_col, A->ell_window, A->ell_coff, A->ell_code};
+  auto kern = A->ell_col ? k_ell_diff<DOT, false> : k_ell_diff<DOT, true>;
+  hipLaunchKernelGGL(kern, dim3(ell_grid(A)), dim3(kEllWaves * kWave), 0, cur_stream(), A->n,
+                     A->ell_nslice, A->ell_off, C, A->ell_val, A->ell_rsum, x, y, st, A->partials,
+                     kEllDiffXcd);
   tm_end(TFS_KC_SPMV32);
 }
 

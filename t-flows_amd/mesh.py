@@ -91,6 +91,8 @@ def _lib():
         lib.tfs_layout_faces.restype = ctypes.c_int
         lib.tfs_layout_faces.argtypes = [ctypes.c_int, ctypes.c_longlong, _I32P, ctypes.c_int,
                                          _I32P, _I32P, ctypes.c_void_p]
+        lib.tfs_layout_short_columns.restype = ctypes.c_int
+        lib.tfs_layout_short_columns.argtypes = [ctypes.c_int] + [ctypes.c_void_p] * 3
         lib.tfs_mesh_read_cns.restype = ctypes.c_int
         lib.tfs_mesh_read_cns.argtypes = [ctypes.c_char_p] + [ctypes.POINTER(ctypes.c_int)] * 3 + \
             [ctypes.c_void_p, ctypes.c_void_p]
@@ -274,6 +276,18 @@ def layout_faces(n_cells, faces_c, base=1):
     if rc < 0:
         raise ValueError("tfs_layout_faces failed")
     return bool(rc), order, first, entry[:first[-1]]
+
+
+def layout_short_columns(off, col):
+    """A sliced ELL's columns as their 16-bit codes give them back, or None
+    where a slice's columns fall in too many windows."""
+    off, col = np.ascontiguousarray(off, np.int64), np.ascontiguousarray(col, np.int32)
+    out = np.full_like(col, -1)
+    rc = _lib().tfs_layout_short_columns(len(off) - 1, off.ctypes.data, col.ctypes.data,
+                                         out.ctypes.data)
+    if rc < 0:
+        raise ValueError("tfs_layout_short_columns failed")
+    return out if rc else None
 
 
 def layout_summary(row, col, dia):
