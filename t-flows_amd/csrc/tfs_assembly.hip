@@ -169,18 +169,24 @@ extern "C" int tfs_assembly_create(tfs_matrix *A, long long n_faces, const int *
   int nrows = 0;
   if (F.reordered) {
     src.assign((size_t)nnz, -1);
-    std::vector<int *> mine;   // where this row's places are
+    std::vector<int *> mine;   // where this row's places are, by place
+    auto add = [&](int *q) {
+      mine.push_back(q);
+      for (size_t j = mine.size() - 1; j > 0 && *mine[j - 1] > *mine[j]; --j)
+        std::swap(mine[j - 1], mine[j]);
+    };
     for (int k = 0; k < n; ++k) {
       const long long i0 = F.off[(size_t)(k / 64)] + k % 64, i1 = F.off[(size_t)(k / 64) + 1];
       mine.clear();
       for (long long i = i0; i < i1; i += 64)
-        if (hpos[(size_t)i] >= 0) mine.push_back(&hpos[(size_t)i]);
-      for (int t = F.tptr.empty() ? 0 : F.tptr[(size_t)k];
-           t < (F.tptr.empty() ? 0 : F.tptr[(size_t)k + 1]); ++t)
-        if (hpos[F.inc.size() + (size_t)t] >= 0) mine.push_back(&hpos[F.inc.size() + (size_t)t]);
+        if (hpos[(size_t)i] >= 0) add(&hpos[(size_t)i]);
+      if (!F.tptr.empty()) {
+        for (int t = F.tptr[(size_t)k]; t < F.tptr[(size_t)k + 1]; ++t)
+          if (hpos[F.inc.size() + (size_t)t] >= 0) mine.push_back(&hpos[F.inc.size() + (size_t)t]);
+        std::stable_sort(mine.begin(), mine.end(), [](int *a, int *b) { return *a < *b; });
+      }
       to_dia[(size_t)k] = hdia[(size_t)F.orig[(size_t)k]];
-      mine.push_back(&to_dia[(size_t)k]);
-      std::stable_sort(mine.begin(), mine.end(), [](int *a, int *b) { return *a < *b; });
+      add(&to_dia[(size_t)k]);
       for (int *q : mine) {
         src[(size_t)*q] = nrows;
         *q = nrows++;
