@@ -216,6 +216,13 @@ def sweep_bytes(n, ntri):
     return 12 * ntri + 32 * n
 
 
+def fp64_sweep_name(A):
+    """The kernel of the FP64 sweeps of this file's boxes: over blocks where the
+    dependency graph is deep (24 levels and more), else level by level."""
+    return (("k_block_sweep" if A.info()["levels_lower"] >= 24 else "k_sweep_syncfree") +
+            " (FP64 forward/backward incomplete-Cholesky sweeps)")
+
+
 def sweep_roofline(A, c, inloop_us, traffic_profile=None):
     """The preconditioner sweeps: the average launch of the forward and
     backward sweeps timed with HIP events inside the timed solves, against
@@ -229,7 +236,7 @@ def sweep_roofline(A, c, inloop_us, traffic_profile=None):
     b2b_us = 1e3 * A.sweep_time(reps=20)
     achieved = algo / (inloop_us * 1e-6) / 1e9
     return {
-        "kernel": "k_sweep_syncfree (FP64 forward/backward incomplete-Cholesky sweeps)",
+        "kernel": fp64_sweep_name(A),
         "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "frac": achieved / HBM_PEAK_GBS,
         "traffic": measured_traffic(traffic_profile) if traffic_profile else None,
@@ -449,13 +456,9 @@ def mixed_vs_fp64(args):
         per = "8 nnz + 12 N + 4 per SpMV (FP32 values and vectors), one SpMV per FP32 iteration"
     elif A.info()["inner_order"] == solvers.TFS_INNER_BRICKS:
         units, per_unit = 2 * inner, fp32_sweep_bytes(c.n, c.nnz)
-        g = A.info()["inner_sweep_groups"]
-        sched = (f"one persistent launch of {g} workgroups per sweep" if g > 0
-                 else "one launch per level")
-        kname = (("k_sweep_syncfree" if g > 0 else "k_level") +
-                 f" (FP32 DIC sweeps of the brick-ordered copy: {A.info()['inner_brick_edge']}^3 "
-                 "bricks in two colours, "
-                 f"{A.info()['inner_levels']} levels, {sched})")
+        kname = (f"k_brick_sweep (FP32 DIC sweeps of the brick-ordered copy: "
+                 f"{A.info()['inner_brick_edge']}^3 bricks in two colours, "
+                 f"{A.info()['inner_levels']} levels, one launch per colour and direction)")
         prof = "k_brick_sweep_poisson256_counters"
         per = ("(8 (nnz - N) + 32 N) / 2 per sweep (FP32 DIC forward + backward pair), two "
                "sweeps per FP32 iteration")
@@ -871,7 +874,7 @@ def ingest(args):
                    "n_faces": nf, "nnz": nnz},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": None,
-                     "scope": "whole call (6 kernels, 2 scratch allocations, 2 readbacks)"},
+                     "scope": "whole call (6 kernels, a scratch allocation, a readback)"},
         "bitwise_equal_host": same,
         "assembly": {"ms": a_ms, "algorithmic_GBs": a_alg / a_ms / 1e6,
                      "values_upload_ms_at_50GBs": upload_ms},
