@@ -128,10 +128,10 @@ int tfs_layout_short_columns(int nslice, const long long *off, const int *col, i
 /* The cells' face lists of the device face loops (pairs c1, c2 numbered from
  * base, c2 below base a boundary face): order[k] = cell at position k, and per
  * cell first[c] .. first[c + 1] its entries 2 face + side in the order they are
- * summed.  Returns 1 if the cells are reordered, 0 if not, -1 on an invalid
+ * summed; meshes of `from` cells and more may be reordered.  Returns 1 if the cells are reordered, 0 if not, -1 on an invalid
  * argument. */
-int tfs_layout_faces(int n, long long n_faces, const int *faces_c, int base, int *order,
-                     int *first, unsigned *entry);
+int tfs_layout_faces(int n, long long n_faces, const int *faces_c, int base, int from,
+                     int *order, int *first, unsigned *entry);
 
 /* The layouts the solver builds for a matrix (0-based CRS): s_orig = caller
  * row at each S (reverse Cuthill-McKee) position; level of each caller row in

@@ -153,7 +153,7 @@ extern "C" int tfs_assembly_create(tfs_matrix *A, long long n_faces, const int *
     }
   }
   FaceLists F;
-  build_face_lists(n, nf, faces_c, base, F);
+  build_face_lists(n, nf, faces_c, base, kReorderAssembly, F);
   std::vector<int> hpos(F.inc.size() + F.tail.size(), kBoundary);
   auto place = [&](unsigned e) {
     const long long s = e >> 1;

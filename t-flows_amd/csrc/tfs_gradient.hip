@@ -564,7 +564,7 @@ extern "C" int tfs_gradient_create(int n_cells, int n_bnd_cells, long long n_fac
     }
   }
   FaceLists F;
-  build_face_lists(n, nf, faces_c, 1, F);
+  build_face_lists(n, nf, faces_c, 1, kReorderGradient, F);
   std::vector<int2> pairs((size_t)nf);
   for (long long s = 0; s < nf; ++s) {
     const int c2 = faces_c[2 * s + 1];

@@ -975,7 +975,7 @@ long long lines_touched(int n, const int *faces, int base, const std::vector<int
 
 }  // namespace
 
-void build_face_lists(int n, long long nf, const int *faces, int base, FaceLists &out) {
+void build_face_lists(int n, long long nf, const int *faces, int base, int from, FaceLists &out) {
   out = FaceLists();
   out.n = n;
   // per cell, its faces in ascending order (a counting sort over the faces)
@@ -995,19 +995,22 @@ void build_face_lists(int n, long long nf, const int *faces, int base, FaceLists
     }
   }
   // the order of first naming (cells of no face last)
-  std::vector<int> orig, of((size_t)n, -1);
-  orig.reserve((size_t)n);
+  std::vector<int> orig, of;
+  if (n >= from) {
+    of.assign((size_t)n, -1);
+    orig.reserve((size_t)n);
+  }
   auto name = [&](int c) {
     if (c < 0 || of[(size_t)c] >= 0) return;
     of[(size_t)c] = (int)orig.size();
     orig.push_back(c);
   };
-  for (long long s = 0; s < nf; ++s) {
+  for (long long s = 0; s < nf && n >= from; ++s) {
     name(faces[2 * s] - base);
     name(faces[2 * s + 1] - base);
   }
-  for (int c = 0; c < n; ++c) name(c);
-  if (lines_touched(n, faces, base, ptr, inc, nullptr, nullptr) >
+  for (int c = 0; c < n && n >= from; ++c) name(c);
+  if (n >= from && lines_touched(n, faces, base, ptr, inc, nullptr, nullptr) >
       2 * lines_touched(n, faces, base, ptr, inc, &orig, &of)) {
     out.reordered = true;
     out.orig = std::move(orig);

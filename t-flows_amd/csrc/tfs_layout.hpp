@@ -251,6 +251,14 @@ struct FaceLists {
 };
 // faces: pairs (c1, c2) in 1..n (base 1) or 0..n-1 (base 0), c1 an interior cell,
 // c2 below that range for a boundary face; at most 2^31 entries in all.
-void build_face_lists(int n, long long nf, const int *faces, int base, FaceLists &out);
+// Cells are reordered in meshes of `from` cells and more: in smaller ones the
+// fields stay in the caches whatever the order, and the passes in and out cost
+// more than they save.  us with the cells reordered / in the caller's order, at
+// 64^3, 72^3, 80^3 and 100^3 numbered at random: gradients 118/107, 135/122,
+// 152/150, 235/276; pressure step 265/285, 328/377, 392/472, 618/841; momentum
+// assembly and residual 110/115, 140/150, 167/187, 303/341 (48^3: 105/94, 220/219,
+// 89/85).
+constexpr int kReorderGradient = 1 << 19, kReorderAssembly = 1 << 18;
+void build_face_lists(int n, long long nf, const int *faces, int base, int from, FaceLists &out);
 
 }  // namespace tfs

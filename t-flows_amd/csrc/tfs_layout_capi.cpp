@@ -100,11 +100,11 @@ extern "C" int tfs_layout_blocks(int n, const int *row, const int *col, const in
   return B.nblk;
 }
 
-extern "C" int tfs_layout_faces(int n, long long nf, const int *faces, int base, int *order,
-                                int *first, unsigned *entry) {
+extern "C" int tfs_layout_faces(int n, long long nf, const int *faces, int base, int from,
+                                int *order, int *first, unsigned *entry) {
   if (n < 1 || nf < 0 || (nf > 0 && !faces) || !order || !first || !entry) return -1;
   tfs::FaceLists F;
-  tfs::build_face_lists(n, nf, faces, base, F);
+  tfs::build_face_lists(n, nf, faces, base, from, F);
   int at = 0;
   for (int c = 0; c < n; ++c) {
     const int k = F.at(c), s = k / 64;

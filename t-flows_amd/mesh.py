@@ -90,7 +90,7 @@ def _lib():
         lib.tfs_layout_blocks.argtypes = [ctypes.c_int, _I32P, _I32P, _I32P, _I32P, _I32P, _I32P]
         lib.tfs_layout_faces.restype = ctypes.c_int
         lib.tfs_layout_faces.argtypes = [ctypes.c_int, ctypes.c_longlong, _I32P, ctypes.c_int,
-                                         _I32P, _I32P, ctypes.c_void_p]
+                                         ctypes.c_int, _I32P, _I32P, ctypes.c_void_p]
         lib.tfs_layout_short_columns.restype = ctypes.c_int
         lib.tfs_layout_short_columns.argtypes = [ctypes.c_int] + [ctypes.c_void_p] * 3
         lib.tfs_mesh_read_cns.restype = ctypes.c_int
@@ -265,14 +265,14 @@ def layout_blocks(row, col, dia):
     return (k, order, block_of, step_of) if k else None
 
 
-def layout_faces(n_cells, faces_c, base=1):
+def layout_faces(n_cells, faces_c, base=1, reorder_from=1 << 18):
     """The cells' face lists of the device face loops: (reordered, order,
     first, entry), entry[first[c]:first[c+1]] = 2 face + side of cell c."""
     faces_c = np.ascontiguousarray(faces_c, np.int32)
     order, first = np.empty(n_cells, np.int32), np.empty(n_cells + 1, np.int32)
     entry = np.empty(max(faces_c.size, 1), np.uint32)
-    rc = _lib().tfs_layout_faces(n_cells, faces_c.size // 2, faces_c, base, order, first,
-                                 entry.ctypes.data)
+    rc = _lib().tfs_layout_faces(n_cells, faces_c.size // 2, faces_c, base, reorder_from, order,
+                                 first, entry.ctypes.data)
     if rc < 0:
         raise ValueError("tfs_layout_faces failed")
     return bool(rc), order, first, entry[:first[-1]]

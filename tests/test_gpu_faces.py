@@ -28,7 +28,9 @@ MESHES = {
     "slice": lambda: box(4, 4, 4, False),
     "slice+1": lambda: box(13, 5, 1, True),
     "ordered": lambda: box(37, 11, 29, False),
-    "reordered": lambda: box(31, 30, 17, True),
+    "permuted": lambda: box(31, 30, 17, True),
+    "assembly reordered": lambda: box(61, 67, 65, True),
+    "reordered": lambda: box(81, 83, 79, True),
     "slots": lambda: star(32),
     "tails": lambda: star(150),
 }

@@ -16,8 +16,8 @@ def expected(n, faces, base):
     return np.concatenate(([0], np.cumsum(np.bincount(cell, minlength=n)))), entry[k]
 
 
-def check(n, faces, base):
-    reordered, order, first, entry = mesh.layout_faces(n, faces, base)
+def check(n, faces, base, reorder_from=2):
+    reordered, order, first, entry = mesh.layout_faces(n, faces, base, reorder_from)
     want_first, want_entry = expected(n, faces, base)
     assert np.array_equal(first, want_first) and np.array_equal(entry, want_entry)
     assert np.array_equal(np.sort(order), np.arange(n))
@@ -31,6 +31,7 @@ def test_box(dims, permute):
     c = mesh.make_case(nx=dims[0], ny=dims[1], nz=dims[2], permute=permute, with_faces=True)
     reordered = check(c.n, c.faces, 1)
     assert reordered == (permute and c.n > 10000)
+    assert not check(c.n, c.faces, 1, c.n + 1)
 
 
 @pytest.mark.parametrize("base", [0, 1])
