@@ -1384,10 +1384,19 @@ k_sweep_syncfree(int n, Tri<T> Tr, T *d, T *b, T *x, T *arm, const KState *st, i
 // would delay the stores everyone waits for.
 //
 // Order and progress: blocks are numbered so that a block depends on earlier
-// ones only; workgroup w takes blocks w, w + G, ... with all G resident, so
-// the lowest unfinished block always runs and every wait ends; the polls are
-// bounded as in k_sweep_syncfree all the same (a halo slot given up is filled
-// with zero, so wavefront 0 always finishes).
+// ones only.  Rank r of a launch of G workgroups owns blocks r, r + G, r + 2 G,
+// ...; a workgroup claims its own rank as it starts (BlockShare), begins its first
+// block once all lower ranks are claimed and the later ones once all are.  Where
+// that stays out -- the GPU is shared and some workgroup cannot start -- the
+// waiting or finished ones claim the lowest rank that is left, and own it.  So
+// every owner of an unfinished block runs and takes its blocks in ascending order,
+// a block is only begun when all before it are owned, the lowest unfinished one is
+// always under way, and every wait ends however few workgroups are resident:
+// the solves of any number of matrices may share the GPU.  Claims cost 0.3 to 1 us
+// a sweep (drawing the blocks from one counter 12 ns each, all in a row: 64
+// systems of 25^3 46 -> 62 us).  The polls are bounded as in k_sweep_syncfree all
+// the same (a halo slot given up is filled with zero, so wavefront 0 always
+// finishes).
 //
 // Every row sum is formed in the caller's entry order; padding entries are
 // 0 * 0 terms, which leave any sum as it is.
@@ -1402,12 +1411,81 @@ k_sweep_syncfree(int n, Tri<T> Tr, T *d, T *b, T *x, T *arm, const KState *st, i
 // Tried and not kept: one wavefront that also polls (its loads wait for its
 // stores: 104 us at 97x75x61, 172 at 128^3), two polling wavefronts (84, 145),
 // polling the whole halo from the start (82, 139), twice the workgroups (82,
-// 141; 264 at 200^3, but two matrices' sweeps must fit side by side).
+// 141; 264 at 200^3, but solves beside this one need room).
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+
+// The ranks a workgroup owns, kept by its wavefront 1 (every lane the same).
+// claim: a bit per rank, 32 a line (so that claims do not queue up behind one
+// another); chain: the rank after each rank of one owner.
+constexpr int kClaimLine = 32;                 // words from one line of claims to the next
+constexpr int kClaimLines = 64;                // one lane each: up to 2048 ranks
+constexpr int kClaimPolls = 16;                // looks before a rank of others is claimed
+struct BlockShare {
+  unsigned *claim;
+  int *chain;
+  int G, own, lane;
+  bool held;                   // `own` is claimed and not begun
+  int head = -1, tail = -1;    // ranks begun, ascending
+  int rank = -1, round = 0;    // the present block is rank + round
+
+  __device__ __forceinline__ bool won(int r) const {
+    unsigned was = 0;
+    if (lane == 0)
+      was = __hip_atomic_fetch_or(claim + r / 32 * kClaimLine, 1u << r % 32, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+    return !(__builtin_amdgcn_readfirstlane(was) >> r % 32 & 1u);
+  }
+  __device__ __forceinline__ int begin(int r) {
+    if (tail < 0) head = r;
+    else if (lane == 0) coherent_store(&chain[tail], r);
+    tail = rank = r;
+    return r;
+  }
+  // the next block; nblk or more: there is none
+  __device__ __forceinline__ int next(int nblk) {
+    if (round > 0) {
+      if (rank == tail) round += G;
+      rank = rank == tail ? head : __builtin_amdgcn_readfirstlane(coherent_load(&chain[rank]));
+      return rank + round;
+    }
+    for (int polls = 0;;) {
+      const int below = (held ? own : G) - 32 * lane;   // ranks of this lane's word
+      unsigned left = 0;
+      if (below > 0) {
+        left = ~coherent_load(claim + lane * kClaimLine);
+        if (below < 32) left &= (1u << below) - 1u;
+      }
+      const unsigned long long any = __ballot(left != 0);
+      if (!any && held) {
+        held = false;
+        return begin(own);
+      }
+      if (!any) {
+        round = G;
+        rank = head;
+        return head < 0 ? nblk : rank + round;
+      }
+      if (polls++ < kClaimPolls) {
+        __builtin_amdgcn_s_sleep(4);
+        continue;
+      }
+      const int l = __builtin_ctzll(any);
+      const int r = 32 * l + __builtin_ctz(__builtin_amdgcn_readlane(left, l));
+      if (won(r)) return begin(r);
+    }
+  }
+};
+
+// The claims of this launch (clear), those of the next one, which it clears (the
+// forward and the backward sweep alternate; the factor's are cleared before it).
+struct BlockClaims {
+  unsigned *mine, *next;
+  int *chain;
+};
 
 struct BlockTri {
   const Block *__restrict__ blk;
@@ -1442,17 +1520,28 @@ template <int OP, int W>
 __global__ void __launch_bounds__(kBlockThreads)
 k_block_sweep(int n, int nblk, BlockTri Tr, const int *__restrict__ src,
               const double *__restrict__ d, double *b, double *out, double *arm, const KState *st,
-              int *err) {
+              int *err, BlockClaims C) {
   constexpr int PL = W <= 3 ? 4 : 8;  // places per row
   extern __shared__ double lds[];
+  __shared__ int then;   // the block after the present one, -1 until it is known
   double *const vv = lds;
   double *const ss = vv + W * kBlockRows, *const dd = ss + kBlockRows;
   unsigned short *const ii = reinterpret_cast<unsigned short *>(dd + kBlockRows);
   int *const tt = reinterpret_cast<int *>(ii + PL * kBlockRows);
   double *const xs = reinterpret_cast<double *>(tt + kWave);
   const int tid = (int)threadIdx.x, lane = tid % kWave;
-  const int done = st ? st->done : 0;  // looked at once the first loads are under way
-  for (int bk = (int)blockIdx.x; bk < nblk; bk += (int)gridDim.x) {
+  const int done = st ? st->done : 0;
+  if (C.next && blockIdx.x == 0 && tid < kClaimLines) coherent_store(C.next + tid * kClaimLine, 0u);
+  BlockShare share{C.mine, C.chain, (int)gridDim.x, (int)blockIdx.x, lane, false};
+  if (tid >= kWave) {
+    share.held = share.won(share.own);
+    const int first = __builtin_amdgcn_readfirstlane(done) ? nblk : share.next(nblk);
+    if (lane == 0) then = first;
+  }
+  __syncthreads();
+  int bk = __builtin_amdgcn_readfirstlane(then);
+  if (__builtin_amdgcn_readfirstlane(done)) return;
+  while (bk < nblk) {
     const Block B = Tr.blk[bk];
     // ---- stage the block.  Indices past an array's end are clamped to its
     // last element, so that every load is unconditional and all are in flight
@@ -1489,9 +1578,11 @@ k_block_sweep(int n, int nblk, BlockTri Tr, const int *__restrict__ src,
       const int t0 = Tr.step[B.step0 + min(tid, B.steps)];
 #pragma unroll
       for (int c = 0; c < kR; ++c) rhs[c] = b[at[c]];
-      if (__builtin_amdgcn_readfirstlane(done)) return;
       __syncthreads();  // the previous block is done with LDS
-      if (tid == 0) xs[0] = 0.0;
+      if (tid == 0) {
+        xs[0] = 0.0;
+        then = -1;
+      }
       if (tid < kWave) tt[tid] = t0;
 #pragma unroll
       for (int c = 0; c < kH; ++c)
@@ -1559,21 +1650,29 @@ k_block_sweep(int n, int nblk, BlockTri Tr, const int *__restrict__ src,
             lack &= ~1u;
           }
         }
+        // all of them loaded before any is looked at (a lane that lacks none of
+        // its own repeats one of another's: the same line)
         double v[kHaloLane];
+        unsigned long long any[kHaloLane];
 #pragma unroll
-        for (int c = 0; c < kHaloLane; ++c)
-          if (c * kWave < B.halo) {
-            v[c] = Sentinel<double>::value();
-            if (lack >> c & 1u) v[c] = coherent_load(&out[hq[c]]);
+        for (int c = 0; c < kHaloLane; ++c) {
+          any[c] = __ballot(lack >> c & 1u);
+          if (any[c]) {
+            const int first = __builtin_amdgcn_readlane(hq[c], __builtin_ctzll(any[c]));
+            v[c] = coherent_load(&out[(lack >> c & 1u) ? hq[c] : first]);
           }
+        }
 #pragma unroll
         for (int c = 0; c < kHaloLane; ++c)
-          if (c * kWave < B.halo && !waiting(v[c])) {
+          if (any[c] && (lack >> c & 1u) && !waiting(v[c])) {
             __hip_atomic_store(slot + c * kWave, v[c], __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_WORKGROUP);
             lack &= ~(1u << c);
           }
       }
+      const int b1 = share.next(nblk);
+      if (lane == 0)
+        __hip_atomic_store(&then, b1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     } else {
       // ---- wavefront 0: the steps.  Row data of the next step is read from
       // LDS while this one computes (two register sets in turn).
@@ -1633,6 +1732,10 @@ k_block_sweep(int n, int nblk, BlockTri Tr, const int *__restrict__ src,
         if (t + 1 < B.steps) advance(r1, r0, t + 1);
       }
     }
+    // (wavefront 1 always gets there: its polls are bounded)
+    do bk = __hip_atomic_load(&then, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    while (bk < 0);
+    bk = __builtin_amdgcn_readfirstlane(bk);
   }
 }
 

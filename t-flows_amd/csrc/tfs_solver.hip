@@ -182,6 +182,8 @@ struct tfs_matrix {
   double *b_diag = nullptr, *b_d = nullptr;  // and the factor
   bool blk_allocated = false;
   int blk_grid = 0;
+  unsigned *blk_claim = nullptr;   // k_block_sweep's ranks
+  int *blk_chain = nullptr;
   bool blk_off = false;       // another sweep schedule set by the caller or the environment
   double *val = nullptr;       // caller-order FP64 values
   Values<double> v64;
@@ -556,11 +558,18 @@ void launch_blocks(tfs_matrix *A, const DevBlocks &D, const double *d, const dou
   const int kc = OP == OP_FACTOR ? TFS_KC_FACTOR : TFS_KC_SWEEP;
   const BlockTri Tr{D.blk, D.step, D.idx, D.val, D.halo};
   const size_t lds = block_lds(A->blk_width, D.halo_max);
+  constexpr int kClaims = kClaimLine * kClaimLines;   // of forward, backward, factor
+  unsigned *const c = A->blk_claim;
+  const BlockClaims claims{c + (OP == OP_FWD ? 0 : OP == OP_BWD ? 1 : 2) * kClaims,
+                           OP == OP_FWD ? c + kClaims : OP == OP_BWD ? c : nullptr, A->blk_chain};
   tm_begin(kc);
+  if (OP == OP_FACTOR)
+    hipLaunchKernelGGL(k_fill<unsigned>, dim3(1), dim3(kRedThreads), 0, cur_stream(), kClaims,
+                       claims.mine, 0u);
   auto kern = A->blk_width == 3 ? k_block_sweep<OP, 3> : k_block_sweep<OP, kBlockWide>;
   hipLaunchKernelGGL(kern, dim3(A->blk_grid), dim3(kBlockThreads), lds, cur_stream(), A->n, A->blk_n,
                      Tr, A->b_to_s, d, const_cast<double *>(b), out, armv,
-                     st, A->sweep_err);
+                     st, A->sweep_err, claims);
   tm_end(kc);
 }
 
@@ -1904,8 +1913,8 @@ int build_ell64(tfs_matrix *A, const Layout &Ly) {
 }
 
 // The block sweeps' structure, if it suits them, and their grid: at most half
-// the workgroups that fit at once, so that two matrices' block sweeps fit
-// beside each other (the static schedule needs all of them resident).
+// the workgroups that fit at once.  Twice as many measured no faster, and none of
+// them has to be resident (k_block_sweep).
 int build_block_sweeps(tfs_matrix *A, const Layout &Ly, const int *row, const int *col,
                        const int *dia) {
   const int n = A->n;
@@ -1953,7 +1962,11 @@ int build_block_sweeps(tfs_matrix *A, const Layout &Ly, const int *row, const in
     per_cu = per_cu == 0 ? b : std::min(per_cu, b);
   }
   if (per_cu < 1) return 0;
-  A->blk_grid = std::max(1, std::min(BL.nblk, n_cu * per_cu / 2));
+  A->blk_grid = std::max(1, std::min({BL.nblk, n_cu * per_cu / 2, 32 * kClaimLines}));
+  const size_t claims = 3 * sizeof(unsigned) * kClaimLine * kClaimLines;
+  TFS_TRY(dev_alloc(A, (void **)&A->blk_claim, claims));
+  TFS_HIP(hipMemset(A->blk_claim, 0, claims));
+  TFS_TRY(dev_alloc(A, (void **)&A->blk_chain, sizeof(int) * (size_t)A->blk_grid));
   A->blk_ok = true;
   return 0;
 }
