@@ -626,6 +626,17 @@ void build_blocks(int n, const int *row, const int *col, const int *dia,
   for (int p = 0; p < n; ++p) out.of_orig[(size_t)out.orig[(size_t)p]] = p;
   std::vector<int> lstep((size_t)n);
   for (int p = 0; p < n; ++p) lstep[(size_t)p] = rlev[(size_t)out.orig[(size_t)p]];
+  long long steps = 0;
+  for (int k = 0; k < nb; ++k)
+    for (int p = bstart[(size_t)k], first = p; p < bstart[(size_t)k + 1]; ++p)
+      if (p == bstart[(size_t)k] || lstep[(size_t)p] != lstep[(size_t)p - 1] ||
+          p - first == kBlockLanes) {
+        first = p;
+        ++steps;
+      }
+  if ((out.width > 3 ? 2.0 : 1.0) * (kBlockNs * nb + kBlockStepNs * (double)steps) >
+      kLevelNs * nlev + kRowNs * n)
+    return;
   if (!build_block_triangle(row, col, dia, true, out.orig, out.of_orig, bstart, lstep, out.width,
                             out.places(), out.L))
     return;
