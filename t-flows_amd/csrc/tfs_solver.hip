@@ -782,15 +782,17 @@ bool cg_precondition(tfs_matrix *A, const T *r, T *yL, T *zU, T *z, const KState
   return false;
 }
 
-// One CG iteration (Cg.f90:97-178) in precision T; Bicg takes the same path
-// (its shadow sequence equals the primary one bit for bit, Bicg.f90:91-175).
 // p = z + beta p, q = A p and (p, q).  Up to kGatherP rows p is formed in the
 // product (a second gather from the caches costs less than a launch); V.p and
-// V.r2 then change places.  Above, in a pass of its own (figures at kFuseGrid).
-constexpr int kGatherP = 1 << 16;
+// V.r2 then change places.  Above, in a pass of its own (figures at kFuseGrid), as
+// where rows are wide, whose every entry gathers twice: us per iteration of
+// diagonal Cg, gathered / own pass, 64 000 rows of 7 entries 23.5 / 25.8, of 11 23.5 /
+// 25.6, of 18 26.2 / 26.9, of 26 28.7 / 27.1, of 114 59.9 / 43.9; 4096 of 244 91.6 / 57.5.
+constexpr int kGatherP = 1 << 16, kGatherRow = 20;
 template <typename T>
 inline bool gathers_p(const tfs_matrix *A) {
-  return sizeof(T) == 8 && A->e64_len > 0 && A->n <= kGatherP;
+  return sizeof(T) == 8 && A->e64_len > 0 && A->n <= kGatherP &&
+         A->nnz <= (long long)kGatherRow * A->n;
 }
 
 template <typename T>
