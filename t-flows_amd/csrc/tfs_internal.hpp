@@ -15,7 +15,9 @@ int sweep_capacity(const tfs_matrix *A);
 void set_sweep_grid(tfs_matrix *A, int groups);
 // tfs_matrix_create for a matrix whose solves run beside other matrices'
 // (the server): without the block sweeps, so that the sweep grids' shares of
-// one kernel's occupancy hold.
+// one kernel's occupancy hold, and with the sweeps' triangles allocated from the
+// start, so that a later request with another preconditioner takes no memory
+// that was not accounted for when the case came in.
 int matrix_create_shared(int n, long long nnz, const int *row, const int *col, const int *dia,
                          int base, tfs_matrix **out);
 }  // namespace tfs

@@ -2164,7 +2164,15 @@ extern "C" int tfs_matrix_create(int n, long long nnz, const int *row, const int
 
 int tfs::matrix_create_shared(int n, long long nnz, const int *row, const int *col, const int *dia,
                               int base, tfs_matrix **out) {
-  return matrix_create(n, nnz, row, col, dia, base, out, nullptr, false, false);
+  TFS_TRY(matrix_create(n, nnz, row, col, dia, base, out, nullptr, false, false));
+  if (n == 0) return TFS_OK;
+  StreamScope scope((*out)->stream);
+  const int rc = alloc_triangles<double>(*out);
+  if (rc < 0) {
+    tfs_matrix_destroy(*out);
+    *out = nullptr;
+  }
+  return rc;
 }
 
 extern "C" int tfs_matrix_destroy(tfs_matrix *A) {
