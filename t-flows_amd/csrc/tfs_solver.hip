@@ -272,7 +272,8 @@ struct tfs_matrix {
 namespace {
 
 int matrix_create(int n, long long nnz, const int *row, const int *col, const int *dia, int base,
-                  tfs_matrix **out, Layout *keep, bool identity_s = false, bool blocks = true);
+                  tfs_matrix **out, Layout *keep, bool identity_s = false, bool blocks = true,
+                  bool direct = true);
 
 int dev_alloc(tfs_matrix *A, void **p, size_t bytes) {
   if (bytes == 0) bytes = 8;
@@ -1346,7 +1347,7 @@ int build_inner(tfs_matrix *A) {
   }
   Layout Ly;
   tfs_matrix *C = nullptr;
-  TFS_TRY(matrix_create(n, nnz, prow.data(), pcol.data(), pdia.data(), 0, &C, &Ly, true, false));
+  TFS_TRY(matrix_create(n, nnz, prow.data(), pcol.data(), pdia.data(), 0, &C, &Ly, true, false, false));
   std::vector<int> from_s(n);
   for (int i = 0; i < n; ++i) from_s[i] = perm[Ly.s_orig[i]];
   int rc = upload(A, &A->inner_emap, emap);
@@ -1983,7 +1984,7 @@ int occupancy(int *per_cu) {
 }
 
 int create_device(tfs_matrix *A, const Layout &Ly, const int *row, const int *col,
-                  const int *dia, bool blocks, bool keep_order) {
+                  const int *dia, bool blocks, bool direct) {
   const int n = A->n;
   TFS_HIP(hipStreamCreateWithFlags(&A->stream, hipStreamNonBlocking));
   TFS_HIP(hipEventCreate(&A->ev0));
@@ -2015,7 +2016,8 @@ int create_device(tfs_matrix *A, const Layout &Ly, const int *row, const int *co
     TFS_TRY(upload(A, &A->s_lpos, lpos));
   }
   if (blocks) TFS_TRY(build_block_sweeps(A, Ly, row, col, dia));
-  if (blocks && !keep_order && n > 0 &&
+  // (`direct`: matrices whose caller can ask for a product of its own vectors)
+  if (direct && n > 0 &&
       gather_lines(n, row, col) <= kDirectLines * gather_lines(n, Ly.s_row.data(), Ly.s_col.data())) {
     const std::vector<int> crow(row, row + n + 1), ccol(col, col + A->nnz);
     const std::vector<int> crb = row_blocks(crow, kSpmvRows);
@@ -2117,7 +2119,7 @@ namespace {
 // touching the device, so a bad structure is rejected without a GPU; then
 // builds the layouts and uploads them.  `keep` receives the host layout.
 int matrix_create(int n, long long nnz, const int *row, const int *col, const int *dia, int base,
-                  tfs_matrix **out, Layout *keep, bool identity_s, bool blocks) {
+                  tfs_matrix **out, Layout *keep, bool identity_s, bool blocks, bool direct) {
   if (!out) return TFS_ERR_INVALID;
   *out = nullptr;
   if (n < 0 || nnz < n || nnz > 0x7ffffffeLL || (base != 0 && base != 1)) return TFS_ERR_INVALID;
@@ -2146,7 +2148,7 @@ int matrix_create(int n, long long nnz, const int *row, const int *col, const in
   tfs_matrix *A = new tfs_matrix;
   A->n = n;
   A->nnz = nnz;
-  const int rc = create_device(A, Ly, hr.data(), hc.data(), hd.data(), blocks, identity_s);
+  const int rc = create_device(A, Ly, hr.data(), hc.data(), hd.data(), blocks, direct);
   if (rc < 0) {
     tfs_matrix_destroy(A);
     return rc;
@@ -2164,7 +2166,7 @@ extern "C" int tfs_matrix_create(int n, long long nnz, const int *row, const int
 
 int tfs::matrix_create_shared(int n, long long nnz, const int *row, const int *col, const int *dia,
                               int base, tfs_matrix **out) {
-  TFS_TRY(matrix_create(n, nnz, row, col, dia, base, out, nullptr, false, false));
+  TFS_TRY(matrix_create(n, nnz, row, col, dia, base, out, nullptr, false, false, false));
   if (n == 0) return TFS_OK;
   StreamScope scope((*out)->stream);
   const int rc = alloc_triangles<double>(*out);
@@ -2880,7 +2882,7 @@ namespace {
 // caller destroys B.
 int batch_build(tfs_batch *B, long long N, long long NNZ, const int *cr, const int *cc,
                 const int *cd, Layout &Ly, bool blocks) {
-  int rc = matrix_create((int)N, NNZ, cr, cc, cd, 0, &B->A, &Ly, false, blocks);
+  int rc = matrix_create((int)N, NNZ, cr, cc, cd, 0, &B->A, &Ly, false, blocks, false);
   if (rc < 0) return rc;
   B->A->sweep_fixed = true;  // the batch picks its sweeps when it captures its graph
   const int nsys = B->nsys;
