@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <future>
 #include <unordered_map>
 #include <cstdlib>
 
@@ -11,6 +12,14 @@ namespace {
 
 // The upper layout is the lower one backwards (see build_sweep).
 constexpr bool kMirrorUpper = true;
+
+// How parts of a layout of n rows are built beside one another: on a thread of
+// their own (where one can be had) or, where that would cost as much, in turn.
+// ms of a box's layout and blocks on eight cores, in turn / beside one another:
+// 26^3 5.0 / 5.4, 32^3 9.7 / 6.9, 48^3 37.5 / 25.7.
+inline std::launch beside(int n) {
+  return n < 1 << 15 ? std::launch::deferred : std::launch::async | std::launch::deferred;
+}
 
 // Breadth-first search from `start` over nodes whose mark differs from
 // `stamp` (marking them); neighbours are taken in ascending degree, ties by
@@ -46,36 +55,63 @@ int cm_bfs(int start, int stamp, const std::vector<int> &row, const std::vector<
   return levels;
 }
 
+// Whether every entry has its mirror (columns ascend, as they do in a matrix).
+bool symmetric_structure(int n, const int *row, const int *col) {
+  std::vector<int> next(row, row + n);  // per row, the first lower entry not yet mirrored
+  for (int i = 0; i < n; ++i) {
+    int lower = 0;
+    for (int e = row[i]; e < row[i + 1]; ++e) {
+      const int k = col[e];
+      if (e > row[i] && k <= col[e - 1]) return false;
+      lower += k < i;
+      if (k <= i) continue;
+      // row k's lower columns ascend, so their mirrors come in order
+      if (next[(size_t)k] >= row[k + 1] || col[next[(size_t)k]] != i) return false;
+      ++next[(size_t)k];
+    }
+    if (next[(size_t)i] != row[i] + lower) return false;
+  }
+  return true;
+}
+
 // Reverse Cuthill-McKee (Cuthill & McKee 1969; George 1971), starting each
 // connected component from a pseudo-peripheral node (George & Liu 1979).
 std::vector<int> rcm(int n, const int *row, const int *col) {
   // symmetric adjacency without the diagonal
-  std::vector<int> cnt(n + 1, 0);
-  for (int i = 0; i < n; ++i)
-    for (int e = row[i]; e < row[i + 1]; ++e)
-      if (col[e] != i) {
-        cnt[i + 1]++;
-        cnt[col[e] + 1]++;
-      }
-  for (int i = 0; i < n; ++i) cnt[i + 1] += cnt[i];
-  std::vector<int> adj(cnt[n]), fill(cnt.begin(), cnt.end() - 1);
-  for (int i = 0; i < n; ++i)
-    for (int e = row[i]; e < row[i + 1]; ++e)
-      if (col[e] != i) {
-        adj[fill[i]++] = col[e];
-        adj[fill[col[e]]++] = i;
-      }
-  // drop duplicates (a structurally symmetric pattern lists each pair twice)
   std::vector<int> arow(n + 1, 0), a2;
-  a2.reserve(adj.size() / 2 + 1);
-  for (int i = 0; i < n; ++i) {
-    std::sort(adj.begin() + cnt[i], adj.begin() + cnt[i + 1]);
-    int prev = -1;
-    for (int e = cnt[i]; e < cnt[i + 1]; ++e)
-      if (adj[e] != prev) a2.push_back(prev = adj[e]);
-    arow[i + 1] = (int)a2.size();
+  if (symmetric_structure(n, row, col)) {
+    a2.reserve((size_t)row[n]);
+    for (int i = 0; i < n; ++i) {
+      for (int e = row[i]; e < row[i + 1]; ++e)
+        if (col[e] != i) a2.push_back(col[e]);
+      arow[i + 1] = (int)a2.size();
+    }
+  } else {
+    std::vector<int> cnt(n + 1, 0);
+    for (int i = 0; i < n; ++i)
+      for (int e = row[i]; e < row[i + 1]; ++e)
+        if (col[e] != i) {
+          cnt[i + 1]++;
+          cnt[col[e] + 1]++;
+        }
+    for (int i = 0; i < n; ++i) cnt[i + 1] += cnt[i];
+    std::vector<int> adj(cnt[n]), fill(cnt.begin(), cnt.end() - 1);
+    for (int i = 0; i < n; ++i)
+      for (int e = row[i]; e < row[i + 1]; ++e)
+        if (col[e] != i) {
+          adj[fill[i]++] = col[e];
+          adj[fill[col[e]]++] = i;
+        }
+    // drop duplicates (a pair that has its mirror is listed twice)
+    a2.reserve(adj.size() / 2 + 1);
+    for (int i = 0; i < n; ++i) {
+      std::sort(adj.begin() + cnt[i], adj.begin() + cnt[i + 1]);
+      int prev = -1;
+      for (int e = cnt[i]; e < cnt[i + 1]; ++e)
+        if (adj[e] != prev) a2.push_back(prev = adj[e]);
+      arow[i + 1] = (int)a2.size();
+    }
   }
-  std::vector<int>().swap(adj);
   std::vector<int> deg(n);
   for (int i = 0; i < n; ++i) deg[i] = arow[i + 1] - arow[i];
 
@@ -236,16 +272,22 @@ int brick_blocks(int r0, int r1, const int *row, const int *col, const int *dia,
   gid.reserve((size_t)n / (size_t)std::max(1, edge * edge * edge) + 16);
   std::vector<int> grp(n);
   std::vector<int> gcount;
+  long long last = -1;  // the row before mostly has the same key
   for (int i = 0; i < n; ++i) {
     const int *f = &phi[(size_t)i * kClasses];
     const long long key = (f[0] / edge) + span * ((f[1] / edge) + span * (long long)(f[2] / edge));
-    auto it = gid.find(key);
-    if (it == gid.end()) {
-      it = gid.emplace(key, (int)gcount.size()).first;
-      gcount.push_back(0);
+    if (key == last) {
+      grp[i] = grp[i - 1];
+    } else {
+      auto it = gid.find(key);
+      if (it == gid.end()) {
+        it = gid.emplace(key, (int)gcount.size()).first;
+        gcount.push_back(0);
+      }
+      grp[i] = it->second;
+      last = key;
     }
-    grp[i] = it->second;
-    gcount[(size_t)it->second]++;
+    gcount[(size_t)grp[i]]++;
   }
   std::vector<int>().swap(phi);
   const int ng = (int)gcount.size();
@@ -467,60 +509,87 @@ int brick_colour_order(int n, const int *row, const int *col, const int *dia, in
 
 namespace {
 
-// One triangle of the blocks in block order: `orig` the caller row of each
-// position, blocks [bstart[b], bstart[b + 1]), and per position its step.
-// False if a limit is exceeded.
-bool build_block_triangle(const int *row, const int *col, const int *dia, bool lower,
-                          const std::vector<int> &orig, const std::vector<int> &of_orig,
-                          const std::vector<int> &bstart, const std::vector<int> &lstep,
+// One triangle of the blocks in block order: `of_orig` the position of each caller
+// row, blocks [bstart[b], bstart[b + 1]), per position its block and its level in it;
+// the upper triangle has everything backwards.  False if a limit is exceeded.
+// The entries go to their rows' places in one pass over the caller's rows, whose
+// neighbours' positions then come in runs; the halo is numbered from there.
+bool build_block_triangle(int n, const int *row, const int *col, const int *dia, bool lower,
+                          const std::vector<int> &of_orig, const std::vector<int> &bstart,
+                          const std::vector<int> &block_at, const std::vector<int> &lstep,
                           int width, int places, BlockTriangle &T) {
   const int nb = (int)bstart.size() - 1;
-  std::vector<int> slot_of(orig.size(), -1), in_halo;  // halo number of a position, this block
+  auto start = [&](int b) { return lower ? bstart[(size_t)b] : n - bstart[(size_t)(nb - b)]; };
+  auto mirror = [&](int p) { return lower ? p : n - 1 - p; };   // position <-> lower position
+  auto level = [&](int p) { return lower ? lstep[(size_t)p] : -lstep[(size_t)(n - 1 - p)]; };
   T.blk.resize((size_t)nb);
+  size_t padded = 0;
   for (int b = 0; b < nb; ++b) {
     Block &B = T.blk[(size_t)b];
-    B.row0 = bstart[(size_t)b];
-    B.rows = bstart[(size_t)b + 1] - B.row0;
+    B.row0 = start(b);
+    B.rows = start(b + 1) - B.row0;
     B.rpad = (B.rows + 7) & ~7;
-    B.ent0 = (int)T.src.size();
-    B.idx0 = (int)(T.idx.size() / (size_t)places);
+    if ((size_t)width * (padded + (size_t)B.rpad) > 0x7fffffffu) return false;
+    B.ent0 = (int)((size_t)width * padded);
+    B.idx0 = (int)padded;
+    padded += (size_t)B.rpad;
+  }
+  T.src.assign((size_t)width * padded, -1);
+  T.idx.assign((size_t)places * padded, 0);
+  std::vector<int> dep((size_t)width * (size_t)n, -1);   // positions of each row's entries
+  for (int i = 0; i < n; ++i) {
+    const int at = mirror(of_orig[(size_t)i]);
+    const int b = block_at[(size_t)of_orig[(size_t)i]];
+    const Block &B = T.blk[(size_t)(lower ? b : nb - 1 - b)];
+    const int j0 = lower ? row[i] : dia[i] + 1, j1 = lower ? dia[i] : row[i + 1];
+    int *const from = &T.src[(size_t)B.ent0 + (size_t)(at - B.row0)];
+    for (int j = j0; j < j1; ++j) {
+      dep[(size_t)width * (size_t)at + (size_t)(j - j0)] = mirror(of_orig[(size_t)col[j]]);
+      from[(size_t)(j - j0) * (size_t)B.rpad] = j;
+    }
+  }
+  // halo number of a position in this block: a table that stays in the caches
+  constexpr unsigned kTable = 1024;
+  static_assert(kTable > 2 * kBlockHalo, "entries of the halo table");
+  struct Slot { int block = -1, q = 0, h = 0; };
+  std::vector<Slot> table(kTable);
+  for (int b = 0; b < nb; ++b) {
+    Block &B = T.blk[(size_t)b];
     B.halo0 = (int)T.halo.size();
     B.step0 = (int)T.step.size();
-    if (T.src.size() + (size_t)width * B.rpad > 0x7fffffffu) return false;
-    T.src.resize(T.src.size() + (size_t)width * B.rpad, -1);
-    T.idx.resize(T.idx.size() + (size_t)places * B.rpad, 0);
-    in_halo.clear();
+    B.halo = 0;
     for (int p = 0; p < B.rows; ++p) {
-      const int i = orig[(size_t)(B.row0 + p)];
-      const int j0 = lower ? row[i] : dia[i] + 1, j1 = lower ? dia[i] : row[i + 1];
-      for (int j = j0; j < j1; ++j) {
-        const int q = of_orig[(size_t)col[j]];
+      const int lev = level(B.row0 + p);
+      const int *const d = &dep[(size_t)width * (size_t)(B.row0 + p)];
+      unsigned short *const at = &T.idx[(size_t)(B.idx0 + p) * (size_t)places];
+      for (int k = 0; k < width && d[k] >= 0; ++k) {
+        const int q = d[k];
         int slot;
         if (q >= B.row0 && q < B.row0 + B.rows) {
-          if (lstep[(size_t)q] >= lstep[(size_t)(B.row0 + p)]) return false;
+          if (level(q) >= lev) return false;
           slot = 1 + q - B.row0;
         } else {
           if (q > B.row0) return false;  // only earlier blocks
-          if (slot_of[(size_t)q] < 0) {
-            slot_of[(size_t)q] = (int)in_halo.size();
-            in_halo.push_back(q);
+          unsigned t = (unsigned)q * 2654435761u >> 22;
+          while (table[t].block == b && table[t].q != q) t = (t + 1) % kTable;
+          if (table[t].block != b) {
+            if (B.halo == kBlockHalo) return false;
+            table[t].block = b;
+            table[t].q = q;
+            table[t].h = B.halo++;
+            T.halo.push_back(q);
           }
-          slot = 1 + B.rows + slot_of[(size_t)q];
+          slot = 1 + B.rows + table[t].h;
         }
-        T.idx[((size_t)B.idx0 + p) * places + (j - j0)] = (unsigned short)(slot * sizeof(double));
-        T.src[(size_t)B.ent0 + (size_t)(j - j0) * B.rpad + p] = j;
+        at[k] = (unsigned short)(slot * sizeof(double));
       }
       // a step: one lane per row, so at most a wavefront of one level's rows
-      if (p == 0 || lstep[(size_t)(B.row0 + p)] != lstep[(size_t)(B.row0 + p - 1)] ||
-          p - T.step.back() == kBlockLanes)
+      if (p == 0 || lev != level(B.row0 + p - 1) || p - T.step.back() == kBlockLanes)
         T.step.push_back((unsigned short)p);
     }
     B.steps = (int)T.step.size() - B.step0;
     T.step.push_back((unsigned short)B.rows);
-    B.halo = (int)in_halo.size();
-    for (int q : in_halo) slot_of[(size_t)q] = -1;
-    if (B.steps > kBlockSteps || B.halo > kBlockHalo) return false;
-    T.halo.insert(T.halo.end(), in_halo.begin(), in_halo.end());
+    if (B.steps > kBlockSteps) return false;
     T.halo_max = std::max(T.halo_max, B.halo);
   }
   return true;
@@ -536,20 +605,9 @@ void build_blocks(int n, const int *row, const int *col, const int *dia,
   // symmetric (the upper sweep runs the lower order backwards, which needs
   // every upper entry to mirror a lower one)
   int width = 0;
-  {
-    std::vector<int> next(row, row + n);  // per row, the first lower entry not yet mirrored
-    for (int i = 0; i < n; ++i) {
-      width = std::max({width, dia[i] - row[i], row[i + 1] - dia[i] - 1});
-      for (int j = dia[i] + 1; j < row[i + 1]; ++j) {
-        const int k = col[j];  // row k's lower columns ascend, so its mirrors come in order
-        if (next[(size_t)k] >= dia[k] || col[next[(size_t)k]] != i) return;
-        ++next[(size_t)k];
-      }
-    }
-    for (int i = 0; i < n; ++i)
-      if (next[(size_t)i] != dia[i]) return;
-  }
-  if (width > kBlockWide) return;
+  for (int i = 0; i < n; ++i)
+    width = std::max({width, dia[i] - row[i], row[i + 1] - dia[i] - 1});
+  if (width > kBlockWide || !symmetric_structure(n, row, col)) return;
   out.width = width <= 3 ? 3 : kBlockWide;
   // blocks per range of rows that no entry leaves (the systems of a batch)
   std::vector<int> blk((size_t)n);
@@ -637,20 +695,16 @@ void build_blocks(int n, const int *row, const int *col, const int *dia,
   if ((out.width > 3 ? 2.0 : 1.0) * (kBlockNs * nb + kBlockStepNs * (double)steps) >
       kLevelNs * nlev + kRowNs * n)
     return;
-  if (!build_block_triangle(row, col, dia, true, out.orig, out.of_orig, bstart, lstep, out.width,
-                            out.places(), out.L))
-    return;
-  // the upper triangle: everything backwards
-  std::vector<int> orig_u(out.orig.rbegin(), out.orig.rend()), of_u((size_t)n),
-      step_u((size_t)n), bstart_u((size_t)nb + 1);
-  for (int q = 0; q < n; ++q) {
-    of_u[(size_t)orig_u[(size_t)q]] = q;
-    step_u[(size_t)q] = -lstep[(size_t)(n - 1 - q)];
-  }
-  for (int k = 0; k <= nb; ++k) bstart_u[(size_t)k] = n - bstart[(size_t)(nb - k)];
-  if (!build_block_triangle(row, col, dia, false, orig_u, of_u, bstart_u, step_u, out.width,
-                            out.places(), out.U))
-    return;
+  std::vector<int> block_at((size_t)n);
+  for (int k = 0; k < nb; ++k)
+    std::fill(block_at.begin() + bstart[(size_t)k], block_at.begin() + bstart[(size_t)k + 1], k);
+  auto triangle = [&](bool lower) {
+    return build_block_triangle(n, row, col, dia, lower, out.of_orig, bstart, block_at, lstep,
+                                out.width, out.places(), lower ? out.L : out.U);
+  };
+  std::future<bool> upper = std::async(beside(n), triangle, false);
+  const bool fits = triangle(true);
+  if (!upper.get() || !fits) return;
   out.nblk = nb;
   out.depth = depth;
   out.ok = true;
@@ -895,18 +949,18 @@ double gather_lines(int n, const int *row, const int *col) {
   const int ngroup = (n + 63) / 64, step = std::max(1, ngroup / 256);
   long long lines = 0;
   int taken = 0;
-  std::vector<int> seen;
-  for (int g = 0; g < ngroup; g += step, ++taken) {
-    seen.clear();
-    for (int e = row[64 * g]; e < row[std::min(n, 64 * g + 64)]; ++e) seen.push_back(col[e] / 16);
-    std::sort(seen.begin(), seen.end());
-    lines += std::unique(seen.begin(), seen.end()) - seen.begin();
-  }
+  std::vector<int> last((size_t)n / 16 + 1, -1);   // the last group that touched each line
+  for (int g = 0; g < ngroup; g += step, ++taken)
+    for (int e = row[64 * g]; e < row[std::min(n, 64 * g + 64)]; ++e) {
+      int &l = last[(size_t)(col[e] / 16)];
+      lines += l != g;
+      l = g;
+    }
   return taken ? (double)lines / taken : 0.0;
 }
 
 void build_layout(int n, const int *row, const int *col, const int *dia, int spmv_rows,
-                  int spmv_cap, int small_level, Layout &out, bool identity_s) {
+                  int spmv_cap, int small_level, Layout &out, bool identity_s, BlockLayout *blocks) {
   out.n = n;
   out.nnz = n > 0 ? row[n] : 0;
   if (identity_s) {
@@ -917,35 +971,43 @@ void build_layout(int n, const int *row, const int *col, const int *dia, int spm
   }
   out.s_of_orig.assign(n, 0);
   for (int k = 0; k < n; ++k) out.s_of_orig[out.s_orig[k]] = k;
-  out.s_row.assign(n + 1, 0);
-  for (int k = 0; k < n; ++k) {
-    const int i = out.s_orig[k];
-    out.s_row[k + 1] = out.s_row[k] + row[i + 1] - row[i];
-  }
-  out.s_col.assign(out.nnz, 0);
-  out.s_src.assign(out.nnz, 0);
-  out.s_diag_src.assign(n, 0);
-  int bw = 0;
-  for (int k = 0; k < n; ++k) {
-    const int i = out.s_orig[k];
-    int e = out.s_row[k];
-    for (int j = row[i]; j < row[i + 1]; ++j, ++e) {
-      out.s_col[e] = out.s_of_orig[col[j]];
-      out.s_src[e] = j;
-      bw = std::max(bw, std::abs(out.s_col[e] - k));
+  // the S copy, beside the sweeps' orders
+  std::future<void> s_copy = std::async(beside(n), [&] {
+    out.s_row.assign(n + 1, 0);
+    for (int k = 0; k < n; ++k) {
+      const int i = out.s_orig[k];
+      out.s_row[k + 1] = out.s_row[k] + row[i + 1] - row[i];
     }
-    out.s_diag_src[k] = dia[i];
-  }
-  out.bandwidth = bw;
-  // SpMV row blocks: <= spmv_rows rows and <= spmv_cap entries each
-  out.s_rblk.assign(1, 0);
-  for (int r = 0; r < n;) {
-    int e = r + 1;
-    while (e < n && e - r < spmv_rows && out.s_row[e + 1] - out.s_row[r] <= spmv_cap) ++e;
-    out.s_rblk.push_back(e);
-    r = e;
-  }
+    out.s_col.assign(out.nnz, 0);
+    out.s_src.assign(out.nnz, 0);
+    out.s_diag_src.assign(n, 0);
+    int bw = 0;
+    for (int k = 0; k < n; ++k) {
+      const int i = out.s_orig[k];
+      int e = out.s_row[k];
+      for (int j = row[i]; j < row[i + 1]; ++j, ++e) {
+        out.s_col[e] = out.s_of_orig[col[j]];
+        out.s_src[e] = j;
+        bw = std::max(bw, std::abs(out.s_col[e] - k));
+      }
+      out.s_diag_src[k] = dia[i];
+    }
+    out.bandwidth = bw;
+    // SpMV row blocks: <= spmv_rows rows and <= spmv_cap entries each
+    out.s_rblk.assign(1, 0);
+    for (int r = 0; r < n;) {
+      int e = r + 1;
+      while (e < n && e - r < spmv_rows && out.s_row[e + 1] - out.s_row[r] <= spmv_cap) ++e;
+      out.s_rblk.push_back(e);
+      r = e;
+    }
+  });
   build_sweep(n, row, col, dia, true, out.s_of_orig, small_level, out.L);
+  std::future<void> block_sweeps;
+  if (blocks)
+    block_sweeps = std::async(beside(n), [&] {
+      build_blocks(n, row, col, dia, out.s_of_orig, out.L.nlev, *blocks);
+    });
   build_sweep(n, row, col, dia, false, out.s_of_orig, small_level, out.U,
               kMirrorUpper ? &out.L : nullptr);
   out.l_to_s.assign(n, 0);
@@ -954,6 +1016,8 @@ void build_layout(int n, const int *row, const int *col, const int *dia, int spm
   for (int p = 0; p < n; ++p) out.l_to_s[p] = out.s_of_orig[out.L.orig[p]];
   for (int q = 0; q < n; ++q) out.u_to_l[q] = out.L.of_orig[out.U.orig[q]];
   for (int k = 0; k < n; ++k) out.s_to_u[k] = out.U.of_orig[out.s_orig[k]];
+  s_copy.get();
+  if (blocks) block_sweeps.get();
 }
 
 namespace {

@@ -232,8 +232,10 @@ void short_columns(const std::vector<long long> &off, const std::vector<int> &co
 // up to 256 such groups spread over the matrix.
 double gather_lines(int n, const int *row, const int *col);
 
+// `blocks`: build_blocks' result too (null: not built).
 void build_layout(int n, const int *row, const int *col, const int *dia, int spmv_rows,
-                  int spmv_cap, int small_level, Layout &out, bool identity_s = false);
+                  int spmv_cap, int small_level, Layout &out, bool identity_s = false,
+                  BlockLayout *blocks = nullptr);
 
 // The faces of every cell for the kernels that give a cell one lane: 64 cells a
 // slice, slot-major, so that a wavefront's list entries are one contiguous run.

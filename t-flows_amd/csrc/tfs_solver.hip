@@ -20,6 +20,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 #include <vector>
 
@@ -296,6 +297,37 @@ int upload(tfs_matrix *A, T **dst, const std::vector<T> &src) {
   TFS_TRY(dev_alloc(A, (void **)dst, sizeof(T) * src.size()));
   if (!src.empty())
     TFS_HIP(hipMemcpy(*dst, src.data(), sizeof(T) * src.size(), hipMemcpyHostToDevice));
+  return 0;
+}
+
+// Arrays that live and go together: one allocation, and one copy while they are
+// small (a copy costs about 20 us however short it is).
+struct Part {
+  void **dst;
+  const void *src;
+  size_t bytes;
+  template <typename T>
+  Part(T **d, const std::vector<T> &v)
+      : dst((void **)d), src(v.data()), bytes(sizeof(T) * v.size()) {}
+};
+int upload(tfs_matrix *A, std::initializer_list<Part> parts) {
+  constexpr size_t kAlign = 256, kTogether = 1 << 20;
+  auto room = [](const Part &p) { return (p.bytes + kAlign - 1) / kAlign * kAlign; };
+  size_t total = 0;
+  for (const Part &p : parts) total += room(p);
+  char *mem = nullptr;
+  TFS_TRY(dev_alloc(A, (void **)&mem, total));
+  std::vector<char> host(total <= kTogether ? total : 0);
+  size_t at = 0;
+  for (const Part &p : parts) {
+    *p.dst = mem + at;
+    if (p.bytes > 0 && !host.empty())
+      std::memcpy(host.data() + at, p.src, p.bytes);
+    else if (p.bytes > 0)
+      TFS_HIP(hipMemcpy(mem + at, p.src, p.bytes, hipMemcpyHostToDevice));
+    at += room(p);
+  }
+  if (!host.empty()) TFS_HIP(hipMemcpy(mem, host.data(), total, hipMemcpyHostToDevice));
   return 0;
 }
 
@@ -1918,23 +1950,10 @@ int build_ell64(tfs_matrix *A, const Layout &Ly) {
 // The block sweeps' structure, if it suits them, and their grid: at most half
 // the workgroups that fit at once.  Twice as many measured no faster, and none of
 // them has to be resident (k_block_sweep).
-int build_block_sweeps(tfs_matrix *A, const Layout &Ly, const int *row, const int *col,
-                       const int *dia) {
+int build_block_sweeps(tfs_matrix *A, const Layout &Ly, const BlockLayout &BL, const int *dia) {
   const int n = A->n;
-  BlockLayout BL;
-  build_blocks(n, row, col, dia, Ly.s_of_orig, Ly.L.nlev, BL);
   if (!BL.ok) return 0;
-  const BlockTriangle *T[2] = {&BL.L, &BL.U};
-  DevBlocks *D[2] = {&A->bL, &A->bU};
-  for (int k = 0; k < 2; ++k) {
-    TFS_TRY(upload(A, &D[k]->blk, T[k]->blk));
-    TFS_TRY(upload(A, &D[k]->step, T[k]->step));
-    TFS_TRY(upload(A, &D[k]->idx, T[k]->idx));
-    TFS_TRY(upload(A, &D[k]->src, T[k]->src));
-    TFS_TRY(upload(A, &D[k]->halo, T[k]->halo));
-    D[k]->slots = (long long)T[k]->src.size();
-    D[k]->halo_max = T[k]->halo_max;
-  }
+  DevBlocks &L = A->bL, &U = A->bU;
   std::vector<int> to_s((size_t)n), bz((size_t)n), dsrc((size_t)n);
   for (int p = 0; p < n; ++p) {
     const int i = BL.orig[(size_t)p];
@@ -1942,10 +1961,15 @@ int build_block_sweeps(tfs_matrix *A, const Layout &Ly, const int *row, const in
     dsrc[(size_t)p] = dia[i];
     bz[(size_t)to_s[(size_t)p]] = n - 1 - p;
   }
-  TFS_TRY(upload(A, &A->b_to_s, to_s));
-  TFS_TRY(upload(A, &A->s_to_bz, bz));
-  TFS_TRY(upload(A, &A->b_diag_src, dsrc));
-  TFS_TRY(upload(A, &A->b_of_orig, BL.of_orig));
+  TFS_TRY(upload(A, {{&L.blk, BL.L.blk}, {&L.step, BL.L.step}, {&L.idx, BL.L.idx},
+                     {&L.src, BL.L.src}, {&L.halo, BL.L.halo}, {&U.blk, BL.U.blk},
+                     {&U.step, BL.U.step}, {&U.idx, BL.U.idx}, {&U.src, BL.U.src},
+                     {&U.halo, BL.U.halo}, {&A->b_to_s, to_s}, {&A->s_to_bz, bz},
+                     {&A->b_diag_src, dsrc}, {&A->b_of_orig, BL.of_orig}}));
+  L.slots = (long long)BL.L.src.size();
+  U.slots = (long long)BL.U.src.size();
+  L.halo_max = BL.L.halo_max;
+  U.halo_max = BL.U.halo_max;
   A->blk_n = BL.nblk;
   A->blk_width = BL.width;
   const size_t lds = block_lds(BL.width, std::max(BL.L.halo_max, BL.U.halo_max));
@@ -1983,8 +2007,8 @@ int occupancy(int *per_cu) {
   return 0;
 }
 
-int create_device(tfs_matrix *A, const Layout &Ly, const int *row, const int *col,
-                  const int *dia, bool blocks, bool direct) {
+int create_device(tfs_matrix *A, const Layout &Ly, const BlockLayout &BL, const int *row,
+                  const int *col, const int *dia, bool direct) {
   const int n = A->n;
   TFS_HIP(hipStreamCreateWithFlags(&A->stream, hipStreamNonBlocking));
   TFS_HIP(hipEventCreate(&A->ev0));
@@ -2015,17 +2039,15 @@ int create_device(tfs_matrix *A, const Layout &Ly, const int *row, const int *co
     for (int k = 0; k < n; ++k) lpos[(size_t)k] = Ly.L.of_orig[(size_t)Ly.s_orig[(size_t)k]];
     TFS_TRY(upload(A, &A->s_lpos, lpos));
   }
-  if (blocks) TFS_TRY(build_block_sweeps(A, Ly, row, col, dia));
   // (`direct`: matrices whose caller can ask for a product of its own vectors)
   if (direct && n > 0 &&
       gather_lines(n, row, col) <= kDirectLines * gather_lines(n, Ly.s_row.data(), Ly.s_col.data())) {
     const std::vector<int> crow(row, row + n + 1), ccol(col, col + A->nnz);
     const std::vector<int> crb = row_blocks(crow, kSpmvRows);
-    TFS_TRY(upload(A, &A->c_row, crow));
-    TFS_TRY(upload(A, &A->c_col, ccol));
-    TFS_TRY(upload(A, &A->c_rblk, crb));
+    TFS_TRY(upload(A, {{&A->c_row, crow}, {&A->c_col, ccol}, {&A->c_rblk, crb}}));
     A->c_nblk = (int)crb.size() - 1;
   }
+  TFS_TRY(build_block_sweeps(A, Ly, BL, dia));
   const size_t nb = sizeof(double) * (size_t)std::max(n, 1);
   TFS_TRY(dev_alloc(A, (void **)&A->val, sizeof(double) * (size_t)std::max(A->nnz, 1LL)));
   TFS_TRY(dev_alloc(A, (void **)&A->stage_x, nb));
@@ -2143,12 +2165,13 @@ int matrix_create(int n, long long nnz, const int *row, const int *col, const in
 
   Layout local;
   Layout &Ly = keep ? *keep : local;
-  build_layout(n, hr.data(), hc.data(), hd.data(), kSpmvRows, kSpmvCap, kSmallLevel, Ly,
-               identity_s);
+  BlockLayout BL;
+  build_layout(n, hr.data(), hc.data(), hd.data(), kSpmvRows, kSpmvCap, kSmallLevel, Ly, identity_s,
+               blocks ? &BL : nullptr);
   tfs_matrix *A = new tfs_matrix;
   A->n = n;
   A->nnz = nnz;
-  const int rc = create_device(A, Ly, hr.data(), hc.data(), hd.data(), blocks, direct);
+  const int rc = create_device(A, Ly, BL, hr.data(), hc.data(), hd.data(), direct);
   if (rc < 0) {
     tfs_matrix_destroy(A);
     return rc;
