@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <future>
 #include <vector>
 
 #include "tfs_faces.hpp"
@@ -103,6 +104,22 @@ __global__ void __launch_bounds__(kThreads) k_zero(long long m, double *__restri
     v[i] = 0.0;
 }
 
+// f(first, last) over [0, n), parts of it beside one another where they are long
+// enough for threads of their own.
+template <typename F>
+void in_parts(int n, F f) {
+  constexpr int kParts = 8;
+  if (n < 1 << 12) {
+    f(0, n);
+    return;
+  }
+  std::future<void> part[kParts];
+  for (int k = 0; k < kParts; ++k)
+    part[k] = std::async(std::launch::async | std::launch::deferred, f,
+                         (int)((long long)n * k / kParts), (int)((long long)n * (k + 1) / kParts));
+  for (std::future<void> &p : part) p.get();
+}
+
 int grid_of(long long m) { return (int)std::max(1LL, std::min(4096LL, (m + kThreads - 1) / kThreads)); }
 
 }  // namespace
@@ -137,11 +154,11 @@ extern "C" int tfs_assembly_create(tfs_matrix *A, long long n_faces, const int *
   const int n = info.n;
   const long long nf = n_faces, nnz = info.nnz;
   std::vector<int> hdia((size_t)n);
-  std::vector<unsigned char> written((size_t)nnz, 0);   // 1 by a face, 2 a diagonal
+  std::vector<bool> diagonal((size_t)nnz);   // bits: they are looked up in any order
   for (int c = 0; c < n; ++c) {
     hdia[(size_t)c] = dia[c] - base;
     if (hdia[(size_t)c] < 0 || hdia[(size_t)c] >= nnz) return TFS_ERR_INVALID;
-    written[(size_t)hdia[(size_t)c]] = 2;
+    diagonal[(size_t)hdia[(size_t)c]] = true;
   }
   for (long long s = 0; s < nf; ++s) {
     const int c1 = faces_c[2 * s] - base, c2 = faces_c[2 * s + 1] - base;
@@ -149,57 +166,78 @@ extern "C" int tfs_assembly_create(tfs_matrix *A, long long n_faces, const int *
     for (int k = 0; k < 2 && c2 >= 0; ++k) {
       const long long q = (long long)pos[2 * s + k] - base;
       if (q < 0 || q >= nnz) return TFS_ERR_INVALID;
-      if (!written[(size_t)q]) written[(size_t)q] = 1;
     }
   }
   FaceLists F;
   build_face_lists(n, nf, faces_c, base, kReorderAssembly, F);
-  std::vector<int> hpos(F.inc.size() + F.tail.size(), kBoundary);
+  // where each entry goes, slice by slice, and how many of a slice go anywhere
+  const int nslice = (n + 63) / 64;
+  std::vector<int> hpos(F.inc.size() + F.tail.size(), kBoundary), first((size_t)nslice + 1, 0);
   auto place = [&](unsigned e) {
     const long long s = e >> 1;
     if (faces_c[2 * s + 1] < base) return kBoundary;
     const int q = pos[2 * s + (e & 1)] - base;
-    return written[(size_t)q] == 2 ? kDropped : q;
+    return diagonal[(size_t)q] ? kDropped : q;
   };
-  for (size_t i = 0; i < F.inc.size(); ++i)
-    if (F.inc[i] != kNoFace) hpos[i] = place(F.inc[i]);
-  for (size_t t = 0; t < F.tail.size(); ++t) hpos[F.inc.size() + t] = place(F.tail[t]);
+  // the tail entries of a slice's cells
+  auto tails = [&](int s, int k) {
+    return F.tptr.empty() ? 0 : F.tptr[(size_t)std::min(n, 64 * s + k)];
+  };
+  in_parts(nslice, [&](int s0, int s1) {
+    for (int s = s0; s < s1; ++s) {
+      int go = std::min(n, 64 * s + 64) - 64 * s;   // the diagonals
+      for (size_t i = (size_t)F.off[(size_t)s]; i < (size_t)F.off[(size_t)s + 1]; ++i)
+        if (F.inc[i] != kNoFace) go += (hpos[i] = place(F.inc[i])) >= 0;
+      for (int t = tails(s, 0); t < tails(s, 64); ++t)
+        go += (hpos[F.inc.size() + (size_t)t] = place(F.tail[(size_t)t])) >= 0;
+      first[(size_t)s + 1] = go;
+    }
+  });
   // rows in the lists' order, each one's entries as they stand in val
   std::vector<int> src, to_dia((size_t)n);
-  int nrows = 0;
+  for (int s = 0; s < nslice; ++s) first[(size_t)s + 1] += first[(size_t)s];
+  const int nrows = first[(size_t)nslice];
+  bool clear = false;   // entries that nothing writes (k_place sets them itself)
   if (F.reordered) {
     src.assign((size_t)nnz, -1);
-    std::vector<int *> mine;   // where this row's places are, by place
-    auto add = [&](int *q) {
-      mine.push_back(q);
-      for (size_t j = mine.size() - 1; j > 0 && *mine[j - 1] > *mine[j]; --j)
-        std::swap(mine[j - 1], mine[j]);
-    };
-    for (int k = 0; k < n; ++k) {
-      const long long i0 = F.off[(size_t)(k / 64)] + k % 64, i1 = F.off[(size_t)(k / 64) + 1];
-      mine.clear();
-      for (long long i = i0; i < i1; i += 64)
-        if (hpos[(size_t)i] >= 0) add(&hpos[(size_t)i]);
-      if (!F.tptr.empty()) {
-        for (int t = F.tptr[(size_t)k]; t < F.tptr[(size_t)k + 1]; ++t)
-          if (hpos[F.inc.size() + (size_t)t] >= 0) mine.push_back(&hpos[F.inc.size() + (size_t)t]);
-        std::stable_sort(mine.begin(), mine.end(), [](int *a, int *b) { return *a < *b; });
+    in_parts(nslice, [&](int s0, int s1) {
+      std::vector<int *> mine;   // where this row's places are, by place
+      auto add = [&](int *q) {
+        mine.push_back(q);
+        for (size_t j = mine.size() - 1; j > 0 && *mine[j - 1] > *mine[j]; --j)
+          std::swap(mine[j - 1], mine[j]);
+      };
+      for (int k = 64 * s0, at = first[(size_t)s0]; k < std::min(n, 64 * s1); ++k) {
+        const long long i0 = F.off[(size_t)(k / 64)] + k % 64, i1 = F.off[(size_t)(k / 64) + 1];
+        mine.clear();
+        for (long long i = i0; i < i1; i += 64)
+          if (hpos[(size_t)i] >= 0) add(&hpos[(size_t)i]);
+        if (!F.tptr.empty()) {
+          for (int t = F.tptr[(size_t)k]; t < F.tptr[(size_t)k + 1]; ++t)
+            if (hpos[F.inc.size() + (size_t)t] >= 0) mine.push_back(&hpos[F.inc.size() + (size_t)t]);
+          std::stable_sort(mine.begin(), mine.end(), [](int *a, int *b) { return *a < *b; });
+        }
+        to_dia[(size_t)k] = hdia[(size_t)F.orig[(size_t)k]];
+        add(&to_dia[(size_t)k]);
+        for (int *q : mine) {
+          src[(size_t)*q] = at;
+          *q = at++;
+        }
       }
-      to_dia[(size_t)k] = hdia[(size_t)F.orig[(size_t)k]];
-      add(&to_dia[(size_t)k]);
-      for (int *q : mine) {
-        src[(size_t)*q] = nrows;
-        *q = nrows++;
-      }
-    }
+    });
   } else {
     to_dia = hdia;
+    std::vector<unsigned char> written((size_t)nnz, 0);
+    for (const int q : hdia) written[(size_t)q] = 1;
+    for (const int q : hpos)
+      if (q >= 0) written[(size_t)q] = 1;
+    clear = std::count(written.begin(), written.end(), (unsigned char)0) > 0;
   }
   auto *S = new tfs_assembly;
   S->A = A;
   S->nf = nf;
   S->nnz = nnz;
-  S->clear = !F.reordered && std::count(written.begin(), written.end(), (unsigned char)0) > 0;
+  S->clear = clear;
   auto up = [](void **dst, const void *src, size_t bytes) -> bool {
     if (hipMalloc(dst, std::max<size_t>(bytes, 8)) != hipSuccess) return false;
     return bytes == 0 || hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice) == hipSuccess;

@@ -1023,27 +1023,31 @@ void build_layout(int n, const int *row, const int *col, const int *dia, int spm
 namespace {
 
 // 128-byte lines of a cell field and of a face field that the slices of an
-// order touch, summed over up to 256 slices spread over the mesh.
-long long lines_touched(int n, const int *faces, int base, const std::vector<int> &ptr,
+// order touch, summed over up to 256 slices spread over the mesh.  Lists and
+// pairs are by position in the order of first naming: that order's lines or, with
+// `orig` and `of`, the caller's.
+long long lines_touched(int n, const std::vector<int> &pair, const std::vector<int> &ptr,
                         const std::vector<unsigned> &inc, const std::vector<int> *orig,
                         const std::vector<int> *of) {
   const int nslice = (n + 63) / 64, step = std::max(1, nslice / 256);
   long long lines = 0;
-  std::vector<long long> seen;
+  // the last slice that touched each line of the cell and of the face field
+  std::vector<int> cell_line((size_t)n / 16 + 1, -1), face_line(pair.size() / 32 + 1, -1);
   for (int s = 0; s < nslice; s += step) {
-    seen.clear();
+    auto touch = [&](int &line) {
+      lines += line != s;
+      line = s;
+    };
     for (int k = 64 * s; k < std::min(n, 64 * s + 64); ++k) {
-      const int c = orig ? (*orig)[(size_t)k] : k;
-      seen.push_back(k / 16);
-      for (int e = ptr[(size_t)c]; e < ptr[(size_t)c + 1]; ++e) {
+      const int p = of ? (*of)[(size_t)k] : k;
+      touch(cell_line[(size_t)(k / 16)]);
+      for (int e = ptr[(size_t)p]; e < ptr[(size_t)p + 1]; ++e) {
         const long long f = inc[(size_t)e] >> 1;
-        const int o = faces[2 * f + ((inc[(size_t)e] & 1) ? 0 : 1)] - base;
-        seen.push_back(-1 - f / 16);
-        if (o >= 0) seen.push_back((of ? (*of)[(size_t)o] : o) / 16);
+        const int o = pair[(size_t)(2 * f + ((inc[(size_t)e] & 1) ? 0 : 1))];
+        touch(face_line[(size_t)(f / 16)]);
+        if (o >= 0) touch(cell_line[(size_t)((orig ? (*orig)[(size_t)o] : o) / 16)]);
       }
     }
-    std::sort(seen.begin(), seen.end());
-    lines += std::unique(seen.begin(), seen.end()) - seen.begin();
   }
   return lines;
 }
@@ -1053,40 +1057,41 @@ long long lines_touched(int n, const int *faces, int base, const std::vector<int
 void build_face_lists(int n, long long nf, const int *faces, int base, int from, FaceLists &out) {
   out = FaceLists();
   out.n = n;
-  // per cell, its faces in ascending order (a counting sort over the faces)
-  std::vector<int> ptr((size_t)n + 1, 0);
-  for (long long s = 0; s < nf; ++s) {
-    ptr[(size_t)(faces[2 * s] - base) + 1]++;
-    if (faces[2 * s + 1] >= base) ptr[(size_t)(faces[2 * s + 1] - base) + 1]++;
-  }
-  for (int c = 0; c < n; ++c) ptr[(size_t)c + 1] += ptr[(size_t)c];
-  std::vector<unsigned> inc((size_t)ptr[(size_t)n]);
-  {
-    std::vector<int> fill(ptr.begin(), ptr.end() - 1);
-    for (long long s = 0; s < nf; ++s) {
-      inc[(size_t)fill[(size_t)(faces[2 * s] - base)]++] = (unsigned)(2 * s);
-      if (faces[2 * s + 1] >= base)
-        inc[(size_t)fill[(size_t)(faces[2 * s + 1] - base)]++] = (unsigned)(2 * s + 1);
-    }
-  }
-  // the order of first naming (cells of no face last)
-  std::vector<int> orig, of;
-  if (n >= from) {
+  // Both cells of each face (boundary: -1), from `from` cells on by position in the
+  // order of first naming (cells of no face last): whatever is done per cell below
+  // then goes through memory in runs, the one random access a face's cell being its
+  // position.
+  const bool named = n >= from;
+  std::vector<int> orig, of, pair((size_t)(2 * nf));
+  if (named) {
     of.assign((size_t)n, -1);
     orig.reserve((size_t)n);
   }
   auto name = [&](int c) {
-    if (c < 0 || of[(size_t)c] >= 0) return;
-    of[(size_t)c] = (int)orig.size();
-    orig.push_back(c);
+    if (c < 0) return -1;
+    if (!named) return c;
+    int &p = of[(size_t)c];
+    if (p < 0) {
+      p = (int)orig.size();
+      orig.push_back(c);
+    }
+    return p;
   };
-  for (long long s = 0; s < nf && n >= from; ++s) {
-    name(faces[2 * s] - base);
-    name(faces[2 * s + 1] - base);
+  for (long long k = 0; k < 2 * nf; ++k) pair[(size_t)k] = name(faces[k] - base);
+  for (int c = 0; c < n && named; ++c) name(c);
+  // per cell, its faces in ascending order (a counting sort over the faces)
+  std::vector<int> ptr((size_t)n + 1, 0);
+  for (const int p : pair)
+    if (p >= 0) ptr[(size_t)p + 1]++;
+  for (int c = 0; c < n; ++c) ptr[(size_t)c + 1] += ptr[(size_t)c];
+  std::vector<unsigned> inc((size_t)ptr[(size_t)n]);
+  {
+    std::vector<int> fill(ptr.begin(), ptr.end() - 1);
+    for (long long k = 0; k < 2 * nf; ++k)
+      if (pair[(size_t)k] >= 0) inc[(size_t)fill[(size_t)pair[(size_t)k]]++] = (unsigned)k;
   }
-  for (int c = 0; c < n && n >= from; ++c) name(c);
-  if (n >= from && lines_touched(n, faces, base, ptr, inc, nullptr, nullptr) >
-      2 * lines_touched(n, faces, base, ptr, inc, &orig, &of)) {
+  if (named && lines_touched(n, pair, ptr, inc, &orig, &of) >
+                   2 * lines_touched(n, pair, ptr, inc, nullptr, nullptr)) {
     out.reordered = true;
     out.orig = std::move(orig);
     out.of = std::move(of);
@@ -1094,7 +1099,7 @@ void build_face_lists(int n, long long nf, const int *faces, int base, int from,
   const int nslice = (n + 63) / 64;
   out.off.assign((size_t)nslice + 1, 0);
   bool tails = false;
-  auto cell = [&](int k) { return out.reordered ? out.orig[(size_t)k] : k; };
+  auto cell = [&](int k) { return named && !out.reordered ? of[(size_t)k] : k; };   // in ptr
   auto width = [&](int c) { return ptr[(size_t)c + 1] - ptr[(size_t)c]; };
   for (int s = 0; s < nslice; ++s) {
     int w = 0;
