@@ -26,7 +26,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <future>
 #include <vector>
 
 #include "tfs_faces.hpp"
@@ -104,22 +103,6 @@ __global__ void __launch_bounds__(kThreads) k_zero(long long m, double *__restri
     v[i] = 0.0;
 }
 
-// f(first, last) over [0, n), parts of it beside one another where they are long
-// enough for threads of their own.
-template <typename F>
-void in_parts(int n, F f) {
-  constexpr int kParts = 8;
-  if (n < 1 << 12) {
-    f(0, n);
-    return;
-  }
-  std::future<void> part[kParts];
-  for (int k = 0; k < kParts; ++k)
-    part[k] = std::async(std::launch::async | std::launch::deferred, f,
-                         (int)((long long)n * k / kParts), (int)((long long)n * (k + 1) / kParts));
-  for (std::future<void> &p : part) p.get();
-}
-
 int grid_of(long long m) { return (int)std::max(1LL, std::min(4096LL, (m + kThreads - 1) / kThreads)); }
 
 }  // namespace
@@ -183,7 +166,7 @@ extern "C" int tfs_assembly_create(tfs_matrix *A, long long n_faces, const int *
   auto tails = [&](int s, int k) {
     return F.tptr.empty() ? 0 : F.tptr[(size_t)std::min(n, 64 * s + k)];
   };
-  in_parts(nslice, [&](int s0, int s1) {
+  in_parts(nslice, 1 << 12, [&](int, int s0, int s1) {
     for (int s = s0; s < s1; ++s) {
       int go = std::min(n, 64 * s + 64) - 64 * s;   // the diagonals
       for (size_t i = (size_t)F.off[(size_t)s]; i < (size_t)F.off[(size_t)s + 1]; ++i)
@@ -200,7 +183,7 @@ extern "C" int tfs_assembly_create(tfs_matrix *A, long long n_faces, const int *
   bool clear = false;   // entries that nothing writes (k_place sets them itself)
   if (F.reordered) {
     src.assign((size_t)nnz, -1);
-    in_parts(nslice, [&](int s0, int s1) {
+    in_parts(nslice, 1 << 12, [&](int, int s0, int s1) {
       std::vector<int *> mine;   // where this row's places are, by place
       auto add = [&](int *q) {
         mine.push_back(q);

@@ -2,6 +2,8 @@
 #include "tfs_layout.hpp"
 
 #include <algorithm>
+#include <atomic>
+#include <climits>
 #include <cstdint>
 #include <future>
 #include <unordered_map>
@@ -718,27 +720,6 @@ void build_bricks(int n, const int *row, const int *col, const int *dia,
   const int nb = (int)colour.size();
   int ncol = 0;
   for (int c : colour) ncol = std::max(ncol, c + 1);
-  // levels inside the blocks, and the couplings between them
-  std::vector<int> lev((size_t)n, 0);
-  for (int i = 0; i < n; ++i) {
-    if (dia[i] - row[i] > kBrickWide || row[i + 1] - dia[i] - 1 > kBrickWide) return;
-    const int b = blk[(size_t)i];
-    for (int e = row[i]; e < row[i + 1]; ++e) {
-      const int j = col[e], bj = blk[(size_t)j];
-      if (bj != b) {
-        if ((j < i) != (colour[(size_t)bj] < colour[(size_t)b]) ||
-            colour[(size_t)bj] == colour[(size_t)b])
-          return;
-      } else if (j < i) {
-        lev[(size_t)i] = std::max(lev[(size_t)i], lev[(size_t)j] + 1);
-      }
-    }
-  }
-  // a block's upper couplings must climb in level (they do where the pattern is
-  // structurally symmetric)
-  for (int i = 0; i < n; ++i)
-    for (int e = dia[i] + 1; e < row[i + 1]; ++e)
-      if (blk[(size_t)col[e]] == blk[(size_t)i] && lev[(size_t)col[e]] <= lev[(size_t)i]) return;
   // units: blocks by colour, then number, merged up to kUnitFull rows
   std::vector<int> unit_of((size_t)nb), brows((size_t)nb, 0), count;
   for (int i = 0; i < n; ++i) brows[(size_t)blk[(size_t)i]]++;
@@ -765,146 +746,213 @@ void build_bricks(int n, const int *row, const int *col, const int *dia,
   }
   auto nlow = [&](int i) { return dia[i] - row[i]; };
   auto nup = [&](int i) { return row[i + 1] - dia[i] - 1; };
-  // per row: its step in the unit, then (per triangle) its slot; per halo row its slot
-  std::vector<int> step_of((size_t)n), slot((size_t)n, -1), hslot((size_t)n, -1), halo, last;
-  std::vector<std::pair<uint64_t, int>> keys;
-  std::vector<int> start;                       // first row of each step
-  std::vector<std::vector<int>> dies;           // slots whose last reader is in a step
+  // per row its level in its block, its step in the unit, then (per triangle) its slot
+  std::vector<int> lev((size_t)n, 0), step_of((size_t)n), slot((size_t)n, -1);
   out.unit.resize((size_t)nu);
-  std::vector<BrickPlaces> more_idx[2];
-  std::vector<BrickSource> more_src[2];
-  for (int k = 0; k < nu; ++k) {
-    BrickUnit &B = out.unit[(size_t)k];
-    B.row0 = first[(size_t)k];
-    B.rows = count[(size_t)k];
-    B.step0 = (int)out.L.step.size();
-    if (B.rows > kUnitRows) return;
-    int *const r = out.row.data() + B.row0;
-    int wl = 0, wu = 0;
-    for (int p = 0; p < B.rows; ++p) {
-      wl = std::max(wl, nlow(r[p]));
-      wu = std::max(wu, nup(r[p]));
-    }
-    auto more = [&](int i) { return (wl > wu ? nlow(i) : nup(i)) > 3; };
-    // by level, rows with second records first, then S position
-    keys.clear();
-    for (int p = 0; p < B.rows; ++p)
-      keys.push_back({(uint64_t)lev[(size_t)r[p]] << 33 | (uint64_t)!more(r[p]) << 32 |
-                          (uint32_t)s_of[(size_t)r[p]],
-                      r[p]});
-    std::sort(keys.begin(), keys.end());
-    for (int p = 0; p < B.rows; ++p) r[p] = keys[(size_t)p].second;
-    start.clear();
-    for (int p = 0; p < B.rows; ++p) {
-      if (p == 0 || lev[(size_t)r[p]] != lev[(size_t)r[p - 1]] || p - start.back() == kBrickLanes)
-        start.push_back(p);
-      step_of[(size_t)r[p]] = (int)start.size() - 1;
-    }
-    B.steps = (int)start.size();
-    start.push_back(B.rows);
-    out.steps = std::max(out.steps, B.steps);
-    const size_t base = out.L.idx.size();
-    for (int t = 0; t < 2; ++t) {
-      BrickTriangle &T = t == 0 ? out.L : out.U;
-      auto when = [&](int x) {  // sweep order of a row's step
-        return t == 0 ? step_of[(size_t)x] : B.steps - 1 - step_of[(size_t)x];
-      };
-      auto entries = [&](int x, auto &&f) {
-        const int e0 = t == 0 ? row[x] : dia[x] + 1, w = t == 0 ? nlow(x) : nup(x);
-        for (int j = 0; j < w; ++j) f(j, e0 + j, col[e0 + j]);
-      };
-      // the last step that reads each value of the unit and its halo
-      halo.clear();
-      last.assign((size_t)B.rows, -1);
-      std::vector<int> hlast;
-      for (int p = 0; p < B.rows; ++p) slot[(size_t)r[p]] = p;  // (for now its row in the unit)
-      for (int p = 0; p < B.rows; ++p)
-        entries(r[p], [&](int, int, int y) {
-          if (blk[(size_t)y] == blk[(size_t)r[p]]) {
-            int &l = last[(size_t)slot[(size_t)y]];
-            l = std::max(l, when(r[p]));
-          } else {
-            if (hslot[(size_t)y] < 0) {
-              hslot[(size_t)y] = (int)halo.size();
-              halo.push_back(y);
-              hlast.push_back(0);
-            }
-            int &l = hlast[(size_t)hslot[(size_t)y]];
-            l = std::max(l, when(r[p]));
-          }
-        });
-      // slots in sweep order
-      if ((int)dies.size() < B.steps) dies.resize((size_t)B.steps);
-      for (int q = 0; q < B.steps; ++q) dies[(size_t)q].clear();
-      int slots = 1 + (int)halo.size();
-      for (size_t h = 0; h < halo.size(); ++h) {
-        dies[(size_t)hlast[h]].push_back(1 + (int)h);
-        hslot[(size_t)halo[h]] = 1 + (int)h;
-      }
-      std::vector<int> unused;
-      T.idx.resize(base + (size_t)B.rows);
-      T.src.resize(base + (size_t)B.rows);
-      const size_t step0 = T.step.size();
-      T.step.resize(step0 + (size_t)B.steps);
-      for (int q = 0; q < B.steps; ++q) {
-        const int at_step = t == 0 ? q : B.steps - 1 - q;
-        const int c = start[(size_t)at_step], m = start[(size_t)at_step + 1] - c;
-        if (q > 0)
-          for (int s : dies[(size_t)q - 1]) unused.push_back(s);
-        for (int i = 0; i < m; ++i) {
-          const int x = r[c + i];
-          const int l = last[(size_t)(c + i)];
-          int s;
-          if (!unused.empty()) {
-            s = unused.back();
-            unused.pop_back();
-          } else {
-            s = slots++;
-          }
-          dies[(size_t)std::max(l, q)].push_back(s);
-          slot[(size_t)x] = s;
-          if (s > 0x3fff) return;  // 16-bit byte offsets
-        }
-        int more_rows = 0;
-        for (int i = 0; i < m; ++i)
-          if ((t == 0 ? nlow(r[c + i]) : nup(r[c + i])) > 3) more_rows = i + 1;
-        T.step[step0 + (size_t)at_step] = {(int)more_idx[t].size(),
-                                           (unsigned)(c | m << 12 | more_rows << 20)};
-        for (int i = 0; i < m; ++i) {
-          const int x = r[c + i];
-          BrickPlaces at[2] = {{{0, 0, 0, 0}}, {{0, 0, 0, 0}}};
-          BrickSource from[2] = {{{-1, -1, -1, x}}, {{-1, -1, -1, -1}}};
-          entries(x, [&](int j, int e, int y) {
-            const int s = blk[(size_t)y] == blk[(size_t)x] ? slot[(size_t)y] : hslot[(size_t)y];
-            at[j / 3].at[j % 3] = (unsigned short)(s * sizeof(float));
-            from[j / 3].e[j % 3] = e;
-          });
-          at[0].at[3] = (unsigned short)(slot[(size_t)x] * sizeof(float));
-          T.idx[base + (size_t)(c + i)] = at[0];
-          T.src[base + (size_t)(c + i)] = from[0];
-          if (i < more_rows) {
-            more_idx[t].push_back(at[1]);
-            more_src[t].push_back(from[1]);
-          }
-        }
-      }
-      (t == 0 ? B.lh0 : B.uh0) = (int)T.halo.size();
-      (t == 0 ? B.lh : B.uh) = (int)halo.size();
-      for (int y : halo) {
-        T.halo.push_back(s_of[(size_t)y]);
-        hslot[(size_t)y] = -1;
-      }
-      out.slots[t] = std::max(out.slots[t], slots);
-    }
+  // Units go in parts beside one another, each with its own steps, second records
+  // and halos, which are joined after.
+  struct Joined {
+    std::vector<BrickStep> step;
+    std::vector<int> halo;
+    std::vector<BrickPlaces> more_idx;
+    std::vector<BrickSource> more_src;
+    int slots = 0;
+  };
+  struct Part {
+    Joined of[2];   // lower, upper
+    int first = 0, last = 0, steps = 0;
+    bool ok = true;
+  };
+  std::vector<Part> part((size_t)kBeside);
+  for (BrickTriangle *T : {&out.L, &out.U}) {
+    T->idx.resize((size_t)n);
+    T->src.resize((size_t)n);
   }
+  in_parts(nu, 64, [&](int which, int k0, int k1) {
+    Part &P = part[(size_t)which];
+    P.first = k0;
+    P.last = k1;
+    P.ok = false;
+    // the halo number of a row in this unit and triangle
+    constexpr unsigned kTable = 1 << 15;
+    constexpr size_t kHaloMost = 0x3ffe;   // more leave no slot for a row (16-bit offsets)
+    struct Entry { int when = -1, y = 0, h = 0; };
+    std::vector<Entry> table(kTable);
+    auto halo_at = [&](int stamp, int y) -> Entry & {
+      unsigned t = (unsigned)y * 2654435761u >> 17;
+      while (table[t].when == stamp && table[t].y != y) t = (t + 1) % kTable;
+      return table[t];
+    };
+    std::vector<int> halo, hlast, last, start, unused;   // start: first row of each step
+    std::vector<std::pair<uint64_t, int>> keys;
+    std::vector<std::vector<int>> dies;           // slots whose last reader is in a step
+    for (int k = k0; k < k1; ++k) {
+      BrickUnit &B = out.unit[(size_t)k];
+      B.row0 = first[(size_t)k];
+      B.rows = count[(size_t)k];
+      B.step0 = (int)P.of[0].step.size();
+      if (B.rows > kUnitRows) return;
+      int *const r = out.row.data() + B.row0;
+      // levels inside the blocks, and the couplings between them
+      int wl = 0, wu = 0;
+      for (int p = 0; p < B.rows; ++p) {
+        const int i = r[p], b = blk[(size_t)i];
+        wl = std::max(wl, nlow(i));
+        wu = std::max(wu, nup(i));
+        for (int e = row[i]; e < row[i + 1]; ++e) {
+          const int j = col[e], bj = blk[(size_t)j];
+          if (bj != b) {
+            if ((j < i) != (colour[(size_t)bj] < colour[(size_t)b]) ||
+                colour[(size_t)bj] == colour[(size_t)b])
+              return;
+          } else if (j < i) {
+            lev[(size_t)i] = std::max(lev[(size_t)i], lev[(size_t)j] + 1);
+          }
+        }
+      }
+      if (wl > kBrickWide || wu > kBrickWide) return;
+      // a block's upper couplings must climb in level (they do where the pattern is
+      // structurally symmetric)
+      for (int p = 0; p < B.rows; ++p)
+        for (int e = dia[r[p]] + 1; e < row[r[p] + 1]; ++e)
+          if (blk[(size_t)col[e]] == blk[(size_t)r[p]] &&
+              lev[(size_t)col[e]] <= lev[(size_t)r[p]])
+            return;
+      auto more = [&](int i) { return (wl > wu ? nlow(i) : nup(i)) > 3; };
+      // by level, rows with second records first, then S position
+      keys.clear();
+      for (int p = 0; p < B.rows; ++p)
+        keys.push_back({(uint64_t)lev[(size_t)r[p]] << 33 | (uint64_t)!more(r[p]) << 32 |
+                            (uint32_t)s_of[(size_t)r[p]],
+                        r[p]});
+      std::sort(keys.begin(), keys.end());
+      for (int p = 0; p < B.rows; ++p) r[p] = keys[(size_t)p].second;
+      start.clear();
+      for (int p = 0; p < B.rows; ++p) {
+        if (p == 0 || lev[(size_t)r[p]] != lev[(size_t)r[p - 1]] || p - start.back() == kBrickLanes)
+          start.push_back(p);
+        step_of[(size_t)r[p]] = (int)start.size() - 1;
+      }
+      B.steps = (int)start.size();
+      start.push_back(B.rows);
+      P.steps = std::max(P.steps, B.steps);
+      for (int t = 0; t < 2; ++t) {
+        BrickTriangle &T = t == 0 ? out.L : out.U;
+        Joined &J = P.of[t];
+        const int stamp = 2 * k + t;
+        auto when = [&](int x) {  // sweep order of a row's step
+          return t == 0 ? step_of[(size_t)x] : B.steps - 1 - step_of[(size_t)x];
+        };
+        auto entries = [&](int x, auto &&f) {
+          const int e0 = t == 0 ? row[x] : dia[x] + 1, w = t == 0 ? nlow(x) : nup(x);
+          for (int j = 0; j < w; ++j) f(j, e0 + j, col[e0 + j]);
+        };
+        // the last step that reads each value of the unit and its halo
+        halo.clear();
+        hlast.clear();
+        last.assign((size_t)B.rows, -1);
+        for (int p = 0; p < B.rows; ++p) slot[(size_t)r[p]] = p;  // (for now its row in the unit)
+        for (int p = 0; p < B.rows; ++p)
+          entries(r[p], [&](int, int, int y) {
+            if (blk[(size_t)y] == blk[(size_t)r[p]]) {
+              int &l = last[(size_t)slot[(size_t)y]];
+              l = std::max(l, when(r[p]));
+            } else if (halo.size() <= kHaloMost) {
+              Entry &E = halo_at(stamp, y);
+              if (E.when != stamp) {
+                E = {stamp, y, (int)halo.size()};
+                halo.push_back(y);
+                hlast.push_back(0);
+              }
+              int &l = hlast[(size_t)E.h];
+              l = std::max(l, when(r[p]));
+            }
+          });
+        if (halo.size() > kHaloMost) return;
+        // slots in sweep order
+        if ((int)dies.size() < B.steps) dies.resize((size_t)B.steps);
+        for (int q = 0; q < B.steps; ++q) dies[(size_t)q].clear();
+        int slots = 1 + (int)halo.size();
+        for (size_t h = 0; h < halo.size(); ++h) dies[(size_t)hlast[h]].push_back(1 + (int)h);
+        unused.clear();
+        const size_t step0 = J.step.size();
+        J.step.resize(step0 + (size_t)B.steps);
+        for (int q = 0; q < B.steps; ++q) {
+          const int at_step = t == 0 ? q : B.steps - 1 - q;
+          const int c = start[(size_t)at_step], m = start[(size_t)at_step + 1] - c;
+          if (q > 0)
+            for (int s : dies[(size_t)q - 1]) unused.push_back(s);
+          for (int i = 0; i < m; ++i) {
+            const int x = r[c + i];
+            const int l = last[(size_t)(c + i)];
+            int s;
+            if (!unused.empty()) {
+              s = unused.back();
+              unused.pop_back();
+            } else {
+              s = slots++;
+            }
+            dies[(size_t)std::max(l, q)].push_back(s);
+            slot[(size_t)x] = s;
+            if (s > 0x3fff) return;  // 16-bit byte offsets
+          }
+          int more_rows = 0;
+          for (int i = 0; i < m; ++i)
+            if ((t == 0 ? nlow(r[c + i]) : nup(r[c + i])) > 3) more_rows = i + 1;
+          J.step[step0 + (size_t)at_step] = {(int)J.more_idx.size(),
+                                             (unsigned)(c | m << 12 | more_rows << 20)};
+          for (int i = 0; i < m; ++i) {
+            const int x = r[c + i];
+            BrickPlaces at[2] = {{{0, 0, 0, 0}}, {{0, 0, 0, 0}}};
+            BrickSource from[2] = {{{-1, -1, -1, x}}, {{-1, -1, -1, -1}}};
+            entries(x, [&](int j, int e, int y) {
+              const int s = blk[(size_t)y] == blk[(size_t)x] ? slot[(size_t)y]
+                                                             : 1 + halo_at(stamp, y).h;
+              at[j / 3].at[j % 3] = (unsigned short)(s * sizeof(float));
+              from[j / 3].e[j % 3] = e;
+            });
+            at[0].at[3] = (unsigned short)(slot[(size_t)x] * sizeof(float));
+            T.idx[(size_t)(B.row0 + c + i)] = at[0];
+            T.src[(size_t)(B.row0 + c + i)] = from[0];
+            if (i < more_rows) {
+              J.more_idx.push_back(at[1]);
+              J.more_src.push_back(from[1]);
+            }
+          }
+        }
+        (t == 0 ? B.lh0 : B.uh0) = (int)J.halo.size();
+        (t == 0 ? B.lh : B.uh) = (int)halo.size();
+        for (int y : halo) J.halo.push_back(s_of[(size_t)y]);
+        J.slots = std::max(J.slots, slots);
+      }
+    }
+    P.ok = true;
+  });
+  for (const Part &P : part)
+    if (!P.ok) return;
   for (int t = 0; t < 2; ++t) {
     BrickTriangle &T = t == 0 ? out.L : out.U;
+    for (const Part &P : part) {
+      const Joined &J = P.of[t];
+      const int more0 = (int)T.idx.size();   // the first records are all there
+      for (int k = P.first; k < P.last; ++k) {
+        BrickUnit &B = out.unit[(size_t)k];
+        if (t == 0) B.step0 += (int)T.step.size();
+        (t == 0 ? B.lh0 : B.uh0) += (int)T.halo.size();
+      }
+      for (BrickStep K : J.step) {
+        K.x0 += more0;
+        T.step.push_back(K);
+      }
+      T.halo.insert(T.halo.end(), J.halo.begin(), J.halo.end());
+      T.idx.insert(T.idx.end(), J.more_idx.begin(), J.more_idx.end());
+      T.src.insert(T.src.end(), J.more_src.begin(), J.more_src.end());
+      out.slots[t] = std::max(out.slots[t], J.slots);
+      out.steps = std::max(out.steps, P.steps);
+    }
     // one spare record: a step without second ones reads the record at its x0
-    more_idx[t].push_back(BrickPlaces{{0, 0, 0, 0}});
-    more_src[t].push_back(BrickSource{{-1, -1, -1, -1}});
-    T.idx.insert(T.idx.end(), more_idx[t].begin(), more_idx[t].end());
-    T.src.insert(T.src.end(), more_src[t].begin(), more_src[t].end());
-    for (BrickStep &K : T.step) K.x0 += n;
+    T.idx.push_back(BrickPlaces{{0, 0, 0, 0}});
+    T.src.push_back(BrickSource{{-1, -1, -1, -1}});
   }
   out.pos.resize((size_t)n);
   for (int p = 0; p < n; ++p) out.pos[(size_t)p] = s_of[(size_t)out.row[(size_t)p]];
@@ -922,27 +970,36 @@ void short_columns(const std::vector<long long> &off, const std::vector<int> &co
     out.off[s + 1] = out.off[s] + 64 * ((w + 1) / 2);
   }
   out.code.assign((size_t)out.off[ns], 0);
-  std::vector<int> seen;
-  for (size_t s = 0; s < ns; ++s) {
-    // each window starts at the smallest column that none before it holds
-    seen.assign(col.begin() + (long)off[s], col.begin() + (long)off[s + 1]);
-    std::sort(seen.begin(), seen.end());
-    int *const first = &out.window[s * kWindows];
-    int nw = 0;
-    for (const int c : seen)
-      if (nw == 0 || c - first[nw - 1] >= kWindow) {
-        if (nw == kWindows) return;
-        first[nw++] = c;
+  std::atomic<bool> fits{true};
+  in_parts((int)ns, 1 << 9, [&](int, int s0, int s1) {
+    for (int s = s0; s < s1 && fits; ++s) {
+      const int *const c = col.data() + off[(size_t)s];
+      const int slots = (int)(off[(size_t)s + 1] - off[(size_t)s]);
+      // each window starts at the smallest column that none before it holds
+      int *const first = &out.window[(size_t)s * kWindows];
+      int nw = 0;
+      for (long long bound = 0;;) {
+        int next = INT_MAX;
+        for (int i = 0; i < slots; ++i) next = c[i] >= bound && c[i] < next ? c[i] : next;
+        if (next == INT_MAX) break;
+        if (nw == kWindows) {
+          fits = false;
+          return;
+        }
+        first[nw++] = next;
+        bound = (long long)next + kWindow;
       }
-    for (long long i = off[s]; i < off[s + 1]; ++i) {
-      const int c = col[(size_t)i];
-      const int k = (int)(std::upper_bound(first, first + nw, c) - first) - 1;
-      const long long slot = (i - off[s]) / 64, lane = (i - off[s]) % 64;
-      out.code[(size_t)(out.off[s] + 64 * (slot / 2) + lane)] |=
-          ((unsigned)k << 12 | (unsigned)(c - first[k])) << (slot % 2 ? 16 : 0);
+      unsigned *const code = out.code.data() + out.off[(size_t)s];
+      for (int i = 0; i < slots; ++i) {
+        int k = 0;
+        while (k + 1 < nw && first[k + 1] <= c[i]) ++k;
+        const int slot = i / 64, lane = i % 64;
+        code[64 * (slot / 2) + lane] |= ((unsigned)k << 12 | (unsigned)(c[i] - first[k]))
+                                        << (slot % 2 ? 16 : 0);
+      }
     }
-  }
-  out.ok = true;
+  });
+  out.ok = fits;
 }
 
 double gather_lines(int n, const int *row, const int *col) {

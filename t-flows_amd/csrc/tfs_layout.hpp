@@ -18,9 +18,24 @@
 #pragma once
 
 #include <cstddef>
+#include <future>
 #include <vector>
 
 namespace tfs {
+
+// f(part, first, last) over [0, n) in kBeside parts, beside one another where there
+// are at least `least` of them in all (else in turn).
+constexpr int kBeside = 8;
+template <typename F>
+void in_parts(int n, int least, F f) {
+  std::future<void> part[kBeside];
+  const std::launch how =
+      n < least ? std::launch::deferred : std::launch::async | std::launch::deferred;
+  for (int k = 0; k < kBeside; ++k)
+    part[k] = std::async(how, f, k, (int)((long long)n * k / kBeside),
+                         (int)((long long)n * (k + 1) / kBeside));
+  for (std::future<void> &p : part) p.get();
+}
 
 struct Segment {
   int l0, l1;  // levels [l0, l1)
