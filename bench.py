@@ -217,10 +217,7 @@ def sweep_bytes(n, ntri):
 
 
 def fp64_sweep_name(A):
-    """The kernel of the FP64 sweeps of this file's boxes: over blocks where the
-    dependency graph is deep (24 levels and more), else level by level."""
-    return (("k_block_sweep" if A.info()["levels_lower"] >= 24 else "k_sweep_syncfree") +
-            " (FP64 forward/backward incomplete-Cholesky sweeps)")
+    return A.sweep_kernel() + " (FP64 forward/backward incomplete-Cholesky sweeps)"
 
 
 def sweep_roofline(A, c, inloop_us, traffic_profile=None):
@@ -368,8 +365,8 @@ INNER_NAMES = {0: "reference", 1: "point-coloured", 2: "brick two-colour"}
 def inner_name(info):
     """The inner order a matrix built, with its brick edge for the brick order."""
     if info["inner_order"] == 2:
-        e = info["inner_brick_edge"]
-        return f"{e}^3-brick two-colour"
+        k = info["inner_colours"]
+        return f"{info['inner_brick_edge']}^3-brick {'two' if k == 2 else k}-colour"
     if info["inner_order"] == 1 and info["inner_block"] > 1:
         return f"{info['inner_block']}-row block multi-colour"
     return INNER_NAMES.get(info["inner_order"], "block multi-colour")
@@ -454,32 +451,22 @@ def mixed_vs_fp64(args):
         kname = "k_ell_diff (FP32 sliced-ELL SpMV, difference form)"
         prof = "k_ell_diff_poisson256_counters"
         per = "8 nnz + 12 N + 4 per SpMV (FP32 values and vectors), one SpMV per FP32 iteration"
-    elif A.info()["inner_order"] == solvers.TFS_INNER_BRICKS:
+    else:
         units, per_unit = 2 * inner, fp32_sweep_bytes(c.n, c.nnz)
-        kname = (f"k_brick_sweep (FP32 DIC sweeps of the brick-ordered copy: "
-                 f"{A.info()['inner_brick_edge']}^3 bricks in two colours, "
-                 f"{A.info()['inner_levels']} levels, one launch per colour and direction)")
-        prof = "k_brick_sweep_poisson256_counters"
+        kernel, info = A.sweep_kernel(inner=True), A.info()
+        how = {"k_brick_sweep": "one launch per colour and direction",
+               "k_colour_sweep": "one launch per colour",
+               "k_sweep_syncfree": f"one persistent launch of {info['inner_sweep_groups']} "
+                                   "workgroups per sweep",
+               "k_level": "one launch per level"}[kernel]
+        kname = (f"{kernel} (FP32 DIC sweeps of the {inner_name(info)} copy, "
+                 f"{info['inner_levels']} levels, {how})")
+        prof = {"k_brick_sweep": "k_brick_sweep_poisson256_counters",
+                "k_colour_sweep": "k_colour_sweep_poisson256_counters"}.get(kernel)
         per = ("(8 (nnz - N) + 32 N) / 2 per sweep (FP32 DIC forward + backward pair), two "
                "sweeps per FP32 iteration")
-    elif (A.info()["inner_order"] == solvers.TFS_INNER_COLOURED
-          and A.info()["inner_block"] == 1):
-        units, per_unit = 2 * inner, fp32_sweep_bytes(c.n, c.nnz)
-        kname = "k_colour_sweep (FP32 point-coloured DIC sweeps, one launch per colour)"
-        prof = "k_colour_sweep_poisson256_counters"
-        per = ("(8 (nnz - N) + 32 N) / 2 per sweep (FP32 DIC forward + backward pair), two "
-               "sweeps per FP32 iteration, spread over the launches of the colours")
-    else:  # the reference order or BFS blocks: the generic sweeps, no counter summary
-        units, per_unit = 2 * inner, fp32_sweep_bytes(c.n, c.nnz)
-        g = A.info()["inner_sweep_groups"]
-        sched = (f"one persistent launch of {g} workgroups per sweep" if g > 0
-                 else "one launch per level")
-        kname = (("k_sweep_syncfree" if g > 0 else "k_level") +
-                 f" (FP32 DIC sweeps of the {inner_name(A.info())}-ordered copy, "
-                 f"{A.info()['inner_levels']} levels, {sched})")
-        prof = None
-        per = ("(8 (nnz - N) + 32 N) / 2 per sweep (FP32 DIC forward + backward pair), two "
-               "sweeps per FP32 iteration")
+        if kernel == "k_colour_sweep":
+            per += ", spread over the launches of the colours"
     algo = per_unit * units * args.steps / max(dom_n.value, 1)  # bytes per launch
     achieved = algo / (dom_launch_ms * 1e-3) / 1e9
     roof = {"kernel": kname, "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,

@@ -85,18 +85,27 @@ int tfs_matrix_values_changed(tfs_matrix *A);
 /* Device address of the matrix's FP64 values (nnz entries). */
 double *tfs_matrix_values_device(tfs_matrix *A);
 
-/* Schedule of the preconditioner sweeps (bitwise the same results):
+/* Schedule of the preconditioner sweeps (bitwise the same results).  Without a
+ * call of this, FP64 matrices whose dependency graph is deep and falls into blocks
+ * (8^3 cells of a lexicographic box) sweep block by block, one persistent launch
+ * per sweep, and the FP32 copies of bricks in two colours brick by brick, one
+ * launch per colour; others use the fastest of STATIC and LEVELS, timed on the
+ * first factor.
  *   TFS_SWEEP_LEVELS       one launch per level of the dependency DAG;
- *   TFS_SWEEP_STATIC       one persistent launch per sweep, workgroup w owning
- *                          row chunks w, w+G, ... (default where it times
- *                          faster than the levels); needs all G workgroups
- *                          resident, which an ordinary launch gets unless a
- *                          never-ending kernel holds CUs -- then the sweep's
- *                          bounded waits end it with TFS_ERR_DEVICE;
+ *   TFS_SWEEP_STATIC       the block and brick sweeps where they are built, else one
+ *                          persistent launch per sweep, workgroup w owning row
+ *                          chunks w, w+G, ...  The latter needs all G workgroups
+ *                          resident, which an ordinary launch gets unless other
+ *                          kernels that wait (several such sweeps side by side, a
+ *                          never-ending kernel) hold the CUs -- then its bounded
+ *                          waits end it with TFS_ERR_DEVICE.  Block sweeps need no
+ *                          number of workgroups resident, brick sweeps wait for none;
  *   TFS_SWEEP_DYNAMIC      one persistent launch taking chunks from a counter --
  *                          safe when several solves share the GPU concurrently;
- *   TFS_SWEEP_COOPERATIVE  the static schedule under a cooperative launch (the
- *                          runtime guarantees co-residency; slower to launch). */
+ *   TFS_SWEEP_COOPERATIVE  row chunks w, w+G, ... under a cooperative launch (the
+ *                          runtime guarantees co-residency; slower to launch).
+ * Every schedule but STATIC switches the block and brick sweeps off, which are 2 to
+ * 4 times faster than the row-by-row ones where they are built. */
 enum {
   TFS_SWEEP_LEVELS = 0,
   TFS_SWEEP_STATIC = 1,
@@ -121,10 +130,15 @@ typedef struct {
   int inner_order;      /* the inner order built (TFS_INNER_*; -1 until then) */
   int sweep_groups;     /* DIC sweeps: workgroups of the persistent launch,
                            0 for one launch per level                        */
-  int inner_sweep_groups; /* the same for the inner copy (-1 until built)    */
+  int inner_sweep_groups; /* the same for the inner copy's row-by-row sweeps
+                             and factor (-1 until built)                     */
   int inner_brick_edge; /* TFS_INNER_BRICKS built: the brick edge, else 0    */
 } tfs_matrix_info;
 int tfs_matrix_get_info(const tfs_matrix *A, tfs_matrix_info *info);
+/* Name of the kernel that the incomplete-Cholesky sweeps of this matrix run, or
+ * with `inner` those of its FP32 copy in the reliable-update refinement ("" until
+ * the copy is built). */
+const char *tfs_matrix_sweep_kernel(const tfs_matrix *A, int inner);
 
 /* ---- the solvers (Cg / Bicg / Cgs) -------------------------------------------
  * Host-memory variant: x1 = c_loc(x(1)) of x(-NB:N), r1 = b(1:N). */

@@ -435,8 +435,9 @@ void launch_sweep(tfs_matrix *A, const DevSweep &S, const Tri<T> &Tr, T *d, cons
     // soon as the workgroups of other, terminating kernels have left; it
     // saves the 10-20 us of queue synchronisation a cooperative launch
     // costs on each side.  Only another never-ending kernel holding CUs
-    // could keep a workgroup out: the bounded polls then end the sweep with
-    // an error (solves sharing the GPU use the dynamic schedule).
+    // (or enough sweeps of this kind side by side) could keep a workgroup out:
+    // the bounded polls then end the sweep with an error (solves sharing the
+    // GPU use the dynamic schedule; block sweeps need no such care).
     tm_begin(kc);
     hipLaunchKernelGGL((k_sweep_syncfree<T, OP, false>), dim3(A->grid_persistent), dim3(kChunk), 0,
                        cur_stream(), A->n, Tr, d, const_cast<T *>(b), x, armv, st, A->sweep_err,
@@ -482,10 +483,9 @@ void launch_sweep(tfs_matrix *A, const DevSweep &S, const Tri<T> &Tr, T *d, cons
 }
 
 // Whether the FP64 sweeps run over blocks (k_block_sweep): where the structure
-// has them (build_blocks), under the static schedule (the default); a server's
-// matrices have none (matrix_create_shared).  No timing decides: wherever the block graph is kBlockGain times
-// shallower than the rows' levels the blocks measured 2 to 4 times faster
-// (figures at k_block_sweep).
+// has them and they cost less than the levels (build_blocks: estimates, no timing),
+// under the static schedule (the default); a server's matrices have none
+// (matrix_create_shared).
 inline bool use_blocks(const tfs_matrix *A) {
   return A->blk_ok && !A->blk_off;
 }
@@ -2282,6 +2282,15 @@ extern "C" int tfs_matrix_get_info(const tfs_matrix *A, tfs_matrix_info *info) {
   info->inner_sweep_groups =
       A->inner ? (A->inner->persistent ? A->inner->grid_persistent : 0) : -1;
   return TFS_OK;
+}
+
+extern "C" const char *tfs_matrix_sweep_kernel(const tfs_matrix *A, int inner) {
+  if (A && inner) A = A->inner;
+  if (!A) return "";
+  if (use_blocks(A)) return "k_block_sweep";
+  if (inner && A->csw_colours > 0) return "k_colour_sweep";
+  if (inner && use_bricks(A)) return "k_brick_sweep";
+  return A->persistent ? "k_sweep_syncfree" : "k_level";
 }
 
 extern "C" int tfs_matrix_tune_spmv(tfs_matrix *A, int *rows_per_block, int *waves_per_group) {

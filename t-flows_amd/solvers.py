@@ -111,6 +111,8 @@ def _lib():
     lib.tfs_matrix_values_device.restype = _VP
     lib.tfs_matrix_values_device.argtypes = [_VP]
     lib.tfs_matrix_get_info.argtypes = [_VP, ctypes.POINTER(_Info)]
+    lib.tfs_matrix_sweep_kernel.restype = ctypes.c_char_p
+    lib.tfs_matrix_sweep_kernel.argtypes = [_VP, ctypes.c_int]
     lib.tfs_solve.argtypes = [_VP, ctypes.c_int, ctypes.c_int, _F64P, _F64P, _IP,
                               ctypes.c_double, _DP, _DP]
     lib.tfs_solve_device.argtypes = [_VP, ctypes.c_int, ctypes.c_int, _VP, _VP, _IP,
@@ -230,6 +232,10 @@ class Matrix:
                     ell64_slices=i.ell64_slices, inner_order=i.inner_order,
                     sweep_groups=i.sweep_groups, inner_sweep_groups=i.inner_sweep_groups,
                     inner_brick_edge=i.inner_brick_edge)
+
+    def sweep_kernel(self, inner=False):
+        """The kernel the sweeps run; `inner`: those of the FP32 copy."""
+        return self._lib.tfs_matrix_sweep_kernel(self._h, int(inner)).decode()
 
     def tune_spmv(self):
         """Times the SpMV shapes and keeps the fastest; returns (rows, waves)."""
