@@ -1392,11 +1392,13 @@ k_sweep_syncfree(int n, Tri<T> Tr, T *d, T *b, T *x, T *arm, const KState *st, i
 // every owner of an unfinished block runs and takes its blocks in ascending order,
 // a block is only begun when all before it are owned, the lowest unfinished one is
 // always under way, and every wait ends however few workgroups are resident:
-// the solves of any number of matrices may share the GPU.  Claims cost 0.3 to 1 us
-// a sweep (drawing the blocks from one counter 12 ns each, all in a row: 64
-// systems of 25^3 46 -> 62 us).  The polls are bounded as in k_sweep_syncfree all
-// the same (a halo slot given up is filled with zero, so wavefront 0 always
-// finishes).
+// the solves of any number of matrices may share the GPU.  Claims cost 0.1 to 0.6 us
+// a sweep of a few blocks per workgroup, 2.4 of 46 us where every block is on its
+// own (64 systems of 25^3; drawing the blocks from one counter 12 ns each, all in
+// a row: 62 us) and 14 of 499 at 256^3 (17 with a hand-over between the wavefronts
+// at every block, also where one rank is followed).  The polls are bounded as in
+// k_sweep_syncfree all the same (a halo slot given up is filled with zero, so
+// wavefront 0 always finishes).
 //
 // Every row sum is formed in the caller's entry order; padding entries are
 // 0 * 0 terms, which leave any sum as it is.
@@ -1405,13 +1407,13 @@ k_sweep_syncfree(int n, Tri<T> Tr, T *d, T *b, T *x, T *arm, const KState *st, i
 // row's arithmetic (about 0.12 us), per block on the chain one halo hop (store,
 // poll, LDS: about 1.2 us) -- and above about 5 M rows the traffic.  us per
 // sweep on MI355X, level-ordered sweeps (k_sweep_syncfree / k_levels_small)
-// before, blocks after: 12^3 30 -> 11, 32^3 113 -> 30, 97x75x61 348 -> 82,
-// 128^3 640 -> 138, 200^3 285 after.  Blocks of 8^3 rather than larger ones:
+// before, blocks after: 12^3 30 -> 12, 32^3 113 -> 30, 97x75x61 348 -> 79,
+// 128^3 640 -> 135, 200^3 288 after.  Blocks of 8^3 rather than larger ones:
 // 16^3 halves the hops but needs several wavefronts and a barrier per step.
 // Tried and not kept: one wavefront that also polls (its loads wait for its
 // stores: 104 us at 97x75x61, 172 at 128^3), two polling wavefronts (84, 145),
 // polling the whole halo from the start (82, 139), twice the workgroups (82,
-// 141; 264 at 200^3, but solves beside this one need room).
+// 141; 264 at 200^3, but a solve beside this one would then wait for its CUs).
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -1424,6 +1426,7 @@ __device__ __forceinline__ void wave_sync() {
 constexpr int kClaimLine = 32;                 // words from one line of claims to the next
 constexpr int kClaimLines = 64;                // one lane each: up to 2048 ranks
 constexpr int kClaimPolls = 16;                // looks before a rank of others is claimed
+constexpr int kOneRank = 1 << 30;              // beside a block: every later one is G on
 struct BlockShare {
   unsigned *claim;
   int *chain;
@@ -1445,6 +1448,8 @@ struct BlockShare {
     tail = rank = r;
     return r;
   }
+  // all ranks are claimed and one of them is this workgroup's
+  __device__ __forceinline__ bool one_rank() const { return round > 0 && head == tail; }
   // the next block; nblk or more: there is none
   __device__ __forceinline__ int next(int nblk) {
     if (round > 0) {
@@ -1540,6 +1545,7 @@ k_block_sweep(int n, int nblk, BlockTri Tr, const int *__restrict__ src,
   }
   __syncthreads();
   int bk = __builtin_amdgcn_readfirstlane(then);
+  int on = 0;   // the way to every later block, once there is one rank to follow
   if (__builtin_amdgcn_readfirstlane(done)) return;
   while (bk < nblk) {
     const Block B = Tr.blk[bk];
@@ -1619,14 +1625,18 @@ k_block_sweep(int n, int nblk, BlockTri Tr, const int *__restrict__ src,
     __syncthreads();
     if (tid >= kWave) {
       // ---- wavefront 1: the halo
+      // (every load unconditional, past the end the last entry again: with
+      // conditional ones the compiler waits for each before the next)
       int hq[kHaloLane];
       unsigned lack = 0;
+      if (B.halo > 0) {
 #pragma unroll
-      for (int c = 0; c < kHaloLane; ++c)
-        if (c * kWave < B.halo) {
+        for (int c = 0; c < kHaloLane; ++c)
           hq[c] = Tr.halo[B.halo0 + min(c * kWave + lane, B.halo - 1)];
+#pragma unroll
+        for (int c = 0; c < kHaloLane; ++c)
           if (c * kWave + lane < B.halo) lack |= 1u << c;
-        }
+      }
       double *const slot = xs + 1 + B.rows + lane;
       bool started = B.halo <= kHaloHead;
       for (unsigned spins = 1; __any(lack != 0); ++spins) {
@@ -1650,29 +1660,27 @@ k_block_sweep(int n, int nblk, BlockTri Tr, const int *__restrict__ src,
             lack &= ~1u;
           }
         }
-        // all of them loaded before any is looked at (a lane that lacks none of
-        // its own repeats one of another's: the same line)
+        // all of them loaded before any is looked at, by the lanes that lack one
+        // (every lane loading, the idle ones a line of another's: 137 us at 128^3
+        // and 81 at 97x75x61, with conditional index loads)
         double v[kHaloLane];
-        unsigned long long any[kHaloLane];
-#pragma unroll
-        for (int c = 0; c < kHaloLane; ++c) {
-          any[c] = __ballot(lack >> c & 1u);
-          if (any[c]) {
-            const int first = __builtin_amdgcn_readlane(hq[c], __builtin_ctzll(any[c]));
-            v[c] = coherent_load(&out[(lack >> c & 1u) ? hq[c] : first]);
-          }
-        }
 #pragma unroll
         for (int c = 0; c < kHaloLane; ++c)
-          if (any[c] && (lack >> c & 1u) && !waiting(v[c])) {
+          if (lack >> c & 1u) v[c] = coherent_load(&out[hq[c]]);
+#pragma unroll
+        for (int c = 0; c < kHaloLane; ++c)
+          if ((lack >> c & 1u) && !waiting(v[c])) {
             __hip_atomic_store(slot + c * kWave, v[c], __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_WORKGROUP);
             lack &= ~(1u << c);
           }
       }
-      const int b1 = share.next(nblk);
-      if (lane == 0)
-        __hip_atomic_store(&then, b1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (on == 0) {
+        const int b1 = share.next(nblk);
+        if (lane == 0)
+          __hip_atomic_store(&then, share.one_rank() ? b1 | kOneRank : b1, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
     } else {
       // ---- wavefront 0: the steps.  Row data of the next step is read from
       // LDS while this one computes (two register sets in turn).
@@ -1732,10 +1740,17 @@ k_block_sweep(int n, int nblk, BlockTri Tr, const int *__restrict__ src,
         if (t + 1 < B.steps) advance(r1, r0, t + 1);
       }
     }
+    if (on > 0) {
+      bk += on;
+      continue;
+    }
     // (wavefront 1 always gets there: its polls are bounded)
-    do bk = __hip_atomic_load(&then, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    while (bk < 0);
-    bk = __builtin_amdgcn_readfirstlane(bk);
+    int b1;
+    do b1 = __hip_atomic_load(&then, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    while (b1 < 0);
+    b1 = __builtin_amdgcn_readfirstlane(b1);
+    if (b1 & kOneRank) on = (int)gridDim.x;
+    bk = b1 & ~kOneRank;
   }
 }
 

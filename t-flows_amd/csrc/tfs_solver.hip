@@ -1948,11 +1948,11 @@ int build_ell64(tfs_matrix *A, const Layout &Ly) {
 }
 
 // The block sweeps' structure, if it suits them, and their grid: at most half
-// the workgroups that fit at once.  Twice as many measured no faster, and none of
+// the workgroups that fit at once, so that a solve beside this one finds room; none of
 // them has to be resident (k_block_sweep).
 int build_block_sweeps(tfs_matrix *A, const Layout &Ly, const BlockLayout &BL, const int *dia) {
   const int n = A->n;
-  if (!BL.ok) return 0;
+  if (!BL.ok || BL.nblk > kOneRank - kWave * 32) return 0;  // a block and its flag share a word
   DevBlocks &L = A->bL, &U = A->bU;
   std::vector<int> to_s((size_t)n), bz((size_t)n), dsrc((size_t)n);
   for (int p = 0; p < n; ++p) {
