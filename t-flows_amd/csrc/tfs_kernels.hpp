@@ -1144,6 +1144,17 @@ template <> struct Sentinel<float> {
   __device__ static bool is(float v) { return (unsigned int)__float_as_int(v) == bits; }
 };
 
+// Kept under 80 registers, six workgroups a CU: the server gives each of its
+// concurrent sweeps a share of what fits on the GPU at once, and the large systems
+// of a mix wait for rows in flight (24 cases of 1.2e4 to 2.7e6 rows, eight workers:
+// 20.3 solves/s at 107 registers and four workgroups, 25.4 at 78).  The entries begin
+// as zeros, and the polls form their addresses anew each time (the empty asm makes
+// the positions opaque): left to itself the compiler keeps eight addresses and
+// copies of the half-set entries over the whole loop.  Not the FP32 sweeps, which fit
+// anyhow (64 systems in a batch 872 -> 959 ms with it).
+template <typename T, int OP>
+constexpr bool kLean = sizeof(T) == 8 || OP == OP_FACTOR;
+
 // One row of a sweep, as a thread holds it.
 template <typename T>
 struct SweepRow {
@@ -1165,6 +1176,13 @@ __device__ __forceinline__ void sweep_load1(SweepRow<T> &r, int p, int n, const 
   r.e0 = r.len = r.used = r.src = 0;
   r.miss = 0;
   r.s = r.dp = 0.0;
+  if (kLean<T, OP>) {
+#pragma unroll
+    for (int k = 0; k < kPrefetch; ++k) {
+      r.pc[k] = 0;
+      r.pv[k] = r.px[k] = 0;
+    }
+  }
   if (r.done) return;
   r.e0 = Tr.ptr[p];
   r.len = Tr.ptr[p + 1] - r.e0;
@@ -1210,6 +1228,10 @@ template <typename T, int OP>
 __device__ __forceinline__ bool sweep_pass(SweepRow<T> &r, const Tri<T> &Tr, T *out, bool first) {
   if (r.done) return true;
   if (first) r.miss = (1u << min(r.len, kPrefetch)) - 1u;
+  if (kLean<T, OP>) {
+#pragma unroll
+    for (int k = 0; k < kPrefetch; ++k) asm volatile("" : "+v"(r.pc[k]));
+  }
 #pragma unroll
   for (int k = 0; k < kPrefetch; ++k)
     if (r.miss >> k & 1u) r.px[k] = first ? out[r.pc[k]] : coherent_load(&out[r.pc[k]]);
