@@ -1,7 +1,7 @@
 """Throughput of the GPU Krylov solve on one MI355X, with the reference CPU
 solver timed beside it.
 
-    python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload 2]
+    python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload 3]
 
 A step is one complete solve of the workload's linear system, as the
 reference's Process makes it after every assembly: Prec_Form (the factor is
@@ -12,11 +12,12 @@ x = 0 on the device (part of the timed work).
 
 Workloads (sizes and seeds in t-flows_amd/cases.py):
   1  Poisson 32^3, Cg + incomplete Cholesky (prec 2) to relative 1e-8.
-  2  (default) momentum matrix on a 128^3 hex mesh (tanh clustering beta 2,
+  2  momentum matrix on a 128^3 hex mesh (tanh clustering beta 2,
      +-10% node jitter, random cell numbering, upwind convection-diffusion nu
      1e-3, inertia V/dt), Bicg + prec 2 to relative 1e-10, FP64.
-  3  Poisson 256^3 stretched to cell aspect ratio 100: FP32-inner PCG in FP64
-     iterative refinement to 1e-10 (the value), plain FP64 Cg timed beside it.
+  3  (default) Poisson 256^3 stretched to cell aspect ratio 100: FP32-inner
+     PCG in FP64 iterative refinement to 1e-10 (the value), plain FP64 Cg timed
+     beside it.
   4  64 Poisson systems of uneven size in one block-diagonal batch, FP32+FP64
      refinement to 1e-10; a step solves all 64.
   5  serving: an open-loop Poisson-arrival request stream (200 req/s, 24
